@@ -44,6 +44,9 @@ struct MmaDesc {
   uint32_t dt, adt;
   uint32_t k0, k1;          // K range of this tile (a K split's share; else 0, K)
   uint32_t S, split, ti;    // K split count, this tile's split, task index
+  uint32_t ldb;             // a k-contiguous B's row stride and batch stride (elements)
+  uint64_t gsb;
+  uint32_t subs;            // tiles of the split scratch per output tile (4: a 256-wide tile as 128-wide ones)
 };
 
 // Store epilogue micro-program (mma.cl:67-96): {n, n x {kind, src, s, t}}, src 0
@@ -103,6 +106,45 @@ VM_DEV v4f epi_inline4(uint32_t kind, v4f x, v4f y, float s, float t) {
     case SUB_MAX: return v4f_make(fmaxf(x.x, y.x), fmaxf(x.y, y.y), fmaxf(x.z, y.z), fmaxf(x.w, y.w));
     case SUB_MIN: return v4f_make(fminf(x.x, y.x), fminf(x.y, y.y), fminf(x.z, y.z), fminf(x.w, y.w));
     default: return x;
+  }
+}
+
+// epi_inline on the sixteen values of a thread's four rows
+VM_DEV void epi_inline16(uint32_t kind, v4f (&x)[4], const v4f (&y)[4], float s, float t) {
+  switch (kind) {
+    case SUB_AFFINE:
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = epi_inline4(SUB_AFFINE, x[u], y[u], s, t);
+      break;
+    case SUB_GELU:
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = epi_inline4(SUB_GELU, x[u], y[u], s, t);
+      break;
+    case SUB_ADD:
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = epi_inline4(SUB_ADD, x[u], y[u], s, t);
+      break;
+    case SUB_MUL:
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = epi_inline4(SUB_MUL, x[u], y[u], s, t);
+      break;
+    case SUB_SUB:
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = epi_inline4(SUB_SUB, x[u], y[u], s, t);
+      break;
+    case SUB_DIV:
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = epi_inline4(SUB_DIV, x[u], y[u], s, t);
+      break;
+    case SUB_MAX:
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = epi_inline4(SUB_MAX, x[u], y[u], s, t);
+      break;
+    case SUB_MIN:
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = epi_inline4(SUB_MIN, x[u], y[u], s, t);
+      break;
+    default: break;
   }
 }
 
@@ -199,7 +241,8 @@ VM_DEV void store_acc(Args A, const MmaDesc& D, const f32x16 (&acc)[MmaCfg<T>::k
 
 __shared__ uint32_t vm_mma_last;       // this lane's split arrived last (K-split combine)
 
-// Store of a general tile: the tile itself, or (K split) its f32 partial.  A
+// K split: publish this split's f32 partial tile; in the split that arrives last,
+// sum all of them into acc and return true (the caller stores the tile).  A
 // partial is written in register order, 16 bytes per thread and step (values
 // 4q .. 4q + 3 of thread x at [(tile S + split) NQ + q] kBlock + x, NQ = T^2 /
 // (4 kBlock)), coalesced.  Each thread waits for its own stores to complete, the
@@ -213,14 +256,12 @@ __shared__ uint32_t vm_mma_last;       // this lane's split arrived last (K-spli
 // several splits' partials before the first add (one memory round trip per
 // batch, not per value).
 template <int T>
-VM_DEV void mma_store(Args A, const MmaDesc& D, f32x16 (&acc)[MmaCfg<T>::kBM][MmaCfg<T>::kBN], uint32_t tile,
-                      uint32_t g, uint32_t m0, uint32_t n0) {
-  if (D.S <= 1) return store_acc<T>(A, D, acc, g, m0, n0);
+VM_DEV bool mma_split_combine(Args A, const MmaDesc& D, f32x16 (&acc)[MmaCfg<T>::kBM][MmaCfg<T>::kBN], uint32_t tile) {
   using C = MmaCfg<T>;
   constexpr uint32_t NQ = C::kBM * C::kBN * 4;             // float4 steps per thread
   constexpr uint32_t B = NQ <= 4 ? 8 : NQ <= 16 ? 2 : 1;   // splits per load batch (<= 32 float4)
   v4f* sp = reinterpret_cast<v4f*>(A->scratch + A->task_scratch[D.ti]);
-  const uint64_t nbase = uint64_t(D.tm) * D.tn * D.G;
+  const uint64_t nbase = uint64_t(D.tm) * D.tn * D.G * D.subs;
   uint32_t* arrivals = reinterpret_cast<uint32_t*>(sp + nbase * D.S * NQ * kBlock);
   v4f* mine = sp + (uint64_t(tile) * D.S + D.split) * NQ * kBlock + threadIdx.x;
 #pragma unroll
@@ -241,7 +282,7 @@ VM_DEV void mma_store(Args A, const MmaDesc& D, f32x16 (&acc)[MmaCfg<T>::kBM][Mm
     vm_mma_last = last;
   }
   __syncthreads();
-  if (!vm_mma_last) return;
+  if (!vm_mma_last) return false;
   const v4f* hp = sp + uint64_t(tile) * D.S * NQ * kBlock + threadIdx.x;
   for (uint32_t s0 = 0; s0 < D.S; s0 += B) {
     v4f part[B][NQ];
@@ -268,6 +309,13 @@ VM_DEV void mma_store(Args A, const MmaDesc& D, f32x16 (&acc)[MmaCfg<T>::kBM][Mm
             }
       }
   }
+  return true;
+}
+
+template <int T>
+VM_DEV void mma_store(Args A, const MmaDesc& D, f32x16 (&acc)[MmaCfg<T>::kBM][MmaCfg<T>::kBN], uint32_t tile,
+                      uint32_t g, uint32_t m0, uint32_t n0) {
+  if (D.S > 1 && !mma_split_combine<T>(A, D, acc, tile)) return;
   store_acc<T>(A, D, acc, g, m0, n0);
 }
 
@@ -433,6 +481,9 @@ VM_DEV MmaDesc load_desc(const MmaDesc* p) {
   D.S = uni(p->S);
   D.split = uni(p->split);
   D.ti = uni(p->ti);
+  D.subs = uni(p->subs);
+  D.ldb = uni(p->ldb);
+  D.gsb = uint64_t(uni(uint32_t(p->gsb))) | uint64_t(uni(uint32_t(p->gsb >> 32))) << 32;
   return D;
 }
 
@@ -445,13 +496,14 @@ VM_DEV void tile_origin(const MmaDesc& D, uint32_t tile, uint32_t T, uint32_t* g
 }
 
 template <int T, bool BF16>
-VM_TILE void mma_tile16(Args A, const MmaDesc* Dp, uint32_t tile) {
+VM_TILE void mma_tile16(Args A, const MmaDesc* Dp, uint32_t tile, uint32_t g, uint32_t m0, uint32_t n0) {
   A = uargs(A);
   const MmaDesc D = load_desc(Dp);
   uint16_t* lds = lds_ptr<uint16_t>();
   using C = MmaCfg<T>;
-  uint32_t g, m0, n0;
-  tile_origin(D, uni(tile), T, &g, &m0, &n0);
+  g = uni(g);
+  m0 = uni(m0);
+  n0 = uni(n0);
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wm = wave >> 1, wn = wave & 1;
   const OperandRead ar = operand_read(aux_of(A), D.av, D.a, D.K, uint64_t(D.G) * D.M * D.K, 8);
@@ -598,19 +650,22 @@ struct FastDma {
 // columns past M / N are computed but not stored; the k past K are zeroed in LDS
 // (RaggedDma::zero) before the stage is published, in both operands, so that
 // they add 0 whatever the clamped data holds.
+template <bool BT>
 struct RaggedDma {
   uint32_t ra, ca, rb, cb;  // per lane: A row within a round and its k chunk; B k row within a round and n chunk
-  uint32_t wo;
+  uint32_t wo, ldb;         // (BT: B's rows and k chunks are placed as A's)
   const gbyte* a;           // A[g, m0, 0]
   const gbyte* b;           // B[g, 0, n0]
   uint32_t M, N, K, m0, n0;
-  VM_DEV void init(const gbyte* a_, const gbyte* b_, uint32_t M_, uint32_t N_, uint32_t K_, uint32_t m0_, uint32_t n0_) {
+  VM_DEV void init(const gbyte* a_, const gbyte* b_, uint32_t M_, uint32_t N_, uint32_t K_, uint32_t m0_, uint32_t n0_,
+                   uint32_t ldb_) {
     const uint32_t l = threadIdx.x & 63, w = threadIdx.x >> 6;
     ra = 8 * w + (l >> 3);
     ca = (l & 7) ^ aswz(ra);
-    rb = 2 * w + (l >> 5);
-    cb = (l & 31) ^ (4 * (rb & 3));
+    rb = BT ? ra : 2 * w + (l >> 5);
+    cb = BT ? ca : (l & 31) ^ (4 * (rb & 3));
     wo = uni(1024 * w);
+    ldb = ldb_;
     a = a_;
     b = b_;
     M = M_;
@@ -625,6 +680,10 @@ struct RaggedDma {
       const uint32_t row = min(m0 + 32 * uint32_t(r) + ra, M - 1) - m0;
       const uint32_t k = min(s * kFBK + 8 * ca, K - 8);
       dma16(a, row * K * 2 + k * 2, st + wo + 4096 * r);
+    } else if constexpr (BT) {
+      const uint32_t row = min(n0 + 32 * uint32_t(r - 8) + rb, N - 1) - n0;
+      const uint32_t k = min(s * kFBK + 8 * cb, K - 8);
+      dma16(b, row * ldb * 2 + k * 2, st + kFStageB + wo + 4096 * (r - 8));
     } else {
       // the slab's rows from a scalar base, so the lane offset stays below 64 rows
       const uint32_t k = min(s * kFBK + 8 * uint32_t(r - 8) + rb, K - 1) - s * kFBK;
@@ -644,7 +703,7 @@ struct RaggedDma {
     }
 #pragma unroll
     for (int r = 0; r < 8; ++r)
-      if (8 * uint32_t(r) + rb >= kv)
+      if (BT ? 8 * cb >= kv : 8 * uint32_t(r) + rb >= kv)
         *(lds_v4u*)uintptr_t(st + kFStageB + wo + 4096 * r + 16 * l) = v4u_make(0, 0, 0, 0);
   }
 };
@@ -795,7 +854,9 @@ VM_DEV void store_fast(Args A, const MmaDesc& D, const f32x16 (&acc)[4][4], uint
   }
 }
 
-template <bool BF16, bool RAG>
+// BT (ragged form only): B is k-contiguous (x . W^T: a tied embedding's logits),
+// its slab placed and read as A's is.
+template <bool BF16, bool RAG, bool BT>
 VM_LEAF void mma_tile16_fast(Args A, const MmaDesc* Dp, uint32_t tile) {
   A = uargs(A);
   const MmaDesc D = load_desc(Dp);
@@ -805,7 +866,7 @@ VM_LEAF void mma_tile16_fast(Args A, const MmaDesc* Dp, uint32_t tile) {
   fast_origin(D, uni(tile), &g, &m0, &n0);
   const uint32_t K = D.K, N = D.N;
   const gbyte* a = D.a + (uint64_t(g) * D.M + m0) * K * 2;        // A[g, m0, 0]
-  const gbyte* b = D.b + (uint64_t(g) * K * N + n0) * 2;           // B[g, 0, n0]
+  const gbyte* b = D.b + (BT ? D.gsb * g + uint64_t(n0) * D.ldb : uint64_t(g) * K * N + n0) * 2;   // B[g, 0, n0]
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wm = wave >> 1, wn = wave & 1;
   f32x16 acc[4][4];
@@ -815,8 +876,9 @@ VM_LEAF void mma_tile16_fast(Args A, const MmaDesc* Dp, uint32_t tile) {
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x16{};
   const uint32_t nk = RAG ? (K + kFBK - 1) / kFBK : K / kFBK;
   FastDma dm;
-  RaggedDma rd;
-  if constexpr (RAG) rd.init(a, b, D.M, N, K, m0, n0);
+  RaggedDma<BT> rd;
+  static_assert(RAG || !BT, "the k-contiguous B takes the ragged form");
+  if constexpr (RAG) rd.init(a, b, D.M, N, K, m0, n0, D.ldb);
   else dm.init(K, N);
   auto slab_a = [&](uint32_t s) { return a + uint64_t(s) * kFBK * 2; };
   auto slab_b = [&](uint32_t s) { return b + uint64_t(s) * kFBK * N * 2; };
@@ -834,6 +896,11 @@ VM_LEAF void mma_tile16_fast(Args A, const MmaDesc* Dp, uint32_t tile) {
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       fb[j] = kFStageB + row * 512 + ((wn * 16 + 4 * (uint32_t(j) ^ e) + 2 * (gq & 1) + (q >> 1)) * 16) + (q & 1) * 8;
+    if constexpr (BT) {                 // indexed by the k step, as A's
+      const uint32_t rn = wn * 128 + (lane & 31), swn = aswz(rn);
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) fb[kk] = kFStageB + rn * 128 + (((2 * kk + (lane >> 5)) ^ swn) * 16);
+    }
   }
   u16x8 af[2][4], bfr[2][4];
   auto frags = [&](int p, uint32_t st, int kk) {
@@ -842,6 +909,10 @@ VM_LEAF void mma_tile16_fast(Args A, const MmaDesc* Dp, uint32_t tile) {
     for (int i = 0; i < 4; ++i) af[p][i] = *(const lds_u16x8*)(S + fa[kk] + 4096 * i);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+      if constexpr (BT) {
+        bfr[p][j] = *(const lds_u16x8*)(S + fb[kk] + 4096 * j);
+        continue;
+      }
       const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(S + fb[j] + 8192 * kk));
       const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(S + fb[j] + 8192 * kk + 2048));
       bfr[p][j] = __builtin_bit_cast(u16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -1012,13 +1083,14 @@ struct Stage32 {
 };
 
 template <int T>
-VM_TILE void mma_tile32(Args A, const MmaDesc* Dp, uint32_t tile) {
+VM_TILE void mma_tile32(Args A, const MmaDesc* Dp, uint32_t tile, uint32_t g, uint32_t m0, uint32_t n0) {
   A = uargs(A);
   const MmaDesc D = load_desc(Dp);
   float* lds = lds_ptr<float>();
   using C = MmaCfg<T>;
-  uint32_t g, m0, n0;
-  tile_origin(D, uni(tile), T, &g, &m0, &n0);
+  g = uni(g);
+  m0 = uni(m0);
+  n0 = uni(n0);
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wm = wave >> 1, wn = wave & 1;
   const bool vec = !D.av && !D.bv && (D.K % 4) == 0 && (D.N % 4) == 0 && ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0;
@@ -1182,9 +1254,15 @@ VM_LEAF void mma_tile32_fast(Args A, const MmaDesc* Dp, uint32_t tile) {
 
 // LDS bytes the matmul tile op needs at its largest tile.
 constexpr int kMaxI(int a, int b) { return a > b ? a : b; }
-constexpr int kMmaLdsBytes0 = kMaxI(kMaxI(Lds16<256>::kBytes, Lds16<128>::kBytes), kMaxI(Lds16<64>::kBytes, Lds32<256>::kBytes));
+constexpr int kMmaLdsBytes0 = kMaxI(kMaxI(Lds16<64>::kBytes, Lds16<128>::kBytes), Lds32<128>::kBytes);
 constexpr int kMmaLdsBytes1 = kFastLdsBytes > kMmaLdsBytes0 ? kFastLdsBytes : kMmaLdsBytes0;
 constexpr int kMmaLdsBytes = kF32FastLdsBytes > kMmaLdsBytes1 ? kF32FastLdsBytes : kMmaLdsBytes1;
+
+}  // namespace vm
+
+#include "tile_mma_pipe.h"
+
+namespace vm {
 
 VM_DEV void mma_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   A = uargs(A);
@@ -1201,36 +1279,69 @@ VM_DEV void mma_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   D.a = resolve(A, t.a);
   D.b = resolve(A, t.b);
   D.d = resolve(A, t.dst);
-  D.av = t.p[4];
-  D.bv = t.p[5];
+  // operand views the loader resolved to strides (kMmaStrided): the view itself follows the strides
+  D.av = t.p[4] & kMmaStrided ? uint32_t(aux_of(A)[(t.p[4] & ~kMmaStrided) + 4]) : t.p[4];
+  D.bv = t.p[5] & kMmaStrided ? uint32_t(aux_of(A)[(t.p[5] & ~kMmaStrided) + 4]) : t.p[5];
   D.epi = t.p[6];
   D.res = t.p[6] ? resolve(A, t.p[7]) : D.a;
   D.dt = (t.tile_op >> 8) & 0xFF;
   D.adt = (t.tile_op >> 16) & 0xFF;
   D.S = 1u << ((t.p[3] >> 28) & 0xF);
   D.ti = ti;
+  D.ldb = 0;
+  D.gsb = 0;
   D.k0 = 0;
   D.k1 = D.K;
   D.split = 0;
   hi = min(hi, D.tm * D.tn * D.G * D.S);
   const bool h16 = D.adt == DT_BF16 || D.adt == DT_F16, bf = D.adt == DT_BF16;
-  // a K split's share: whole slabs of the general tiles (32 16-bit or 16 f32 k)
-  const uint32_t bk = h16 ? uint32_t(kBK16) : uint32_t(kBK32);
+  const bool epi_ok = (D.dt == DT_F32 || D.dt == DT_BF16 || D.dt == DT_F16) && epi_inline_ok(A, D.epi);
+  // a K split's share: whole slabs of the pipelined tiles (64 16-bit or 32 f32 k)
+  const uint32_t bk = h16 ? 64u : 32u;
   const uint32_t ksh = ((D.K + D.S - 1) / D.S + bk - 1) / bk * bk;
-  const bool fast = D.S == 1 && h16 && T == 256 && !D.av && !D.bv && D.M % 256 == 0 && D.N % 256 == 0 && D.K % kFBK == 0 &&
-                    D.N < (1u << 22) && ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0 &&
-                    (D.dt == DT_F32 || D.dt == DT_BF16 || D.dt == DT_F16) && epi_inline_ok(A, D.epi);
-  // the same tile for ragged shapes: 16-byte rows (K, N multiples of 8), offsets
-  // within 32 bits (RaggedDma)
-  const bool fastr = !fast && D.S == 1 && h16 && T == 256 && !D.av && !D.bv && D.K >= 8 && D.K % 8 == 0 && D.N % 8 == 0 &&
-                     D.K < (1u << 22) && D.N < (1u << 22) && ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0 &&
-                     (D.dt == DT_F32 || D.dt == DT_BF16 || D.dt == DT_F16) && epi_inline_ok(A, D.epi);
-  const bool fast32 = D.S == 1 && D.adt == DT_F32 && T == 256 && !D.av && !D.bv && D.M % 256 == 0 && D.N % 256 == 0 &&
-                      D.K % kF32BK == 0 && D.N < (1u << 22) && ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0 &&
-                      (D.dt == DT_F32 || D.dt == DT_BF16 || D.dt == DT_F16) && epi_inline_ok(A, D.epi);
-  const bool fast32r = !fast32 && D.S == 1 && D.adt == DT_F32 && T == 256 && !D.av && !D.bv && D.K >= 4 &&
-                       D.K % 4 == 0 && D.N % 4 == 0 && D.N < (1u << 22) && ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0 &&
-                       (D.dt == DT_F32 || D.dt == DT_BF16 || D.dt == DT_F16) && epi_inline_ok(A, D.epi);
+  // 256-wide tiles: the big square GEMMs' fast paths.  Ragged shapes need 16-byte
+  // rows (K, N multiples of 8, f32: of 4) and offsets within 32 bits.
+  const bool plain = D.S == 1 && T == 256 && !D.av && !D.bv && D.N < (1u << 22) &&
+                     ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0 && epi_ok;
+  const bool fast = plain && h16 && D.M % 256 == 0 && D.N % 256 == 0 && D.K % kFBK == 0;
+  const bool fastr = plain && !fast && h16 && D.K >= 8 && D.K % 8 == 0 && D.N % 8 == 0 && D.K < (1u << 22);
+  const bool fast32 = plain && !h16 && D.M % 256 == 0 && D.N % 256 == 0 && D.K % kF32BK == 0;
+  const bool fast32r = plain && !fast32 && !h16 && D.K >= 4 && D.K % 4 == 0 && D.N % 4 == 0;
+  // A loop of its own for each fast tile: what is live across the call is little
+  // (the tile takes every register, so the kernel keeps its values in scratch).
+#define VM_FAST_TILES(COND, CALL)                                      \
+  if (COND) {                                                          \
+    for (uint32_t tile = lo; tile < hi; ++tile) CALL(A, &D, tile);     \
+    return;                                                            \
+  }
+  VM_FAST_TILES(fast && bf, (mma_tile16_fast<true, false, false>))
+  VM_FAST_TILES(fast, (mma_tile16_fast<false, false, false>))
+  VM_FAST_TILES(fastr && bf, (mma_tile16_fast<true, true, false>))
+  VM_FAST_TILES(fastr, (mma_tile16_fast<false, true, false>))
+  VM_FAST_TILES(fast32, mma_tile32_fast<false>)
+  VM_FAST_TILES(fast32r, mma_tile32_fast<true>)
+  MmaOp ops[2];
+  ops[0] = mma_op(aux_of(A), t.p[4], D.a, D.M, D.K, D.G, true, h16 ? 2 : 4);
+  ops[1] = mma_op(aux_of(A), t.p[5], D.b, D.N, D.K, D.G, false, h16 ? 2 : 4);
+  // The pipelined tiles where both operands are strided matrices (or A is read in
+  // whole chunks through its view, which only go global -> LDS directly, so B's
+  // have to as well), the general ones otherwise.
+  const bool pipe = epi_ok && ops[0].cls != MOP_NONE && ops[1].cls != MOP_NONE &&
+                    (ops[0].cls != MOP_RUNS || ops[1].cls == MOP_DMA);
+  // a k-contiguous B: the ragged 16-bit tile with B staged as A is
+  if (pipe && D.S == 1 && T == 256 && h16 && !D.av && ops[1].kc && ops[1].cls == MOP_DMA && D.K >= 8 && D.K % 8 == 0 &&
+      D.N % 8 == 0 && D.K < (1u << 22) && D.N < (1u << 22) && (uintptr_t(D.a) & 15) == 0) {
+    D.ldb = ops[1].ld;
+    D.gsb = ops[1].gs;
+    D.b = ops[1].p;
+    VM_FAST_TILES(bf, (mma_tile16_fast<true, true, true>))
+    VM_FAST_TILES(true, (mma_tile16_fast<false, true, true>))
+  }
+#undef VM_FAST_TILES
+  // a 256-wide tile outside the fast paths is done as four 128-wide ones
+  const uint32_t sub = T == 256 ? 2u : 1u, E = T / sub;
+  D.subs = sub * sub;
+  const uint32_t route = (pipe ? 0u : 6u) + (E == 128 ? 3u : 0u) + (!h16 ? 2u : bf ? 0u : 1u);
   for (uint32_t ts = lo; ts < hi; ++ts) {
     uint32_t tile = ts;
     if (D.S > 1) {                      // split ts % S of output tile ts / S
@@ -1239,24 +1350,25 @@ VM_DEV void mma_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
       D.k0 = min(D.split * ksh, D.K);
       D.k1 = min(D.k0 + ksh, D.K);
     }
-    if (fast32) {
-      mma_tile32_fast<false>(A, &D, tile);
-    } else if (fast32r) {
-      mma_tile32_fast<true>(A, &D, tile);
-    } else if (fast) {
-      if (bf) mma_tile16_fast<true, false>(A, &D, tile);
-      else mma_tile16_fast<false, false>(A, &D, tile);
-    } else if (fastr) {
-      if (bf) mma_tile16_fast<true, true>(A, &D, tile);
-      else mma_tile16_fast<false, true>(A, &D, tile);
-    } else if (h16) {
-      if (T == 256) { if (bf) mma_tile16<256, true>(A, &D, tile); else mma_tile16<256, false>(A, &D, tile); }
-      else if (T == 128) { if (bf) mma_tile16<128, true>(A, &D, tile); else mma_tile16<128, false>(A, &D, tile); }
-      else { if (bf) mma_tile16<64, true>(A, &D, tile); else mma_tile16<64, false>(A, &D, tile); }
-    } else {
-      if (T == 256) mma_tile32<256>(A, &D, tile);
-      else if (T == 128) mma_tile32<128>(A, &D, tile);
-      else mma_tile32<64>(A, &D, tile);
+    uint32_t g, m0, n0;
+    tile_origin(D, tile, T, &g, &m0, &n0);
+    for (uint32_t q = 0; q < sub * sub; ++q) {
+      const uint32_t m = m0 + q / sub * E, n = n0 + q % sub * E, id = tile * D.subs + q;
+      if (m >= D.M || n >= D.N) continue;
+      switch (route) {
+        case 0: mma_pipe_tile<64, ELT_BF16>(A, &D, ops, id, g, m, n); break;
+        case 1: mma_pipe_tile<64, ELT_F16>(A, &D, ops, id, g, m, n); break;
+        case 2: mma_pipe_tile<64, ELT_F32>(A, &D, ops, id, g, m, n); break;
+        case 3: mma_pipe_tile<128, ELT_BF16>(A, &D, ops, id, g, m, n); break;
+        case 4: mma_pipe_tile<128, ELT_F16>(A, &D, ops, id, g, m, n); break;
+        case 5: mma_pipe_tile<128, ELT_F32>(A, &D, ops, id, g, m, n); break;
+        case 6: mma_tile16<64, true>(A, &D, id, g, m, n); break;
+        case 7: mma_tile16<64, false>(A, &D, id, g, m, n); break;
+        case 8: mma_tile32<64>(A, &D, id, g, m, n); break;
+        case 9: mma_tile16<128, true>(A, &D, id, g, m, n); break;
+        case 10: mma_tile16<128, false>(A, &D, id, g, m, n); break;
+        default: mma_tile32<128>(A, &D, id, g, m, n); break;
+      }
     }
   }
 }

@@ -68,6 +68,9 @@ constexpr uint32_t kArgmaxMaxSplits = 256;
 constexpr uint32_t kGemvMaxM = 8;
 // TOP_MMA: log2 of the K split (task p3 bits 28-31) at most.
 constexpr uint32_t kMmaMaxSplitLog2 = 5;
+// TOP_MMA p4 / p5 on the device: an operand view the loader resolved to strides
+// (vmrt.cpp `resolve_mma_view`), as this bit | the index of its five aux words.
+constexpr uint32_t kMmaStrided = 0x80000000u;
 constexpr int kMaxPorts = 256;          // power of two: handles mask the port index
 
 // Per-program control buffer: status words, then one arrival word per lane.

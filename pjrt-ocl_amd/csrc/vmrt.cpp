@@ -893,7 +893,8 @@ static uint64_t task_scratch_bytes(const Task& t, uint32_t mma_t) {
     const uint32_t code = (t.p[3] >> 24) & 0xF;
     const uint64_t T = code == 1 ? 64 : code == 2 ? 128 : code == 3 ? 256 : mma_t;
     const uint64_t tiles = ((t.p[0] + T - 1) / T) * ((t.p[1] + T - 1) / T) * std::max<uint64_t>(1, t.p[3] & 0xFFFFFF);
-    return (tiles * (uint64_t(1) << (t.p[3] >> 28)) * T * T + tiles) * 4;
+    // a 256-wide tile runs as four 128-wide ones, each with a counter of its own
+    return (tiles * (uint64_t(1) << (t.p[3] >> 28)) * T * T + tiles * (T == 256 ? 4 : 1)) * 4;
   }
   if ((t.tile_op & 0xFF) == TOP_ARGMAX_SEG && t.p[3] > 1) return (2ull * t.p[0] * t.p[3] + t.p[0]) * 4;
   if ((t.tile_op & 0xFF) == TOP_DECODE_ATTN && (t.p[4] >> 16) > 1) {
@@ -914,6 +915,56 @@ static std::vector<LaneSpan> device_lanes(const std::vector<LaneSpan>& lanes, co
     if (s.root_len && s.off < entries.size() && entries[s.off].task < ENT_FOR) s.pad = entries[s.off].task;
   }
   return out;
+}
+
+// A matmul operand's view as one stride per matrix dimension, when it has them:
+// logical [G, outer, inner] (A: G, M, K; B: G, K, N) with a constant stride along
+// each -- a transpose, a head's columns of a wider row, a slice -- and one of the two
+// matrix strides 1.  Appended to the device aux pool as {k-contiguous, row stride,
+// batch stride, offset, view}, so that a tile reads its operand by strides and
+// never walks the view.  Views that split a dimension over several strides, or
+// whose numbers leave 31 bits, stay views.  The loader has checked the view.
+static bool resolve_mma_view(const Program& P, uint32_t view, uint64_t G, uint64_t outer, uint64_t inner, bool is_a,
+                             std::vector<int32_t>* aux, uint32_t* word) {
+  const int32_t* x = P.aux.data() + (view - 1);
+  const int rank = x[0];
+  const int64_t off = x[1 + 2 * rank];
+  int e = rank - 1;
+  uint64_t dim = 1;              // what is left of the view dimension being read, and its stride
+  int64_t stride = 0;
+  auto take = [&](uint64_t size, int64_t* st) {
+    uint64_t got = 1;
+    *st = 0;
+    while (got < size) {
+      while (dim == 1) {
+        if (e < 0) return false;
+        dim = uint64_t(x[1 + e]);
+        stride = x[1 + rank + e];
+        --e;
+      }
+      const uint64_t want = size / got;
+      const uint64_t n = std::min(dim, want);
+      if (size % (got * n) || dim % n) return false;
+      if (got == 1) *st = stride;
+      else if (stride != *st * int64_t(got)) return false;
+      got *= n;
+      dim /= n;
+      stride *= int64_t(n);
+    }
+    return true;
+  };
+  int64_t si, so, sg;
+  if (!take(inner, &si) || !take(outer, &so) || !take(G, &sg)) return false;
+  const int64_t sk = is_a ? si : so, sr = is_a ? so : si;
+  const uint64_t nk = is_a ? inner : outer, nr = is_a ? outer : inner;
+  const bool kc = sk == 1 || nk == 1;
+  if (!kc && !(sr == 1 || nr == 1)) return false;
+  const int64_t ld = kc ? sr : sk;
+  for (int64_t v : {ld, sg, off})
+    if (v < 0 || v > INT32_MAX) return false;
+  *word = kMmaStrided | uint32_t(aux->size());
+  for (int64_t v : {int64_t(kc), ld, sg, off, int64_t(view)}) aux->push_back(int32_t(v));
+  return true;
 }
 
 // Host half of a load: parse, validate, choose ports, patch buffer ids to handles
@@ -1035,6 +1086,14 @@ static int prepare_program(vmrt_runtime* rt, vmrt_program* lp, const void* bytes
       const int32_t rank = P.aux[x];
       for (int d = 0; d < rank; ++d) aux[x + 1 + 3 * rank + d] = int32_t(handle(uint32_t(P.aux[x + 1 + 4 * rank + d])));
     }
+  }
+  // ---- matmul operand views with one stride per matrix dimension ----
+  for (Task& t : tasks) {
+    if ((t.tile_op & 0xFF) != TOP_MMA) continue;
+    const uint64_t M = t.p[0], N = t.p[1], K = t.p[2], G = std::max<uint32_t>(1, t.p[3] & 0xFFFFFF);
+    if (!M || !N || !K) continue;
+    if (t.p[4]) resolve_mma_view(P, t.p[4], G, M, K, true, &aux, &t.p[4]);
+    if (t.p[5]) resolve_mma_view(P, t.p[5], G, K, N, false, &aux, &t.p[5]);
   }
   // ---- patch control entries: cond buffer -> handle, pad -> cond format ----
   std::vector<Entry>& entries = pr->entries;

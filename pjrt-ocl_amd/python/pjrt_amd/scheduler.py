@@ -480,7 +480,8 @@ def instr_to_task(ins: V.Instr, prog: V.VMProgram, cfg: DeviceConfig) -> V.Task:
         else:
             code = V.MMA_TILE_CODES.get(ins.mma_tile, 0)
             if not code and cfg.mma_autotile:
-                code = V.MMA_TILE_CODES[_auto_mma_tile(M, N, G, cfg, adt, K, bool(aview or bview))]
+                code = V.MMA_TILE_CODES[_auto_mma_tile(M, N, G, cfg, adt, K, bool(aview or bview),
+                                                       not aview and _b_rows_contiguous(bview, prog, K))]
             edge = V.MMA_CODE_TILE.get(code, cfg.mma_t)
             split = mma_split_log2(M, N, K, G, edge, adt, cfg)
             t = V.Task(V.TOP_MMA, ins.dst, ins.a, ins.b, M, N, K,
@@ -493,36 +494,52 @@ def instr_to_task(ins: V.Instr, prog: V.VMProgram, cfg: DeviceConfig) -> V.Task:
     return t
 
 
+def _b_rows_contiguous(bview: int, prog: V.VMProgram, K: int) -> bool:
+    """Whether B [K, N] is read through a view with k contiguous and 16-byte rows
+    of a 16-bit type (x @ W.T: the fast tile's transposed form)."""
+    if not bview:
+        return False
+    x = prog.aux[bview - 1:bview + 5]
+    return x[0] == 2 and x[1] == K and x[3] == 1 and x[4] % 8 == 0 and x[5] % 8 == 0
+
+
 def _auto_mma_tile(M: int, N: int, G: int, cfg: DeviceConfig, adt: int = V.DT_F32, K: int = 0,
-                   views: bool = False) -> int:
-    """Largest output tile edge whose tile count still covers the lanes (big
-    tiles raise MFMA arithmetic intensity; small matmuls need the parallelism).
-    A 16-bit matmul the 256-wide fast tile takes (no operand view; K and N
-    multiples of 8) keeps 256 down to an eighth of the lanes: measured on MI355X,
-    bf16 1536^3 0.045 ms against 0.113 with the general tile the count rule picks,
-    3072^3 0.073 against 0.248, 2048^3 0.054 against 0.068; at 1024^3 (16 tiles)
-    the general tiles win, 0.030 against 0.034.  A long K (>= 4096) with at most
-    a sixth of the lanes' worth of 256-wide tiles takes 128-wide tiles instead,
-    which the K split then spreads over the lanes (one 256 x 256 x 4096 tile is
-    ~90 us of one CU's matrix cores): bf16 256x4096x4096 0.058 ms against 0.095,
-    512x2048x4096 0.058 against 0.095, 128x4096x4096 0.051 against 0.059,
-    512x4096x4096 0.079 against 0.088, 512x4096x11008 0.154 against 0.207; with
-    48 or more 256-wide tiles (768x4096x4096, 384x8192x4096) or K <= 3072 the
-    rules above win.  Where the 64-wide tiles fit the lanes in one round they
-    take it (their 128-deep K slabs and transposed B reads): 256x4096x4096
-    0.042 ms against 0.053 with 128, 128x4096x4096 0.036 against 0.049; with
-    more than a round of them (512x4096x11008) 128 stays ahead, 0.125 against
-    0.186."""
-    t256 = math.ceil(M / 256) * math.ceil(N / 256) * G
-    fast16 = adt in (V.DT_BF16, V.DT_F16) and not views and K >= 8 and K % 8 == 0 and N % 8 == 0
-    if fast16 and K >= 4096 and t256 * 6 < cfg.nlanes:
-        return 64 if math.ceil(M / 64) * math.ceil(N / 64) * G <= cfg.nlanes else 128
-    if fast16 and t256 * 8 >= cfg.nlanes:
+                   views: bool = False, b_rows: bool = False) -> int:
+    """Output tile edge of a matmul.  A 256-wide tile has the most arithmetic per
+    byte and its own fast kernels, but few of them leave lanes idle, and one such
+    tile of K = 4096 is ~90 us of a CU; the 64- and 128-wide ones stream K through
+    four LDS stages and cost ~8 us plus 0.9-1.8 us per 1024 k (f32: x 4).  Measured
+    on MI355X (us, 64 / 128 / 256-wide, K split where the rule below splits):
+
+      16-bit 1024^3             14.9 / 34.5 / 30.9    512x768x2304 19.6 / 25.8 / 26.9
+             1024x784x2048      22.3 / 32.7 / 31.7    512x3072x768 22.3 / 36.0 / 66.6
+             2048^3             63.5 / 33.4 / 52.2    512x768x32000 117 / 73.7 / 41.8
+      f32    1024^3             31.0 / 46.9 / 264     2048^3       180 / 146 / 519
+             512x768x32000      304 / 237 / 212       1001x777x1130 57 / 58 / 274
+
+    So: the largest edge whose tiles cover the lanes, with these exceptions for
+    operands the fast tiles take (no view; K and N multiples of 8, f32 of 4; a
+    16-bit B may be k-contiguous, ``b_rows``): 256 already at seven eighths of the
+    lanes; for 16-bit and K > 1024 down to an eighth of them (1536^3: 0.045 ms, with
+    the general tiles of the time 0.113; 3072^3 0.073) unless the 128-wide tiles
+    fill at least seven eighths of one round; and for K >= 4096 with at most a
+    sixth of the lanes' worth of 256-wide tiles, 128, or 64 where those fit the
+    lanes in one round (the K split then spreads them: 512x4096x11008 0.125 ms
+    against 0.186 with 64 and 0.207 with 256; 256x4096x4096 0.042 with 64)."""
+    t256, t128, t64 = (math.ceil(M / t) * math.ceil(N / t) * G for t in (256, 128, 64))
+    n = cfg.nlanes
+    h16 = adt in (V.DT_BF16, V.DT_F16)
+    per = 8 if h16 else 4
+    fast = (not views or (h16 and b_rows)) and K >= per and K % per == 0 and N % per == 0
+    if fast and t256 * 8 >= 7 * n:
         return 256
-    for t in (256, 128, 64):
-        if math.ceil(M / t) * math.ceil(N / t) * G >= cfg.nlanes:
-            return t
-    return 64
+    if fast and h16 and not views:
+        if K >= 4096 and t256 * 6 < n:
+            return 64 if t64 <= n else 128
+        if K > 1024 and t256 * 8 >= n and not 7 * n <= 8 * t128 <= 8 * n:
+            return 256
+    # a 256-wide tile outside the fast paths is four 128-wide ones
+    return 128 if t128 >= n else 64
 
 
 def mma_split_log2(M: int, N: int, K: int, G: int, edge: int, adt: int, cfg: DeviceConfig) -> int:
@@ -534,15 +551,24 @@ def mma_split_log2(M: int, N: int, K: int, G: int, edge: int, adt: int, cfg: Dev
     on its own loads only once per slab, so the loads of a deep, narrow product
     (config 1's [256, 512] x [512, 64]: four 64 x 64 tiles) no longer run one
     slab after another on a few lanes.  256-wide tiles are never split (they
-    cover large outputs, and their combine would hold 64 float4 per thread)."""
+    cover large outputs, and their combine would hold 64 float4 per thread).
+    With more tiles than that, a long K is still split 2 or 4 ways where the last
+    round is nearly empty (288 tiles on 256 lanes) and the rounds saved are worth
+    the combine: a tile costs about 1.3 us plus its K loop (64-wide: 7.4 us per
+    1024 k in 16 bits, 23 in f32; 128-wide: three times that), a split 3 us more."""
     if not cfg.mma_splitk:
         return 0
     tiles = math.ceil(M / edge) * math.ceil(N / edge) * max(1, G)
     slab = 16 if adt == V.DT_F32 else 32
-    if tiles * 2 > cfg.nlanes or K < 4 * slab:
+    if K < 4 * slab or edge == 256:
         return 0
-    if edge == 256:
-        return 0
+    if tiles * 2 > cfg.nlanes:
+        per_k = (0.023 if adt == V.DT_F32 else 0.0074) * (3 if edge == 128 else 1)
+
+        def cost(lg):
+            return math.ceil((tiles << lg) / cfg.nlanes) * (1.3 + (3.0 if lg else 0.0) + per_k * K / (1 << lg))
+        best = min((0, 1, 2), key=cost)
+        return best if cost(best) <= 0.85 * cost(0) else 0
     lg = 0
     while (lg < V.MMA_MAX_SPLIT_LOG2 and tiles << (lg + 1) <= cfg.nlanes
            and math.ceil(K / (1 << (lg + 1))) >= 2 * slab):

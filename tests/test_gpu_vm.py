@@ -623,6 +623,65 @@ def test_dot_split_k_exact(dt, Gb, M, K, N):
         lp.close()
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("Gb,M,K,N,tile", [(1, 200, 520, 136, 64), (1, 264, 72, 392, 128), (2, 129, 200, 72, 64),
+                                           (1, 61, 131, 77, 64), (1, 259, 333, 131, 128), (3, 70, 9, 67, 64),
+                                           (1, 300, 261, 515, 256), (1, 64, 1100, 64, 0), (1, 8, 8, 9, 64)])
+def test_dot_operand_layouts_exact(dt, ta, tb, Gb, M, K, N, tile):
+    """The 64- and 128-wide tiles with each operand k-contiguous or
+    row-contiguous (a transposed view), in whole 16-byte chunks (sizes multiples
+    of 8: stages go global -> LDS directly; K one, several and a partial stage)
+    and in odd sizes (through registers, chunks cut at the operands' ends), a
+    batch, a K split (tile 0: the scheduler's choice), and a 256-wide tile done
+    as four.  Integer-valued operands give the exact result, whose bias and
+    residual epilogue reads ragged rows."""
+    rng = np.random.default_rng(79)
+    a = rng.integers(-3, 4, (Gb, M, K)).astype(np.float32)
+    b = rng.integers(-3, 4, (Gb, K, N)).astype(np.float32)
+    res = rng.integers(-9, 10, (Gb, M, N)).astype(np.float32)
+    g = G.Graph()
+    sa, sb = ((Gb, K, M) if ta else a.shape), ((Gb, N, K) if tb else b.shape)
+    x, y, r = g.input(sa, dt), g.input(sb, dt), g.input(res.shape)
+    if ta:
+        x = g.transpose_view(x, (0, 2, 1))
+    if tb:
+        y = g.transpose_view(y, (0, 2, 1))
+    g.output(g.dot(x, y, tile=tile, residual=r, epilogue=[(V.SUB_ADD, 1, 0.0, 0.0), (V.SUB_MAX, 3, 0.5, 0.0)]))
+    blob, _ = blob_for(g.build())
+    print(f"[gpu] case: layouts {dt} ta={ta} tb={tb} G={Gb} M={M} K={K} N={N} tile={tile}", file=sys.stderr, flush=True)
+    args = [np.ascontiguousarray(a.transpose(0, 2, 1)) if ta else a, np.ascontiguousarray(b.transpose(0, 2, 1)) if tb else b, res]
+    want = np.maximum(np.matmul(a.astype(np.float64), b.astype(np.float64)) + res, 0.5)
+    for _ in range(2):
+        np.testing.assert_array_equal(run_gpu(blob, args)[0], want)
+
+
+def test_dot_operand_slices_exact():
+    """Operands that are columns of a wider row (heads of a fused projection) and
+    a chunk-wise view with heads split over two strides, as strided matrices and
+    through their view."""
+    rng = np.random.default_rng(80)
+    H, T, hd = 3, 150, 64
+    qkv = rng.integers(-3, 4, (T, 3 * H * hd)).astype(np.float32)
+    att = rng.integers(-3, 4, (H, T, hd)).astype(np.float32)
+    w = rng.integers(-3, 4, (H * hd, 100)).astype(np.float32)
+    w8 = np.ascontiguousarray(np.pad(w, ((0, 0), (0, 4))))
+    q = qkv[:, :H * hd].reshape(T, H, hd).transpose(1, 0, 2).astype(np.float64)
+    k = qkv[:, H * hd:2 * H * hd].reshape(T, H, hd).transpose(1, 0, 2).astype(np.float64)
+    rows = att.transpose(1, 0, 2).reshape(T, H * hd).astype(np.float64)
+    for dt in ("bf16", "f32"):
+        g = G.Graph()
+        xq, xa, xw, xw8 = g.input(qkv.shape, dt), g.input(att.shape, dt), g.input(w.shape, dt), g.input(w8.shape, dt)
+        vq = g.view(xq, (H, T, hd), (hd, 3 * H * hd, 1), 0)
+        vk = g.view(xq, (H, hd, T), (hd, 1, 3 * H * hd), H * hd)
+        va = G.Tensor(xa.buf, (T, H * hd), xa.dtype, view=g.transpose_view(xa, (1, 0, 2)).view)
+        g.output(g.dot(vq, vk), g.dot(va, xw), g.dot(va, xw8))
+        got = run_gpu(blob_for(g.build())[0], [qkv, att, w, w8])
+        np.testing.assert_array_equal(got[0], np.matmul(q, k.transpose(0, 2, 1)))
+        np.testing.assert_array_equal(got[1], rows @ w)
+        np.testing.assert_array_equal(got[2], rows @ w8)
+
+
 def test_dot_fast_path_random_bf16():
     rng = np.random.default_rng(1003)
     M = K = N = 1024
