@@ -1296,8 +1296,8 @@ VM_DEV void mma_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   hi = min(hi, D.tm * D.tn * D.G * D.S);
   const bool h16 = D.adt == DT_BF16 || D.adt == DT_F16, bf = D.adt == DT_BF16;
   const bool epi_ok = (D.dt == DT_F32 || D.dt == DT_BF16 || D.dt == DT_F16) && epi_inline_ok(A, D.epi);
-  // a K split's share: whole slabs of the pipelined tiles (64 16-bit or 32 f32 k)
-  const uint32_t bk = h16 ? 64u : 32u;
+  // a K split's share: a multiple of 32 (16-bit) or 16 (f32) k
+  const uint32_t bk = h16 ? uint32_t(kBK16) : uint32_t(kBK32);
   const uint32_t ksh = ((D.K + D.S - 1) / D.S + bk - 1) / bk * bk;
   // 256-wide tiles: the big square GEMMs' fast paths.  Ragged shapes need 16-byte
   // rows (K, N multiples of 8, f32: of 4) and offsets within 32 bits.

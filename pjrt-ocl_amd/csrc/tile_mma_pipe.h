@@ -10,7 +10,7 @@
 // (x . W^T: a tied embedding's logits, the gradient of an input) or in neither
 // (x^T . g: the gradient of a weight), and each operand keeps its own layout in LDS:
 //   k-contiguous (kc): T rows of 128 bytes (64 16-bit or 32 f32 k); the eight
-//     16-byte chunks of row r at slots chunk ^ aswz(r); a fragment is one
+//     16-byte chunks of row r at slots chunk ^ kc_swz(r); a fragment is one
 //     ds_read_b128;
 //   row-contiguous (rc): 64 (16-bit) or 32 (f32) k rows of T elements, slots
 //     chunk ^ swz(k); a 16-bit fragment is two ds_read_b64_tr_b16, an f32 one a
@@ -103,9 +103,19 @@ struct Pipe {
   static constexpr uint32_t kRowC = kRowB / 16;             // its chunks
 };
 
+// f32: MFMA step kk of a 16-deep slab takes k = kk in lanes 0-31 and k = 8 + kk in
+// lanes 32-63, as every f32 tile here does, so the tiles' sums are the same bits
+// (a sum near 0 decides a relu's gradient).  The two halves of a wave then read
+// chunks c and c ^ 2 of their rows, and rows k and k + 8: eight consecutive rows of
+// one parity take swizzles {0, 1, 4, 5} or {2, 3, 6, 7}.
+template <int ELT>
+VM_DEV uint32_t kc_swz(uint32_t r) {
+  if constexpr (ELT == ELT_F32) return ((r >> 1) & 1) | (((r >> 3) & 1) << 1) | (((r >> 2) & 1) << 2);
+  else return aswz(r);
+}
 template <int T, int ELT>
 VM_DEV uint32_t rc_swz(uint32_t k) {
-  if constexpr (ELT == ELT_F32) return 8 * ((k >> 2) & 1);
+  if constexpr (ELT == ELT_F32) return 8 * ((k >> 3) & 1);
   else if constexpr (T == 128) return 4 * (k & 3);
   else return 4 * ((k >> 1) & 1);
 }
@@ -120,9 +130,9 @@ struct PipeSrc {
   uint32_t ld, k1;
   uint32_t off[P::kRounds]; // kc: row byte offset; rc: row byte offset of the round within a full sub-slab + column bytes
   uint32_t kq;              // kc: first k of this lane's chunk in a sub-slab; rc: its k row in round 0
-  uint32_t cut;             // rc, through registers: elements of the chunk past R
+  uint32_t cut[P::kRounds]; // rc, through registers: elements of the chunk past R
   bool edge;                // some lane's cut is not 0
-  uint32_t colb;            // rc: column byte offset (clamped into the operand)
+  uint32_t colb[P::kRounds];   // rc: column byte offset (clamped into the operand)
   // MOP_RUNS
   ViewMap map;
   uint32_t lin[P::kRounds];
@@ -132,12 +142,11 @@ struct PipeSrc {
     const uint32_t l = threadIdx.x & 63, w = threadIdx.x >> 6;
     ld = o.ld;
     k1 = k1_;
-    cut = 0;
     edge = false;
     if constexpr (KC) {
       base = o.p + (o.gs * g + uint64_t(r0) * ld) * P::kEsz;
       const uint32_t row0 = 8 * w + (l >> 3);
-      kq = ((l & 7) ^ aswz(row0)) * P::kPer;
+      kq = ((l & 7) ^ kc_swz<ELT>(row0)) * P::kPer;
 #pragma unroll
       for (int j = 0; j < P::kRounds; ++j) {
         const uint32_t row = min(row0 + 32 * j + r0, o.R - 1);
@@ -150,15 +159,16 @@ struct PipeSrc {
       }
     } else {
       base = o.p + o.gs * g * P::kEsz;
-      constexpr uint32_t kPerRound = 1024 / P::kRowB * 4;   // k rows of one round of the block
       kq = (1024 / P::kRowB) * w + l / P::kRowC;
-      const uint32_t c = ((l % P::kRowC) ^ rc_swz<T, ELT>(kq)) * P::kPer + r0;
-      const uint32_t cc = min(c, o.R - P::kPer);
-      cut = c - cc;
-      edge = __builtin_amdgcn_ballot_w64(cut != 0) != 0;
-      colb = cc * P::kEsz;
 #pragma unroll
-      for (int j = 0; j < P::kRounds; ++j) off[j] = (kq + kPerRound * j) * ld * P::kEsz + colb;
+      for (int j = 0; j < P::kRounds; ++j) {
+        const uint32_t c = ((l % P::kRowC) ^ rc_swz<T, ELT>(krow(kq, j))) * P::kPer + r0;
+        const uint32_t cc = min(c, o.R - P::kPer);
+        cut[j] = c - cc;
+        colb[j] = cc * P::kEsz;
+        off[j] = krow(kq, j) * ld * P::kEsz + colb[j];
+        edge |= __builtin_amdgcn_ballot_w64(c != cc) != 0;
+      }
     }
   }
   // k row of round j (rc)
@@ -173,7 +183,7 @@ struct PipeSrc {
       if constexpr (RUNS) return uint32_t(view_at(map, aux, view, lin[j] + kk)) * P::kEsz;
       return off[j] + kk * P::kEsz;
     } else {
-      return (min(k + krow(kq, j), k1 - 1) - k) * ld * P::kEsz + colb;
+      return (min(k + krow(kq, j), k1 - 1) - k) * ld * P::kEsz + colb[j];
     }
   }
   // sub-slab at k (below k1) into LDS at st
@@ -207,7 +217,7 @@ struct PipeSrc {
     for (int j = 0; j < P::kRounds; ++j) {
       uint32_t o;
       if constexpr (KC) o = off[j] + min(k + kq, k1 - P::kPer) * P::kEsz;
-      else o = (min(k + krow(kq, j), k1 - 1) - min(k, k1 - 1)) * ld * P::kEsz + colb;
+      else o = (min(k + krow(kq, j), k1 - 1) - min(k, k1 - 1)) * ld * P::kEsz + colb[j];
       r[j] = *(const VM_G v4u_any*)(b + o);
     }
   }
@@ -234,7 +244,7 @@ struct PipeSrc {
       if constexpr (KC) {
         v = shift_out(r[j], min(k + kq - min(k + kq, k1 - P::kPer), 16u));
       } else {
-        v = shift_out(r[j], min(cut, 16u));
+        v = shift_out(r[j], min(cut[j], 16u));
         if (k + krow(kq, j) >= k1) v = v4u_make(0, 0, 0, 0);
       }
       *(lds_v4u*)uintptr_t(at + 4096 * j) = v;
@@ -253,9 +263,12 @@ struct PipeFrag {
     if constexpr (KC) {
       const uint32_t r = w2 * (T / 2) + (lane & 31);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) a[q] = r * 128 + (((2 * q + (lane >> 5)) ^ aswz(r)) * 16);
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t c = ELT == ELT_F32 ? 4 * (q >> 1) + (q & 1) + 2 * (lane >> 5) : 2 * q + (lane >> 5);
+        a[q] = r * 128 + ((c ^ kc_swz<ELT>(r)) * 16);
+      }
     } else if constexpr (ELT == ELT_F32) {
-      const uint32_t c = w2 * (T / 2) + (lane & 31), row = 4 * (lane >> 5);
+      const uint32_t c = w2 * (T / 2) + (lane & 31), row = 8 * (lane >> 5);
 #pragma unroll
       for (int b = 0; b < P::kB; ++b)
         a[b] = row * P::kRowB + ((((c + 32 * b) >> 2) ^ rc_swz<T, ELT>(row)) * 16) + (c & 3) * 4;
@@ -279,14 +292,14 @@ struct PipeFrag {
       return __builtin_bit_cast(u16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
   }
-  // f32: the four values of block b for k steps 8 q + {0, 1, 2, 3} (+ 4 in lanes 32-63)
+  // f32: the four values of block b for k 16 (q / 2) + 4 (q % 2) + {0, 1, 2, 3} (+ 8 in lanes 32-63)
   VM_DEV v4f frag32(const lds_u8* S, int q, int b) const {
     typedef __attribute__((address_space(3))) v4f lds_v4f;
     typedef __attribute__((address_space(3))) float lds_f;
     if constexpr (KC) {
       return *(const lds_v4f*)(S + a[q] + 4096 * b);
     } else {
-      const lds_u8* p = S + a[b] + 8 * q * P::kRowB;
+      const lds_u8* p = S + a[b] + (16 * (q >> 1) + 4 * (q & 1)) * P::kRowB;
       return v4f_make(*(const lds_f*)p, *(const lds_f*)(p + P::kRowB), *(const lds_f*)(p + 2 * P::kRowB),
                       *(const lds_f*)(p + 3 * P::kRowB));
     }
