@@ -1019,18 +1019,30 @@ class TaskRunner:
     # 15: strided partial-axis reduce
     def top15(self, t, lo, hi):
         n_out, red, inner, kind = t.p[0], t.p[1], t.p[2], t.p[3]
-        a0, a1 = lo * self.ts, min(hi * self.ts, n_out)
+        if t.p[4]:
+            # extension: tile t is split t % p4 of the 64 outputs at 64 (t // p4);
+            # they are written once all their splits have run (in any order)
+            for tile in range(lo, hi):
+                key = (id(t), tile // t.p[4])
+                self.splits[key] = self.splits.get(key, 0) + 1
+                if self.splits[key] == t.p[4]:
+                    del self.splits[key]
+                    self._red_strided(t, 64 * key[1], min(64 * key[1] + 64, n_out))
+            return
+        self._red_strided(t, lo * self.ts, min(hi * self.ts, n_out))
+
+    def _red_strided(self, t, a0, a1):
+        n_out, red, inner, kind = t.p[0], t.p[1], t.p[2], t.p[3]
         if a0 >= a1:
             return
-        outer = n_out // inner
-        if t.dt in INTS or t.dt == BOOL:
-            src = self.m.view(t.a, t.dt)[:outer * red * inner].reshape(outer, red, inner)
-            r = reduce_np(src, kind, t.dt, axis=1).reshape(-1)
-            self.m.view(t.dst, t.dt)[a0:a1] = r[a0:a1]
+        ints = t.dt in INTS or t.dt == BOOL
+        q = np.arange(a0, a1)
+        src = self.m.view(t.a, t.dt if ints else t.adt)[:n_out * red].reshape(n_out // inner, red, inner)
+        src = src[q // inner, :, q % inner]               # [outputs, red]
+        if ints:
+            self.m.view(t.dst, t.dt)[a0:a1] = reduce_np(src, kind, t.dt, axis=1)
         else:
-            src = self.m.load_f(t.a, t.adt)[:outer * red * inner].reshape(outer, red, inner)
-            r = _red_float(src, kind, 1).reshape(-1)
-            self.m.store_f(t.dst, slice(a0, a1), r[a0:a1], t.dt)
+            self.m.store_f(t.dst, slice(a0, a1), _red_float(bf16_to_f32(src) if t.adt == BF16 else src, kind, 1), t.dt)
 
     # 16: data-dependent gather (gather.cl:108+)
     def top16(self, t, lo, hi):
@@ -1178,6 +1190,8 @@ def _whole_tiles(t: Task, ew_ts: int, mma_t: int) -> int:
     if t.top in (0, 2, 5, 6, 7, 8, 9, 13, 16, 17, 18):
         return max(1, -(-p[1] // ew_ts))
     if t.top == 15:
+        if t.p[4]:                      # extension: p4 splits of 64 outputs
+            return max(1, -(-t.p[0] // 64) * t.p[4])
         return max(1, -(-p[0] // ew_ts))
     if t.top == 1:
         T = {1: 64, 2: 128, 3: 256}.get((p[3] >> 24) & 0xF, mma_t)

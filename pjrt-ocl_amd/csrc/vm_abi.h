@@ -64,6 +64,8 @@ constexpr uint32_t kDecMaxSplits = 1024;
 constexpr uint32_t kDecSplitKeys = 64;
 // TOP_ARGMAX_SEG: splits per row at most.
 constexpr uint32_t kArgmaxMaxSplits = 256;
+// TOP_RED_STRIDED: row splits per block of 64 outputs (p4, extension) at most.
+constexpr uint32_t kRedMaxSplits = 64;
 // TOP_GEMV: rows (M) per task at most.
 constexpr uint32_t kGemvMaxM = 8;
 // TOP_MMA: log2 of the K split (task p3 bits 28-31) at most.

@@ -382,7 +382,7 @@ struct Checker {
       case TOP_EW: case TOP_GATHER: case TOP_IOTA_DIM: case TOP_SCATTER: case TOP_DYN_GATHER:
       case TOP_DYN_SCATTER: case TOP_MAP_REGION: case TOP_GATHER_INDEX:
         return std::max<uint64_t>(1, cdiv(t.p[1], ew_ts));
-      case TOP_RED_STRIDED: return std::max<uint64_t>(1, cdiv(t.p[0], ew_ts));
+      case TOP_RED_STRIDED: return std::max<uint64_t>(1, t.p[4] ? cdiv(t.p[0], 64) * t.p[4] : cdiv(t.p[0], ew_ts));
       case TOP_MMA: {
         const uint32_t code = (t.p[3] >> 24) & 0xF;
         const uint64_t T = code == 1 ? 64 : code == 2 ? 128 : code == 3 ? 256 : mma_t;
@@ -517,7 +517,9 @@ struct Checker {
       case TOP_RED_STRIDED: {
         const uint64_t n_out = t.p[0], red = t.p[1], inner = t.p[2];
         if (!inner || n_out % inner || t.p[3] > 6) return fail(ti, "strided reduce shape");
-        const uint32_t src_dt = (dt == DT_I32 || dt == DT_U32 || dt == DT_I64 || dt == DT_BOOL) ? dt : adt;
+        const bool ints = dt == DT_I32 || dt == DT_U32 || dt == DT_I64 || dt == DT_BOOL;
+        if (t.p[4] > kRedMaxSplits || (t.p[4] && (ints || !red || !n_out))) return fail(ti, "strided reduce splits");
+        const uint32_t src_dt = ints ? dt : adt;
         return (has(t.a, n_out / inner * red * inner, src_dt) && has(t.dst, n_out, dt)) ||
                fail(ti, "strided reduce operands");
       }
@@ -886,7 +888,8 @@ void vmrt_unload(vmrt_program* p) {
 
 // Scratch bytes a task needs (0: none): a split decode attention keeps one
 // partial (running max, sum, hd channels) per split and head, and one arrival
-// counter per head; a K-split matmul one f32 partial tile per split and output
+// counter per head; a split column reduction 64 partials per split and block of
+// outputs, and one counter per block; a K-split matmul one f32 partial tile per split and output
 // tile, and one arrival counter per output tile.
 static uint64_t task_scratch_bytes(const Task& t, uint32_t mma_t) {
   if ((t.tile_op & 0xFF) == TOP_MMA && (t.p[3] >> 28)) {
@@ -895,6 +898,10 @@ static uint64_t task_scratch_bytes(const Task& t, uint32_t mma_t) {
     const uint64_t tiles = ((t.p[0] + T - 1) / T) * ((t.p[1] + T - 1) / T) * std::max<uint64_t>(1, t.p[3] & 0xFFFFFF);
     // a 256-wide tile runs as four 128-wide ones, each with a counter of its own
     return (tiles * (uint64_t(1) << (t.p[3] >> 28)) * T * T + tiles * (T == 256 ? 4 : 1)) * 4;
+  }
+  if ((t.tile_op & 0xFF) == TOP_RED_STRIDED && t.p[4] > 1) {
+    const uint64_t blocks = (uint64_t(t.p[0]) + 63) / 64;
+    return (blocks * t.p[4] * 64 + blocks) * 4;
   }
   if ((t.tile_op & 0xFF) == TOP_ARGMAX_SEG && t.p[3] > 1) return (2ull * t.p[0] * t.p[3] + t.p[0]) * 4;
   if ((t.tile_op & 0xFF) == TOP_DECODE_ATTN && (t.p[4] >> 16) > 1) {

@@ -175,7 +175,7 @@ def n_tiles(task: V.Task, cfg: DeviceConfig) -> int:
                V.TOP_SCATTER_INDEX):
         return max(1, math.ceil(task.p1 / cfg.ew_ts))
     if top == V.TOP_RED_STRIDED:
-        return max(1, math.ceil(task.p0 / cfg.ew_ts))
+        return max(1, math.ceil(task.p0 / 64) * task.p4 if task.p4 else math.ceil(task.p0 / cfg.ew_ts))
     if top == V.TOP_MMA:
         t = mma_tile_edge(task, cfg)
         g = max(1, task.p3 & 0xFFFFFF)
@@ -271,6 +271,19 @@ def row_interleave(n_rows: int, cfg: DeviceConfig) -> int:
     if not cfg.ln_interleave or cfg.nlanes <= 1 or n_rows < 2 * cfg.nlanes or n_rows % cfg.nlanes:
         return 0
     return n_rows // cfg.nlanes
+
+
+def red_splits(n_out: int, red: int, dt: int, cfg: DeviceConfig) -> int:
+    """TOP_RED_STRIDED p4 (extension): tiles of 64 outputs, each over 1 / p4 of the
+    reduced rows; 0 (integer types): the reference's tiles of ew_ts outputs, which
+    gave a 2048-column sum one lane.  Rows are split while lanes would idle and a
+    split keeps 128 rows, one batch of its loads (1024 x 2048 f32: 32 blocks x 8)."""
+    if dt not in (V.DT_F32, V.DT_BF16, V.DT_F16) or n_out <= 0 or red <= 0:
+        return 0
+    s, blocks = 1, -(-n_out // 64)
+    while s < 64 and blocks * s * 2 <= cfg.nlanes and red >= 256 * s:
+        s *= 2
+    return s
 
 
 def argmax_splits(n_out: int, seg: int, cfg: DeviceConfig) -> int:
@@ -433,7 +446,8 @@ def instr_to_task(ins: V.Instr, prog: V.VMProgram, cfg: DeviceConfig) -> V.Task:
                    ins.imm & 0x0FFFFFFF, ins.imm >> 28)
     elif op == V.OP_REDUCE_STRIDED:
         t = V.Task(V.TOP_RED_STRIDED, ins.dst, ins.a, ins.a, ins.n,
-                   ins.imm & 0x0FFFFFFF, ins.imm2, ins.imm >> 28)
+                   ins.imm & 0x0FFFFFFF, ins.imm2, ins.imm >> 28,
+                   red_splits(ins.n, ins.imm & 0x0FFFFFFF, bufs[ins.dst].dtype, cfg))
     elif op == V.OP_SOFTMAX:
         t = V.Task(V.TOP_SOFTMAX_SEG, ins.dst, ins.a, ins.a, ins.n, ins.imm)
     elif op == V.OP_LAYERNORM:
