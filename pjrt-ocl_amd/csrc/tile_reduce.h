@@ -9,6 +9,8 @@
 // Float reductions accumulate in f32 through DPP wave reductions; integer ones are
 // exact.  Kinds: 0 sum, 1 max, 2 min, 3 prod, 4 and, 5 or, 6 xor.
 #pragma once
+#include <type_traits>
+
 #include "vm_math.h"
 
 namespace vm {
@@ -216,7 +218,7 @@ VM_TILE void red_seg_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
 // row phases added through LDS in a fixed order.  One thread per output and one
 // load at a time left a CU with 1 KiB in flight, and put a column sum of 8192 x 4096
 // f32, a tile, on one CU: 41.4 ms; now 30.4 us (4.4 TB/s, what bounds it).  1024 x
-// 2048 f32 inside a gradient step: 3029 -> 440 us for the step's two sums and the rest.
+// 2048 and 1024 x 256 f32 in the gradient step of an MLP: 3029 -> 440 us for the step.
 constexpr uint32_t kRedCols = 64, kRedBatch = 8;
 
 template <class Op, bool VEC>
@@ -854,66 +856,198 @@ VM_DEV void layernorm_rows(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   return ln_rows_vec<8>(A, ti, lo, hi);
 }
 
-// SOFTMAX_SEG rows: exp(x - max) / sum.
-template <int NV>
-VM_TILE void softmax_rows_vec(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
-  A = uargs(A);
+// SOFTMAX_SEG rows: exp(x - max) / sum, f32 arithmetic.
+//
+// Rows are read in groups of 4 elements with 16- or 8-byte accesses that need only
+// the element's own alignment, so odd row lengths stream like even ones; a row whose
+// length is not a multiple of 4 ends in a group that overlaps the one before (its
+// repeated elements count once in the sum and are stored twice, with one value).
+// Loads are not predicated (ln_load's reason): groups past the row re-read its last.
+// Three forms, by how many registers a row takes:
+//   up to 4096 elements: a wave per row, four rows in flight per CU and the next
+//     ones prefetched, DPP reductions and no block barrier;
+//   up to 32768: a row over the block's registers, the next row prefetched;
+//   longer: two passes over the row, the first keeping a running maximum and sum
+//     per thread.
+// Memory bounds them (MI355X, whole launches): 512 x 32000 f32 257 -> 34.9 us (3.75
+// TB/s: two rows per CU, so the first row's load and the last one's store overlap
+// nothing), 8192 x 4096 65 -> 53 (5.06), 4096 x 1000 20 -> 10.6, 1000 x 777 14.4 -> 6.9;
+// before, odd and long rows were read three times in single elements and a row of
+// any length took the whole block and two block barriers.
+template <bool IN16>
+struct RowRaw {
+  typedef typename std::conditional<IN16, v2u, v4f>::type Raw;
+  typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+  typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(2)));
+  static VM_DEV Raw load(const gbyte* row, uint32_t e) {
+    if constexpr (IN16) return *(const VM_G v2u_any*)(gcast<uint16_t>(row) + e);
+    else return *(const VM_G v4f_any*)(gcast<float>(row) + e);
+  }
+  static VM_DEV v4f value(Raw r, bool bf) {
+    if constexpr (IN16)
+      return bf ? v4f_make(__uint_as_float(r.x << 16), __uint_as_float(r.x & 0xFFFF0000u), __uint_as_float(r.y << 16),
+                           __uint_as_float(r.y & 0xFFFF0000u))
+                : v4f_make(f16_to_f32(r.x & 0xFFFF), f16_to_f32(r.x >> 16), f16_to_f32(r.y & 0xFFFF), f16_to_f32(r.y >> 16));
+    else return r;
+  }
+};
+VM_DEV void row_store(gbyte* row, uint32_t dt, uint32_t e, v4f v) {
+  typedef float v4f_any __attribute__((ext_vector_type(4), aligned(4)));
+  typedef uint32_t v2u_any __attribute__((ext_vector_type(2), aligned(2)));
+  if (dt == DT_F32) {
+    *(VM_G v4f_any*)(gcast<float>(row) + e) = v;
+  } else if (dt == DT_BF16) {
+    *(VM_G v2u_any*)(gcast<uint16_t>(row) + e) = v2u_make(pack_bf16x2(v.x, v.y), pack_bf16x2(v.z, v.w));
+  } else {
+    *(VM_G v2u_any*)(gcast<uint16_t>(row) + e) = v2u_make(f32_to_f16(v.x) | (uint32_t(f32_to_f16(v.y)) << 16),
+                                                          f32_to_f16(v.z) | (uint32_t(f32_to_f16(v.w)) << 16));
+  }
+}
+// A row of seg >= 4 elements in groups of 4: group q starts at element at(q); its
+// first dup(q) elements belong to the group before.
+struct RowGroups {
+  uint32_t seg, n;
+  VM_DEV explicit RowGroups(uint32_t s) : seg(s), n((s + 3) >> 2) {}
+  VM_DEV uint32_t at(uint32_t q) const { return min(4 * q, seg - 4); }
+  VM_DEV uint32_t dup(uint32_t q) const { return 4 * q - at(q); }
+};
+VM_DEV float sum4(v4f v, uint32_t dup) {
+  return (dup > 0 ? 0.0f : v.x) + (dup > 1 ? 0.0f : v.y) + ((dup > 2 ? 0.0f : v.z) + v.w);
+}
+
+// Rows r0, r0 + step, ... < r1, a row over the TH threads (64: the wave; kBlock: the
+// block), this thread's groups t, t + TH, ...
+template <int NV, bool IN16, int TH>
+VM_DEV void softmax_rows(Args A, uint32_t ti, uint32_t r0, uint32_t r1, uint32_t step) {
+  typedef RowRaw<IN16> R;
   const VM_K Task& t = task_of(A, ti);
   float* red = lds_f32();
-  const uint32_t seg = t.p[1];
+  const RowGroups G(t.p[1]);
   const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
+  const bool bf = adt == DT_BF16;
   const gbyte* a = resolve(A, t.a);
   gbyte* d = resolve(A, t.dst);
-  const uint32_t nv4 = seg >> 2;
-  Row<NV> x, xn;
-  row_load(x, a, adt, uint64_t(r0) * seg, nv4);
-  for (uint32_t r = r0; r < r1; ++r) {
-    if (r + 1 < r1) row_load(xn, a, adt, uint64_t(r + 1) * seg, nv4);
+  const uint32_t me = TH == 64 ? threadIdx.x & 63 : threadIdx.x;
+  const uint32_t dsz = dt == DT_F32 ? 4 : 2;
+  if (r0 >= r1) return;
+  typename R::Raw x[NV], xn[NV];
+  auto load = [&](typename R::Raw (&buf)[NV], uint32_t r) {
+    const gbyte* row = a + uint64_t(r) * G.seg * (IN16 ? 2 : 4);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) buf[k] = R::load(row, G.at(min(me + TH * k, G.n - 1)));
+  };
+  load(x, r0);
+  for (uint32_t r = r0; r < r1; r += step) {
+    load(xn, r + step < r1 ? r + step : r);
     float m = -INFINITY;
 #pragma unroll
-    for (int k = 0; k < NV; ++k)
-      if (threadIdx.x + k * kBlock < nv4) m = fmaxf(m, fmaxf(fmaxf(x.v[k].x, x.v[k].y), fmaxf(x.v[k].z, x.v[k].w)));
-    m = block_reduce(m, OpMax(), red);
+    for (int k = 0; k < NV; ++k) {
+      const v4f v = R::value(x[k], bf);
+      m = fmaxf(m, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+    }
+    if constexpr (TH == 64) m = wave_max(m);
+    else m = block_reduce(m, OpMax(), red);
+    v4f y[NV];
     float s = 0.0f;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      if (threadIdx.x + k * kBlock < nv4) {
-        x.v[k].x = __expf(x.v[k].x - m);
-        x.v[k].y = __expf(x.v[k].y - m);
-        x.v[k].z = __expf(x.v[k].z - m);
-        x.v[k].w = __expf(x.v[k].w - m);
-        s += (x.v[k].x + x.v[k].y) + (x.v[k].z + x.v[k].w);
-      }
+      const v4f v = R::value(x[k], bf);
+      y[k] = v4f_make(__expf(v.x - m), __expf(v.y - m), __expf(v.z - m), __expf(v.w - m));
+      const uint32_t q = me + TH * k;
+      s += q < G.n ? sum4(y[k], G.dup(q)) : 0.0f;
     }
-    s = block_reduce(s, OpSum(), red + kWaves);
+    if constexpr (TH == 64) s = wave_sum(s);
+    else s = block_reduce(s, OpSum(), red + kWaves);
     const float inv = 1.0f / s;
-    const uint64_t base = uint64_t(r) * seg;
+    gbyte* row = d + uint64_t(r) * G.seg * dsz;
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      const uint32_t q = threadIdx.x + k * kBlock;
-      if (q < nv4) st4(d, dt, base + 4ull * q, v4f_make(x.v[k].x * inv, x.v[k].y * inv, x.v[k].z * inv, x.v[k].w * inv));
+      const uint32_t q = me + TH * k;
+      if (q < G.n) row_store(row, dt, G.at(q), y[k] * inv);
     }
-    if (r + 1 < r1) x = xn;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) x[k] = xn[k];
   }
 }
 
-VM_TILE void softmax_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+// Rows too long for the registers: a running maximum and sum per thread, then a
+// second read (from L2 and the memory-side cache) to store.
+template <bool IN16>
+VM_DEV void softmax_rows_long(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
+  typedef RowRaw<IN16> R;
+  const VM_K Task& t = task_of(A, ti);
+  float* red = lds_f32();
+  const RowGroups G(t.p[1]);
+  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
+  const bool bf = adt == DT_BF16;
+  constexpr int U = 8;
+  for (uint32_t r = r0; r < r1; ++r) {
+    const gbyte* src = resolve(A, t.a) + uint64_t(r) * G.seg * (IN16 ? 2 : 4);
+    gbyte* row = resolve(A, t.dst) + uint64_t(r) * G.seg * (dt == DT_F32 ? 4 : 2);
+    float m = -INFINITY, s = 0.0f;
+    for (uint32_t q0 = threadIdx.x; q0 < G.n; q0 += U * kBlock) {
+      typename R::Raw x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = R::load(src, G.at(min(q0 + u * kBlock, G.n - 1)));
+      float nm = m;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const v4f v = R::value(x[u], bf);
+        nm = fmaxf(nm, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+      }
+      const float at = nm == -INFINITY ? 0.0f : nm;      // nothing but -inf so far: every term is 0
+      s *= __expf(m - at);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const v4f v = R::value(x[u], bf);
+        const uint32_t q = q0 + u * kBlock;
+        s += q < G.n ? sum4(v4f_make(__expf(v.x - at), __expf(v.y - at), __expf(v.z - at), __expf(v.w - at)), G.dup(q)) : 0.0f;
+      }
+      m = nm;
+    }
+    const float M = block_reduce(m, OpMax(), red);
+    s = block_reduce(m == -INFINITY ? 0.0f * s : s * __expf(m - M), OpSum(), red + kWaves);
+    const float inv = 1.0f / s;
+    for (uint32_t q0 = threadIdx.x; q0 < G.n; q0 += U * kBlock) {
+      typename R::Raw x[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) x[u] = R::load(src, G.at(min(q0 + u * kBlock, G.n - 1)));
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const v4f v = R::value(x[u], bf);
+        const uint32_t q = q0 + u * kBlock;
+        if (q < G.n)
+          row_store(row, dt, G.at(q), v4f_make(__expf(v.x - M), __expf(v.y - M), __expf(v.z - M), __expf(v.w - M)) * inv);
+      }
+    }
+  }
+}
+
+template <bool IN16>
+VM_DEV void softmax_dispatch(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  const uint32_t n = (task_of(A, ti).p[1] + 3) >> 2, wave = uni(threadIdx.x >> 6);
+  if (n <= 4 * 64) softmax_rows<4, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (n <= 16 * 64) softmax_rows<16, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (n <= 8 * kBlock) softmax_rows<8, IN16, kBlock>(A, ti, lo, hi, 1);
+  else if (n <= 32 * kBlock) softmax_rows<32, IN16, kBlock>(A, ti, lo, hi, 1);
+  else softmax_rows_long<IN16>(A, ti, lo, hi);
+}
+
+// A leaf with its row forms inlined, as layernorm_tiles.
+VM_LEAF void softmax_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   A = uargs(A);
   const VM_K Task& t = task_of(A, ti);
   float* red = lds_f32();
   const uint32_t n_out = t.p[0], seg = t.p[1];
   const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
-  hi = min(hi, n_out);
+  lo = uni(lo);
+  hi = uni(min(hi, n_out));
   if (lo >= hi) return;
   const gbyte* a = resolve(A, t.a);
   gbyte* d = resolve(A, t.dst);
-  if (row_vec_ok(seg, a, d, adt, dt)) {
-    const uint32_t nv4 = seg >> 2;
-    if (nv4 <= 1 * kBlock) return softmax_rows_vec<1>(A, ti, lo, hi);
-    if (nv4 <= 2 * kBlock) return softmax_rows_vec<2>(A, ti, lo, hi);
-    if (nv4 <= 4 * kBlock) return softmax_rows_vec<4>(A, ti, lo, hi);
-    return softmax_rows_vec<8>(A, ti, lo, hi);
-  }
+  const bool out_ok = dt == DT_F32 || dt == DT_BF16 || dt == DT_F16;
+  if (out_ok && seg >= 4 && adt == DT_F32) return softmax_dispatch<false>(A, ti, lo, hi);
+  if (out_ok && seg >= 4 && (adt == DT_BF16 || adt == DT_F16)) return softmax_dispatch<true>(A, ti, lo, hi);
   for (uint32_t r = lo; r < hi; ++r) {
     const uint64_t base = uint64_t(r) * seg;
     float m = -INFINITY;

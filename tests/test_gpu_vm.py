@@ -241,6 +241,33 @@ def test_float_reductions(kind):
         assert_rel(gv, wv, 1e-5 if kind != 3 else 1e-4, 1e-5, f"kind {kind} out {k}")
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape,axis", [((1000, 777), 0), ((4099, 68), 0), ((129, 2048), 0), ((5, 300, 36), 1),
+                                        ((3, 7, 5), 1), ((2, 3), 0), ((1, 70), 0), ((700, 1), 0), ((33, 64, 4096), 1)])
+def test_column_reductions_exact(dt, shape, axis):
+    """Reductions over an outer or middle axis: blocks of 64 outputs whose rows are
+    split over lanes (4099 rows: 64 splits of two blocks; 129: no split), in 16-byte
+    and single-element reads, ragged blocks, blocks over several outer indices and
+    outputs fewer than one read.  Small integers make the sum exact; max and min are
+    exact anyway.  Twice, so the second run finds the split counters reset."""
+    rng = np.random.default_rng(24)
+    a = rng.integers(-2, 3, shape).astype(np.float32)
+    if dt != "f32":                       # sums within the 8 bits of a bf16 result
+        a = np.where(rng.random(shape) < 64 / max(64, 4 * shape[axis]), a, 0).astype(np.float32)   # (no -0)
+    g = G.Graph()
+    x = g.input(shape, dt)
+    g.output(*(g.reduce_axis(x, axis, k) for k in (0, 1, 2)))
+    blob, _ = blob_for(g.build())
+    print(f"[gpu] case: column reduction {dt} {shape} axis {axis}", file=sys.stderr, flush=True)
+    arg = a if dt == "f32" else a.astype(np.float16) if dt == "f16" else vmref.f32_to_bf16(a)
+    want = [a.sum(axis, dtype=np.float64), a.max(axis), a.min(axis)]
+    oracle = vmref.execute_schedule(blob, [arg], check_order=False)
+    for _ in range(2):
+        for gv, wv, ov in zip(run_gpu(blob, [arg]), want, oracle):
+            np.testing.assert_array_equal(as_f32(gv, V.DT_BY_NAME[dt]), wv)
+            np.testing.assert_array_equal(np.asarray(gv), np.asarray(ov).reshape(np.shape(gv)))
+
+
 @pytest.mark.parametrize("dt", ["i32", "u32", "i64", "bool"])
 @pytest.mark.parametrize("kind", [0, 1, 2, 3, 4, 5, 6])
 def test_integer_reductions_bit_exact(dt, kind):
@@ -295,6 +322,40 @@ def test_softmax_and_layernorm_rows(seg):
     got, want = run_both(g.build(), [a])
     assert_rel(got[0], want[0], 2e-5, 1e-9, "softmax")
     assert_rel(got[1], want[1], 1e-5, 2e-5, "layernorm core")
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("seg", [3, 4, 5, 255, 1023, 1025, 4095, 4097, 8191, 8193, 32766, 32769, 50257])
+def test_softmax_row_forms(dt, seg):
+    """Each row form (wave, block, two passes in memory) at the edges of its
+    lengths, odd lengths (the last group of four overlaps the one before), rows
+    with -inf entries (one thread's share all -inf among them), a row of -inf
+    only (NaN) and a +inf (NaN in that row).  f32 arithmetic: each exponential is
+    within 2 ulp plus its argument's rounding (|x - max| <= 40: 40 * 2^-24), the sum's
+    error smaller, so 2e-5 of the float64 value; a 16-bit result adds its rounding."""
+    rng = np.random.default_rng(52)
+    rows = 9
+    a = (rng.standard_normal((rows, seg)) * 4).astype(np.float32)
+    a[1, rng.random(seg) < 0.5] = -np.inf
+    a[2, : seg - seg // 4] = -np.inf
+    a[3] = -np.inf
+    a[4, seg // 2] = np.inf
+    if dt == "bf16":
+        a = vmref.bf16_to_f32(vmref.f32_to_bf16(a))
+    elif dt == "f16":
+        a = a.astype(np.float16).astype(np.float32)
+    g = G.Graph()
+    x = g.input(a.shape, dt)
+    g.output(g.softmax_last(x), g.softmax_last(x, out_dtype="f32"))
+    blob, _ = blob_for(g.build())
+    print(f"[gpu] case: softmax {dt} {seg}", file=sys.stderr, flush=True)
+    got = run_gpu(blob, [a])
+    with np.errstate(invalid="ignore"):
+        e = np.exp(a.astype(np.float64) - a.max(1, keepdims=True))
+        want = e / e.sum(1, keepdims=True)
+    ulp = {"f32": 0.0, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}[dt]
+    assert_rel(as_f32(got[0], V.DT_BY_NAME[dt]), want, 2e-5 + ulp, 2.0 ** -24 if dt == "f16" else 1e-37, "softmax")
+    assert_rel(got[1], want, 2e-5, 1e-37, "softmax to f32")
 
 
 @pytest.mark.parametrize("in_dt", ["f32", "bf16"])
