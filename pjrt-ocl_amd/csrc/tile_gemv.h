@@ -429,6 +429,9 @@ VM_DEV void gemv_tile(Args A, uint32_t ti, uint32_t tile) {
 // release writes back).  Called only from the kernel and never as a tail call,
 // a leaf leaves the saving to the kernel, which keeps what it needs in
 // registers the leaf does not touch.
+// One row (a decode step) has a leaf of its own in every type: the eight-row one
+// accumulates, reduces and fetches (35 KB of code against 21) eight rows whatever M
+// is.  One step of six f32 layers of 512 on MI355X: 507 -> 366 us.
 template <uint32_t ADT, int MM>
 VM_LEAF void gemv_run(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   A = uargs(A);
@@ -446,9 +449,11 @@ VM_DEV void gemv_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
     if (M == 1) gemv_run<DT_BF16, 1>(A, ti, lo, hi);
     else gemv_run<DT_BF16, kGemvMaxM>(A, ti, lo, hi);
   } else if (adt == DT_F16) {
-    gemv_run<DT_F16, kGemvMaxM>(A, ti, lo, hi);
+    if (M == 1) gemv_run<DT_F16, 1>(A, ti, lo, hi);
+    else gemv_run<DT_F16, kGemvMaxM>(A, ti, lo, hi);
   } else {
-    gemv_run<DT_F32, kGemvMaxM>(A, ti, lo, hi);
+    if (M == 1) gemv_run<DT_F32, 1>(A, ti, lo, hi);
+    else gemv_run<DT_F32, kGemvMaxM>(A, ti, lo, hi);
   }
 }
 
