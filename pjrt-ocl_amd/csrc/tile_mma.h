@@ -458,52 +458,70 @@ VM_DEV f32x16 mfma16(const u16x8& a, const u16x8& b, const f32x16& c) {
                                                   0, 0);
 }
 
-// The descriptor arrives through a pointer; every field is wave-uniform.
-VM_DEV MmaDesc load_desc(const MmaDesc* p) {
+VM_DEV const VM_K MmaRec& rec_of(Args A, uint32_t ti) {
+  return *(const VM_K MmaRec*)(aux_of(A) + task_of(A, ti).p[0]);
+}
+
+// The task's tiles by index: split ts % S of output tile ts / S, of which the
+// first D.S splits do the work.  False: nothing to do for this index.
+struct MmaPos {
+  uint32_t id, g, m0, n0;               // id: the tile in the split scratch
+};
+VM_DEV uint32_t rec_quo(const VM_K MmaDiv& d, uint32_t x) {
+  const uint32_t t = uint32_t((uint64_t(d.m) * x) >> 32);
+  return (t + ((x - t) >> d.s1)) >> d.s2;
+}
+
+VM_DEV MmaDesc mma_desc(Args A, uint32_t ti) {
+  const VM_K Task& t = task_of(A, ti);
+  const VM_K MmaRec& r = rec_of(A, ti);
   MmaDesc D;
-  D.M = uni(p->M);
-  D.N = uni(p->N);
-  D.K = uni(p->K);
-  D.G = uni(p->G);
-  D.tm = uni(p->tm);
-  D.tn = uni(p->tn);
-  D.a = uni_ptr(p->a);
-  D.b = uni_ptr(p->b);
-  D.d = uni_ptr(p->d);
-  D.res = uni_ptr(p->res);
-  D.av = uni(p->av);
-  D.bv = uni(p->bv);
-  D.epi = uni(p->epi);
-  D.dt = uni(p->dt);
-  D.adt = uni(p->adt);
-  D.k0 = uni(p->k0);
-  D.k1 = uni(p->k1);
-  D.S = uni(p->S);
-  D.split = uni(p->split);
-  D.ti = uni(p->ti);
-  D.subs = uni(p->subs);
-  D.ldb = uni(p->ldb);
-  D.gsb = uint64_t(uni(uint32_t(p->gsb))) | uint64_t(uni(uint32_t(p->gsb >> 32))) << 32;
+  D.M = r.M;
+  D.N = r.N;
+  D.K = r.K;
+  D.G = r.G;
+  D.tm = r.tm;
+  D.tn = r.tn;
+  D.a = resolve(A, t.a);
+  D.b = resolve(A, t.b);
+  D.d = resolve(A, t.dst);
+  D.epi = r.epi;
+  D.res = r.epi ? resolve(A, t.p[7]) : D.a;
+  D.av = r.a.view;
+  D.bv = r.b.view;
+  D.dt = r.dt;
+  D.adt = r.adt;
+  D.S = r.S;
+  D.split = 0;
+  D.k0 = 0;
+  D.k1 = r.K;
+  D.ti = ti;
+  D.subs = r.subs;
+  D.ldb = r.b.ld;
+  D.gsb = uint64_t(r.b.gs_lo) | uint64_t(r.b.gs_hi) << 32;
   return D;
 }
 
-VM_DEV void tile_origin(const MmaDesc& D, uint32_t tile, uint32_t T, uint32_t* g, uint32_t* m0, uint32_t* n0) {
-  const uint32_t per = D.tm * D.tn;
-  *g = tile / per;
-  const uint32_t loc = tile % per;
-  *m0 = (loc / D.tn) * T;
-  *n0 = (loc % D.tn) * T;
+// Index ts, sub-tile q (0 unless a 256-wide tile is done as four 128-wide ones):
+// its place, and its K share in D.
+VM_DEV bool mma_pos(const VM_K MmaRec& r, MmaDesc& D, uint32_t ts, uint32_t q, MmaPos* p) {
+  const uint32_t tile = rec_quo(r.split, ts);
+  D.split = ts - tile * r.split.d;
+  if (D.split >= r.S) return false;
+  D.k0 = min(D.split * r.ksh, r.K);
+  D.k1 = min(D.k0 + r.ksh, r.K);
+  p->id = tile * r.subs + q;
+  p->g = rec_quo(r.per, tile);
+  const uint32_t loc = tile - p->g * r.per.d, tr = rec_quo(r.row, loc);
+  p->m0 = tr * r.T + (q >> 1) * 128;
+  p->n0 = (loc - tr * r.row.d) * r.T + (q & 1) * 128;
+  return p->m0 < r.M && p->n0 < r.N;
 }
 
 template <int T, bool BF16>
-VM_TILE void mma_tile16(Args A, const MmaDesc* Dp, uint32_t tile, uint32_t g, uint32_t m0, uint32_t n0) {
-  A = uargs(A);
-  const MmaDesc D = load_desc(Dp);
+VM_DEV void mma_tile16_one(Args A, const MmaDesc& D, uint32_t tile, uint32_t g, uint32_t m0, uint32_t n0) {
   uint16_t* lds = lds_ptr<uint16_t>();
   using C = MmaCfg<T>;
-  g = uni(g);
-  m0 = uni(m0);
-  n0 = uni(n0);
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wm = wave >> 1, wn = wave & 1;
   const OperandRead ar = operand_read(aux_of(A), D.av, D.a, D.K, uint64_t(D.G) * D.M * D.K, 8);
@@ -559,7 +577,21 @@ VM_TILE void mma_tile16(Args A, const MmaDesc* Dp, uint32_t tile, uint32_t g, ui
     if (ks + 1 < nk) st.store(lds + ((ks + 1) & 1) * Lds16<T>::kBuf);
     __syncthreads();
   }
-  mma_store<T>(A, D, acc, uni(tile), g, m0, n0);
+  mma_store<T>(A, D, acc, tile, g, m0, n0);
+}
+
+// A task's tiles [lo, hi) through the general tile: a leaf with its loop, as the
+// pipelined one.
+template <int T, bool BF16>
+VM_LEAF void mma_tile16(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  A = uargs(A);
+  MmaDesc D = mma_desc(A, uni(ti));
+  const VM_K MmaRec& r = rec_of(A, D.ti);
+  for (uint32_t ts = uni(lo); ts < uni(hi); ++ts)
+    for (uint32_t q = 0; q < r.subs; ++q) {
+      MmaPos p;
+      if (mma_pos(r, D, ts, q, &p)) mma_tile16_one<T, BF16>(A, D, p.id, p.g, p.m0, p.n0);
+    }
 }
 
 // ---------------------------------------------------------------------------------
@@ -857,16 +889,16 @@ VM_DEV void store_fast(Args A, const MmaDesc& D, const f32x16 (&acc)[4][4], uint
 // BT (ragged form only): B is k-contiguous (x . W^T: a tied embedding's logits),
 // its slab placed and read as A's is.
 template <bool BF16, bool RAG, bool BT>
-VM_LEAF void mma_tile16_fast(Args A, const MmaDesc* Dp, uint32_t tile) {
+VM_LEAF void mma_tile16_fast(Args A, uint32_t ti, uint32_t tile) {
   A = uargs(A);
-  const MmaDesc D = load_desc(Dp);
+  const MmaDesc D = mma_desc(A, uni(ti));
   const uint32_t lds0 = uni(uint32_t(reinterpret_cast<uintptr_t>(lds_ptr<lds_u8>())));
   const lds_u8* L = (const lds_u8*)uintptr_t(lds0);
   uint32_t g, m0, n0;
   fast_origin(D, uni(tile), &g, &m0, &n0);
   const uint32_t K = D.K, N = D.N;
   const gbyte* a = D.a + (uint64_t(g) * D.M + m0) * K * 2;        // A[g, m0, 0]
-  const gbyte* b = D.b + (BT ? D.gsb * g + uint64_t(n0) * D.ldb : uint64_t(g) * K * N + n0) * 2;   // B[g, 0, n0]
+  const gbyte* b = D.b + (BT ? D.gsb * g + uint64_t(n0) * D.ldb + rec_of(A, D.ti).b.off : uint64_t(g) * K * N + n0) * 2;   // B[g, 0, n0]
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wm = wave >> 1, wn = wave & 1;
   f32x16 acc[4][4];
@@ -1083,14 +1115,9 @@ struct Stage32 {
 };
 
 template <int T>
-VM_TILE void mma_tile32(Args A, const MmaDesc* Dp, uint32_t tile, uint32_t g, uint32_t m0, uint32_t n0) {
-  A = uargs(A);
-  const MmaDesc D = load_desc(Dp);
+VM_DEV void mma_tile32_one(Args A, const MmaDesc& D, uint32_t tile, uint32_t g, uint32_t m0, uint32_t n0) {
   float* lds = lds_ptr<float>();
   using C = MmaCfg<T>;
-  g = uni(g);
-  m0 = uni(m0);
-  n0 = uni(n0);
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wm = wave >> 1, wn = wave & 1;
   const bool vec = !D.av && !D.bv && (D.K % 4) == 0 && (D.N % 4) == 0 && ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0;
@@ -1128,7 +1155,19 @@ VM_TILE void mma_tile32(Args A, const MmaDesc* Dp, uint32_t tile, uint32_t g, ui
     if (ks + 1 < nk) st.store(lds + ((ks + 1) & 1) * Lds32<T>::kBuf);
     __syncthreads();
   }
-  mma_store<T>(A, D, acc, uni(tile), g, m0, n0);
+  mma_store<T>(A, D, acc, tile, g, m0, n0);
+}
+
+template <int T>
+VM_LEAF void mma_tile32(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  A = uargs(A);
+  MmaDesc D = mma_desc(A, uni(ti));
+  const VM_K MmaRec& r = rec_of(A, D.ti);
+  for (uint32_t ts = uni(lo); ts < uni(hi); ++ts)
+    for (uint32_t q = 0; q < r.subs; ++q) {
+      MmaPos p;
+      if (mma_pos(r, D, ts, q, &p)) mma_tile32_one<T>(A, D, p.id, p.g, p.m0, p.n0);
+    }
 }
 
 // ---- f32 fast path ---------------------------------------------------------------
@@ -1193,9 +1232,9 @@ struct F32Stage {
 };
 
 template <bool RAG>
-VM_LEAF void mma_tile32_fast(Args A, const MmaDesc* Dp, uint32_t tile) {
+VM_LEAF void mma_tile32_fast(Args A, uint32_t ti, uint32_t tile) {
   A = uargs(A);
-  const MmaDesc D = load_desc(Dp);
+  const MmaDesc D = mma_desc(A, uni(ti));
   float* lds = lds_ptr<float>();
   uint32_t g, m0, n0;
   fast_origin(D, uni(tile), &g, &m0, &n0);
@@ -1264,112 +1303,35 @@ constexpr int kMmaLdsBytes = kF32FastLdsBytes > kMmaLdsBytes1 ? kF32FastLdsBytes
 
 namespace vm {
 
+// An entry's tiles [lo, hi): the loader chose the tile kernel, for operand bases
+// that are 16-byte aligned and for others.
 VM_DEV void mma_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
-  A = uargs(A);
   const VM_K Task& t = task_of(A, ti);
-  MmaDesc D;
-  D.M = t.p[0];
-  D.N = t.p[1];
-  D.K = t.p[2];
-  D.G = max(1u, t.p[3] & 0xFFFFFFu);
-  const uint32_t code = (t.p[3] >> 24) & 0xF;
-  const uint32_t T = code == 1 ? 64u : code == 2 ? 128u : code == 3 ? 256u : A->mma_t;
-  D.tm = (D.M + T - 1) / T;
-  D.tn = (D.N + T - 1) / T;
-  D.a = resolve(A, t.a);
-  D.b = resolve(A, t.b);
-  D.d = resolve(A, t.dst);
-  // operand views the loader resolved to strides (kMmaStrided): the view itself follows the strides
-  D.av = t.p[4] & kMmaStrided ? uint32_t(aux_of(A)[(t.p[4] & ~kMmaStrided) + 4]) : t.p[4];
-  D.bv = t.p[5] & kMmaStrided ? uint32_t(aux_of(A)[(t.p[5] & ~kMmaStrided) + 4]) : t.p[5];
-  D.epi = t.p[6];
-  D.res = t.p[6] ? resolve(A, t.p[7]) : D.a;
-  D.dt = (t.tile_op >> 8) & 0xFF;
-  D.adt = (t.tile_op >> 16) & 0xFF;
-  D.S = 1u << ((t.p[3] >> 28) & 0xF);
-  D.ti = ti;
-  D.ldb = 0;
-  D.gsb = 0;
-  D.k0 = 0;
-  D.k1 = D.K;
-  D.split = 0;
-  hi = min(hi, D.tm * D.tn * D.G * D.S);
-  const bool h16 = D.adt == DT_BF16 || D.adt == DT_F16, bf = D.adt == DT_BF16;
-  const bool epi_ok = (D.dt == DT_F32 || D.dt == DT_BF16 || D.dt == DT_F16) && epi_inline_ok(A, D.epi);
-  // a K split's share: a multiple of 32 (16-bit) or 16 (f32) k
-  const uint32_t bk = h16 ? uint32_t(kBK16) : uint32_t(kBK32);
-  const uint32_t ksh = ((D.K + D.S - 1) / D.S + bk - 1) / bk * bk;
-  // 256-wide tiles: the big square GEMMs' fast paths.  Ragged shapes need 16-byte
-  // rows (K, N multiples of 8, f32: of 4) and offsets within 32 bits.
-  const bool plain = D.S == 1 && T == 256 && !D.av && !D.bv && D.N < (1u << 22) &&
-                     ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0 && epi_ok;
-  const bool fast = plain && h16 && D.M % 256 == 0 && D.N % 256 == 0 && D.K % kFBK == 0;
-  const bool fastr = plain && !fast && h16 && D.K >= 8 && D.K % 8 == 0 && D.N % 8 == 0 && D.K < (1u << 22);
-  const bool fast32 = plain && !h16 && D.M % 256 == 0 && D.N % 256 == 0 && D.K % kF32BK == 0;
-  const bool fast32r = plain && !fast32 && !h16 && D.K >= 4 && D.K % 4 == 0 && D.N % 4 == 0;
-  // A loop of its own for each fast tile: what is live across the call is little
-  // (the tile takes every register, so the kernel keeps its values in scratch).
-#define VM_FAST_TILES(COND, CALL)                                      \
-  if (COND) {                                                          \
-    for (uint32_t tile = lo; tile < hi; ++tile) CALL(A, &D, tile);     \
-    return;                                                            \
-  }
-  VM_FAST_TILES(fast && bf, (mma_tile16_fast<true, false, false>))
-  VM_FAST_TILES(fast, (mma_tile16_fast<false, false, false>))
-  VM_FAST_TILES(fastr && bf, (mma_tile16_fast<true, true, false>))
-  VM_FAST_TILES(fastr, (mma_tile16_fast<false, true, false>))
-  VM_FAST_TILES(fast32, mma_tile32_fast<false>)
-  VM_FAST_TILES(fast32r, mma_tile32_fast<true>)
-  MmaOp ops[2];
-  ops[0] = mma_op(aux_of(A), t.p[4], D.a, D.M, D.K, D.G, true, h16 ? 2 : 4);
-  ops[1] = mma_op(aux_of(A), t.p[5], D.b, D.N, D.K, D.G, false, h16 ? 2 : 4);
-  // The pipelined tiles where both operands are strided matrices (or A is read in
-  // whole chunks through its view, which only go global -> LDS directly, so B's
-  // have to as well), the general ones otherwise.
-  const bool pipe = epi_ok && ops[0].cls != MOP_NONE && ops[1].cls != MOP_NONE &&
-                    (ops[0].cls != MOP_RUNS || ops[1].cls == MOP_DMA);
-  // a k-contiguous B: the ragged 16-bit tile with B staged as A is
-  if (pipe && D.S == 1 && T == 256 && h16 && !D.av && ops[1].kc && ops[1].cls == MOP_DMA && D.K >= 8 && D.K % 8 == 0 &&
-      D.N % 8 == 0 && D.K < (1u << 22) && D.N < (1u << 22) && (uintptr_t(D.a) & 15) == 0) {
-    D.ldb = ops[1].ld;
-    D.gsb = ops[1].gs;
-    D.b = ops[1].p;
-    VM_FAST_TILES(bf, (mma_tile16_fast<true, true, true>))
-    VM_FAST_TILES(true, (mma_tile16_fast<false, true, true>))
-  }
-#undef VM_FAST_TILES
-  // a 256-wide tile outside the fast paths is done as four 128-wide ones
-  const uint32_t sub = T == 256 ? 2u : 1u, E = T / sub;
-  D.subs = sub * sub;
-  const uint32_t route = (pipe ? 0u : 6u) + (E == 128 ? 3u : 0u) + (!h16 ? 2u : bf ? 0u : 1u);
-  for (uint32_t ts = lo; ts < hi; ++ts) {
-    uint32_t tile = ts;
-    if (D.S > 1) {                      // split ts % S of output tile ts / S
-      tile = ts / D.S;
-      D.split = ts % D.S;
-      D.k0 = min(D.split * ksh, D.K);
-      D.k1 = min(D.k0 + ksh, D.K);
-    }
-    uint32_t g, m0, n0;
-    tile_origin(D, tile, T, &g, &m0, &n0);
-    for (uint32_t q = 0; q < sub * sub; ++q) {
-      const uint32_t m = m0 + q / sub * E, n = n0 + q % sub * E, id = tile * D.subs + q;
-      if (m >= D.M || n >= D.N) continue;
-      switch (route) {
-        case 0: mma_pipe_tile<64, ELT_BF16>(A, &D, ops, id, g, m, n); break;
-        case 1: mma_pipe_tile<64, ELT_F16>(A, &D, ops, id, g, m, n); break;
-        case 2: mma_pipe_tile<64, ELT_F32>(A, &D, ops, id, g, m, n); break;
-        case 3: mma_pipe_tile<128, ELT_BF16>(A, &D, ops, id, g, m, n); break;
-        case 4: mma_pipe_tile<128, ELT_F16>(A, &D, ops, id, g, m, n); break;
-        case 5: mma_pipe_tile<128, ELT_F32>(A, &D, ops, id, g, m, n); break;
-        case 6: mma_tile16<64, true>(A, &D, id, g, m, n); break;
-        case 7: mma_tile16<64, false>(A, &D, id, g, m, n); break;
-        case 8: mma_tile32<64>(A, &D, id, g, m, n); break;
-        case 9: mma_tile16<128, true>(A, &D, id, g, m, n); break;
-        case 10: mma_tile16<128, false>(A, &D, id, g, m, n); break;
-        default: mma_tile32<128>(A, &D, id, g, m, n); break;
-      }
-    }
+  const VM_K MmaRec& r = rec_of(A, ti);
+  hi = min(hi, r.tiles);
+  const bool aligned = ((uintptr_t(resolve(A, t.a)) | uintptr_t(resolve(A, t.b))) & 15) == 0;
+  switch (aligned ? r.route : r.route_u) {
+    case MR_PIPE: mma_pipe_tiles<64, ELT_BF16>(A, ti, lo, hi); break;
+    case MR_PIPE + 1: mma_pipe_tiles<64, ELT_F16>(A, ti, lo, hi); break;
+    case MR_PIPE + 2: mma_pipe_tiles<64, ELT_F32>(A, ti, lo, hi); break;
+    case MR_PIPE + 3: mma_pipe_tiles<128, ELT_BF16>(A, ti, lo, hi); break;
+    case MR_PIPE + 4: mma_pipe_tiles<128, ELT_F16>(A, ti, lo, hi); break;
+    case MR_PIPE + 5: mma_pipe_tiles<128, ELT_F32>(A, ti, lo, hi); break;
+    case MR_GENERAL: mma_tile16<64, true>(A, ti, lo, hi); break;
+    case MR_GENERAL + 1: mma_tile16<64, false>(A, ti, lo, hi); break;
+    case MR_GENERAL + 2: mma_tile32<64>(A, ti, lo, hi); break;
+    case MR_GENERAL + 3: mma_tile16<128, true>(A, ti, lo, hi); break;
+    case MR_GENERAL + 4: mma_tile16<128, false>(A, ti, lo, hi); break;
+    case MR_GENERAL + 5: mma_tile32<128>(A, ti, lo, hi); break;
+    // the fast tiles fill the registers: one call each, the loop in the kernel
+    case MR_FAST16: for (; lo < hi; ++lo) mma_tile16_fast<true, false, false>(A, ti, lo); break;
+    case MR_FAST16 + 1: for (; lo < hi; ++lo) mma_tile16_fast<false, false, false>(A, ti, lo); break;
+    case MR_RAGGED16: for (; lo < hi; ++lo) mma_tile16_fast<true, true, false>(A, ti, lo); break;
+    case MR_RAGGED16 + 1: for (; lo < hi; ++lo) mma_tile16_fast<false, true, false>(A, ti, lo); break;
+    case MR_BT16: for (; lo < hi; ++lo) mma_tile16_fast<true, true, true>(A, ti, lo); break;
+    case MR_BT16 + 1: for (; lo < hi; ++lo) mma_tile16_fast<false, true, true>(A, ti, lo); break;
+    case MR_FAST32: for (; lo < hi; ++lo) mma_tile32_fast<false>(A, ti, lo); break;
+    default: for (; lo < hi; ++lo) mma_tile32_fast<true>(A, ti, lo); break;
   }
 }
 

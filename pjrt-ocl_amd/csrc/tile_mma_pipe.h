@@ -33,9 +33,7 @@
 
 namespace vm {
 
-// An operand as the pipelined tiles read it: element (g, r, k) at
-// p + (g gs + (kc ? r ld + k : k ld + r)) esz, r a row of A or a column of B.
-enum : uint32_t { MOP_DMA = 0, MOP_RUNS = 1, MOP_REG = 2, MOP_NONE = 3 };
+// An operand as the pipelined tiles read it (vm_abi.h MmaOperand, its base resolved).
 struct MmaOp {
   const gbyte* p;
   uint64_t gs;
@@ -43,46 +41,16 @@ struct MmaOp {
   uint32_t kc, cls;
   uint32_t view;          // MOP_RUNS: the view (aux offset + 1) its chunks are read through
 };
-
-// A view operand word with this bit set is an index into the aux pool of a
-// strided operand the loader resolved: {kc, ld, gs, offset, view} (vmrt.cpp
-// `resolve_mma_view`); without it, a view descriptor (aux offset + 1) or 0.
-VM_DEV MmaOp mma_op(const VM_K int32_t* aux, uint32_t view, const gbyte* base, uint32_t R, uint32_t K, uint32_t G,
-                    bool is_a, uint32_t esz) {
-  const uint32_t per = 16 / esz;
-  MmaOp o;
-  o.p = base;
-  o.R = R;
-  o.view = 0;
-  o.cls = MOP_NONE;
-  o.kc = is_a;
-  o.ld = is_a ? K : R;
-  o.gs = uint64_t(R) * K;
-  if (view & kMmaStrided) {
-    const VM_K int32_t* x = aux + (view & ~kMmaStrided);
-    o.kc = uint32_t(x[0]);
-    o.ld = uint32_t(x[1]);
-    o.gs = uint32_t(x[2]);
-    o.p = base + uint64_t(uint32_t(x[3])) * esz;          // x[4]: the view itself
-  } else if (view) {
-    // chunk runs of a view (A only): see operand_read
-    if (!is_a) return o;
-    const OperandRead r = operand_read(aux, view, base, K, uint64_t(G) * R * K, per);
-    int64_t last = r.map.off;                             // the view's largest element index
-#pragma unroll
-    for (int k = 0; k < kViewRank; ++k)
-      if (k < r.map.rank && r.map.stride[k] > 0) last += int64_t(r.map.dim[k].d - 1) * r.map.stride[k];
-    if (r.mode == 1 && K >= per && uint64_t(last) * esz <= 0xFFFFFFFFull) {
-      o.cls = MOP_RUNS;
-      o.view = view;
-    }
-    return o;
-  }
-  // the longest row offset of a tile stays within 32 bits
-  if (o.ld >= (1u << 22) || (o.kc ? K : R) < per) return o;
-  const bool whole = (uintptr_t(o.p) & 15) == 0 && o.ld % per == 0 && o.gs % per == 0 && (o.kc ? K : R) % per == 0;
-  o.cls = whole ? MOP_DMA : MOP_REG;
-  return o;
+VM_DEV MmaOp mma_op(const VM_K MmaOperand& o, const gbyte* base, uint32_t R, uint32_t esz) {
+  MmaOp x;
+  x.p = base + uint64_t(o.off) * esz;
+  x.gs = uint64_t(o.gs_lo) | uint64_t(o.gs_hi) << 32;
+  x.ld = o.ld;
+  x.R = R;
+  x.kc = o.kc;
+  x.cls = o.cls;
+  x.view = o.view;
+  return x;
 }
 
 enum { ELT_BF16 = 0, ELT_F16 = 1, ELT_F32 = 2 };
@@ -544,28 +512,9 @@ VM_DEV void store_pipe(Args A, const MmaDesc& D, const f32x16 (&acc)[T / 64][T /
   }
 }
 
-// One T x T tile (or a K split's share of it).  The operands' classes and layouts
-// are the task's, so every tile of a task takes the same route.
+// One T x T tile (or a K split's share of it).
 template <int T, int ELT>
-VM_LEAF void mma_pipe_tile(Args A, const MmaDesc* Dp, const MmaOp* ops, uint32_t tile, uint32_t g, uint32_t m0,
-                           uint32_t n0) {
-  A = uargs(A);
-  const MmaDesc D = load_desc(Dp);
-  auto load_op = [](const MmaOp* p) {
-    MmaOp o;
-    o.p = uni_ptr(p->p);
-    o.gs = uint64_t(uni(uint32_t(p->gs))) | uint64_t(uni(uint32_t(p->gs >> 32))) << 32;
-    o.ld = uni(p->ld);
-    o.R = uni(p->R);
-    o.kc = uni(p->kc);
-    o.cls = uni(p->cls);
-    o.view = uni(p->view);
-    return o;
-  };
-  const MmaOp oa = load_op(ops), ob = load_op(ops + 1);
-  g = uni(g);
-  m0 = uni(m0);
-  n0 = uni(n0);
+VM_DEV void mma_pipe_one(Args A, const MmaDesc& D, const MmaOp& oa, const MmaOp& ob, bool dma, const MmaPos& at) {
   using P = Pipe<T, ELT>;
   const uint32_t lds0 = uni(uint32_t(reinterpret_cast<uintptr_t>(lds_ptr<lds_u8>())));
   f32x16 acc[P::kB][P::kB];
@@ -574,15 +523,14 @@ VM_LEAF void mma_pipe_tile(Args A, const MmaDesc* Dp, const MmaOp* ops, uint32_t
 #pragma unroll
     for (int j = 0; j < P::kB; ++j) acc[i][j] = f32x16{};
   if (D.k1 > D.k0) {
-    const bool dma = oa.cls <= MOP_RUNS && ob.cls == MOP_DMA;
 #define VM_PIPE(KA, KB)                                                                                              \
   {                                                                                                                  \
     if (dma && oa.cls == MOP_RUNS) {                                                                                 \
-      if constexpr (KA) pipe_loop_dma<T, ELT, KA, KB, true>(A, oa, ob, g, m0, n0, D.K, D.k0, D.k1, lds0, acc);       \
+      if constexpr (KA) pipe_loop_dma<T, ELT, KA, KB, true>(A, oa, ob, at.g, at.m0, at.n0, D.K, D.k0, D.k1, lds0, acc); \
     } else if (dma) {                                                                                                \
-      pipe_loop_dma<T, ELT, KA, KB, false>(A, oa, ob, g, m0, n0, D.K, D.k0, D.k1, lds0, acc);                        \
+      pipe_loop_dma<T, ELT, KA, KB, false>(A, oa, ob, at.g, at.m0, at.n0, D.K, D.k0, D.k1, lds0, acc);               \
     } else {                                                                                                         \
-      pipe_loop_reg<T, ELT, KA, KB>(A, oa, ob, g, m0, n0, D.K, D.k0, D.k1, lds0, acc);                               \
+      pipe_loop_reg<T, ELT, KA, KB>(A, oa, ob, at.g, at.m0, at.n0, D.K, D.k0, D.k1, lds0, acc);                      \
     }                                                                                                                \
   }
     if (oa.kc) {
@@ -592,8 +540,25 @@ VM_LEAF void mma_pipe_tile(Args A, const MmaDesc* Dp, const MmaOp* ops, uint32_t
     }
 #undef VM_PIPE
   }
-  if (D.S > 1 && !mma_split_combine<T>(A, D, acc, uni(tile))) return;
-  store_pipe<T>(A, D, acc, g, m0, n0);
+  if (D.S > 1 && !mma_split_combine<T>(A, D, acc, at.id)) return;
+  store_pipe<T>(A, D, acc, at.g, at.m0, at.n0);
+}
+
+// A task's tiles [lo, hi): one leaf with the loop and the tile inlined.  The
+// classes and layouts of the operands are the task's, so every tile of it takes the
+// same route.
+template <int T, int ELT>
+VM_LEAF void mma_pipe_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  A = uargs(A);
+  MmaDesc D = mma_desc(A, uni(ti));
+  const VM_K MmaRec& r = rec_of(A, D.ti);
+  const MmaOp oa = mma_op(r.a, D.a, r.M, Pipe<T, ELT>::kEsz), ob = mma_op(r.b, D.b, r.N, Pipe<T, ELT>::kEsz);
+  const bool dma = oa.cls <= MOP_RUNS && ob.cls == MOP_DMA && ((uintptr_t(D.a) | uintptr_t(D.b)) & 15) == 0;
+  for (uint32_t ts = uni(lo); ts < uni(hi); ++ts)
+    for (uint32_t q = 0; q < r.subs; ++q) {
+      MmaPos p;
+      if (mma_pos(r, D, ts, q, &p)) mma_pipe_one<T, ELT>(A, D, oa, ob, dma, p);
+    }
 }
 
 }  // namespace vm

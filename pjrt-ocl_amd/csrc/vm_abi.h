@@ -70,9 +70,35 @@ constexpr uint32_t kRedMaxSplits = 64;
 constexpr uint32_t kGemvMaxM = 8;
 // TOP_MMA: log2 of the K split (task p3 bits 28-31) at most.
 constexpr uint32_t kMmaMaxSplitLog2 = 5;
-// TOP_MMA p4 / p5 on the device: an operand view the loader resolved to strides
-// (vmrt.cpp `resolve_mma_view`), as this bit | the index of its five aux words.
-constexpr uint32_t kMmaStrided = 0x80000000u;
+// A TOP_MMA task as the kernel reads it, worked out by the loader (vmrt.cpp
+// `mma_record`) and kept in the device's aux pool at word p0: sizes, tile counts
+// and their invariant divisors, operand strides and the tile kernel to run, so that
+// an entry reaches its first load after two scalar reads, with no division and no
+// descriptor passed through scratch memory.
+struct MmaOperand {    // element (g, r, k) at off + g gs + (kc ? r ld + k : k ld + r), r a row of A or a column of B
+  uint32_t kc, ld, gs_lo, gs_hi, off;
+  uint32_t cls;        // MmaClass where both bases are 16-byte aligned
+  uint32_t view;       // the view (aux offset + 1; 0: none)
+  uint32_t pad;
+};
+enum MmaClass : uint32_t { MOP_DMA = 0, MOP_RUNS = 1, MOP_REG = 2, MOP_NONE = 3 };
+struct MmaDiv { uint32_t d, m, s1, s2; };   // DivU32 (vm_divu32.h)
+struct MmaRec {
+  uint32_t M, N, K, tiles;             // tiles: of the whole task
+  uint32_t tm, tn, G, S;               // S: the K split that does the work, at most the task's
+  uint32_t ksh, dt, adt, epi;          // ksh: k of a split
+  uint32_t route, route_u, T, subs;    // MmaRoute where both bases are 16-byte aligned, and else; subs: see MmaDesc
+  MmaOperand a, b;
+  MmaDiv split, per, row;              // by the task's split, tm tn, tn
+  uint32_t pad[4];
+};
+static_assert(sizeof(MmaRec) == 192, "MmaRec layout");
+// Tile kernels.  0-11: + 0 bf16, 1 f16, 2 f32, + 3 for 128-wide tiles.
+enum MmaRoute : uint32_t {
+  MR_PIPE = 0, MR_GENERAL = 6,
+  MR_FAST16 = 12, MR_RAGGED16 = 14, MR_BT16 = 16,   // 256-wide, + 1 f16
+  MR_FAST32 = 18, MR_RAGGED32 = 19
+};
 constexpr int kMaxPorts = 256;          // power of two: handles mask the port index
 
 // Per-program control buffer: status words, then one arrival word per lane.

@@ -71,6 +71,10 @@ VM_DEV void warm_entry(Args A, const VM_K Entry* ents, uint32_t i, uint32_t end)
   const VM_K Task& t = task_of(A, e.task);
   const uint32_t top = t.tile_op, p5 = t.p[5], p6 = t.p[6];
   asm volatile("" ::"s"(t.dst), "s"(t.a), "s"(t.b), "s"(t.p[0]), "s"(t.p[4]), "s"(t.p[7]));
+  if ((top & 0xFF) == TOP_MMA) {
+    const VM_K MmaRec& r = rec_of(A, e.task);
+    asm volatile("" ::"s"(r.M), "s"(r.a.ld), "s"(r.split.d));
+  }
   if ((top & 0xFF) != TOP_GEMV) return;
   if (p5) {
     const VM_K Task& L = task_of(A, p5 - 1);

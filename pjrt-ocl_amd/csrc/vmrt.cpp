@@ -26,6 +26,9 @@
 #include "../../include/vmrt.h"
 #include "launch_slots.h"
 #include "vm_abi.h"
+#define VM_HD inline
+#include "vm_divu32.h"
+#undef VM_HD
 
 extern "C" int vm_kernel_smem_bytes();
 extern "C" hipError_t vm_kernel_prepare();
@@ -924,15 +927,15 @@ static std::vector<LaneSpan> device_lanes(const std::vector<LaneSpan>& lanes, co
   return out;
 }
 
+// ---- matmul records (vm_abi.h MmaRec) ----------------------------------------------------
 // A matmul operand's view as one stride per matrix dimension, when it has them:
 // logical [G, outer, inner] (A: G, M, K; B: G, K, N) with a constant stride along
 // each -- a transpose, a head's columns of a wider row, a slice -- and one of the two
-// matrix strides 1.  Appended to the device aux pool as {k-contiguous, row stride,
-// batch stride, offset, view}, so that a tile reads its operand by strides and
-// never walks the view.  Views that split a dimension over several strides, or
-// whose numbers leave 31 bits, stay views.  The loader has checked the view.
+// matrix strides 1, so that a tile reads its operand by strides and never walks
+// the view.  Views that split a dimension over several strides, or whose numbers
+// leave 31 bits, stay views.  The loader has checked the view.
 static bool resolve_mma_view(const Program& P, uint32_t view, uint64_t G, uint64_t outer, uint64_t inner, bool is_a,
-                             std::vector<int32_t>* aux, uint32_t* word) {
+                             MmaOperand* o) {
   const int32_t* x = P.aux.data() + (view - 1);
   const int rank = x[0];
   const int64_t off = x[1 + 2 * rank];
@@ -969,9 +972,119 @@ static bool resolve_mma_view(const Program& P, uint32_t view, uint64_t G, uint64
   const int64_t ld = kc ? sr : sk;
   for (int64_t v : {ld, sg, off})
     if (v < 0 || v > INT32_MAX) return false;
-  *word = kMmaStrided | uint32_t(aux->size());
-  for (int64_t v : {int64_t(kc), ld, sg, off, int64_t(view)}) aux->push_back(int32_t(v));
+  o->kc = kc;
+  o->ld = uint32_t(ld);
+  o->gs_lo = uint32_t(sg);
+  o->gs_hi = 0;
+  o->off = uint32_t(off);
   return true;
+}
+
+// Whether A's view is read in whole aligned 16-byte chunks of `per` elements: at
+// most four dims, the innermost contiguous, it, the other strides and the offset
+// multiples of `per`, and every byte offset within 32 bits (a decoder's attention
+// output read as [tokens, heads * head_dim]).
+static bool mma_view_runs(const Program& P, uint32_t view, uint64_t n, uint32_t K, uint32_t per, uint32_t esz) {
+  const int32_t* x = P.aux.data() + (view - 1);
+  const int rank = x[0];
+  if (rank < 1 || rank > 4 || K % per || n > 0xFFFFFFFFull) return false;
+  int64_t last = x[1 + 2 * rank];
+  if (x[rank] % int32_t(per) || x[2 * rank] != 1 || last % int64_t(per)) return false;
+  for (int k = 0; k < rank; ++k) {
+    const int64_t st = x[1 + rank + k];
+    if (k < rank - 1 && st % int64_t(per)) return false;
+    if (st > 0) last += int64_t(x[1 + k] - 1) * st;
+  }
+  return uint64_t(last) * esz <= 0xFFFFFFFFull;
+}
+
+static MmaDiv mma_div(uint32_t d) {
+  const DivU32 x = div_u32(std::max(1u, d));
+  return MmaDiv{x.d, x.m, x.s1, x.s2};
+}
+
+// The kernel's micro-op kinds that a store evaluates inline (tile_mma.h epi_inline4), up to four of them.
+static bool mma_epi_inline(const Program& P, uint32_t epi) {
+  if (!epi) return true;
+  const int32_t* e = P.aux.data() + (epi - 1);
+  if (e[0] > 4) return false;
+  for (int k = 0; k < e[0]; ++k) {
+    const uint32_t kind = uint32_t(e[1 + 4 * k]);
+    if (!(kind == SUB_AFFINE || kind == SUB_GELU || kind == SUB_COPY || kind <= SUB_DIV || kind == SUB_MAX || kind == SUB_MIN))
+      return false;
+  }
+  return true;
+}
+
+static MmaRec mma_record(const Program& P, const Task& t, uint32_t mma_t) {
+  MmaRec r{};
+  r.M = t.p[0];
+  r.N = t.p[1];
+  r.K = t.p[2];
+  r.G = std::max<uint32_t>(1, t.p[3] & 0xFFFFFF);
+  const uint32_t code = (t.p[3] >> 24) & 0xF, S = 1u << (t.p[3] >> 28);
+  r.T = code == 1 ? 64 : code == 2 ? 128 : code == 3 ? 256 : mma_t;
+  r.tm = (r.M + r.T - 1) / r.T;
+  r.tn = (r.N + r.T - 1) / r.T;
+  r.tiles = r.tm * r.tn * r.G * S;
+  r.dt = (t.tile_op >> 8) & 0xFF;
+  r.adt = (t.tile_op >> 16) & 0xFF;
+  r.epi = t.p[6];
+  const bool h16 = r.adt == DT_BF16 || r.adt == DT_F16;
+  const uint32_t f16 = r.adt == DT_F16, per = h16 ? 8 : 4, esz = h16 ? 2 : 4;
+  const bool epi_ok = (r.dt == DT_F32 || r.dt == DT_BF16 || r.dt == DT_F16) && mma_epi_inline(P, t.p[6]);
+  auto operand = [&](MmaOperand* o, uint32_t view, bool is_a) {
+    const uint32_t R = is_a ? r.M : r.N;
+    const uint64_t gs = uint64_t(R) * r.K;
+    o->kc = is_a;
+    o->ld = is_a ? r.K : R;
+    o->gs_lo = uint32_t(gs);
+    o->gs_hi = uint32_t(gs >> 32);
+    o->view = view;
+    o->cls = MOP_NONE;
+    if (!R || !r.K) return;
+    if (view && !resolve_mma_view(P, view, r.G, is_a ? r.M : r.K, is_a ? r.K : r.N, is_a, o)) {
+      if (is_a && mma_view_runs(P, view, gs * r.G, r.K, per, esz)) o->cls = MOP_RUNS;
+      return;
+    }
+    // the longest row offset of a tile stays within 32 bits
+    if (o->ld >= (1u << 22) || (o->kc ? r.K : R) < per) return;
+    const bool whole = o->ld % per == 0 && o->gs_lo % per == 0 && o->off % per == 0 && (o->kc ? r.K : R) % per == 0;
+    o->cls = whole ? MOP_DMA : MOP_REG;
+  };
+  operand(&r.a, t.p[4], true);
+  operand(&r.b, t.p[5], false);
+  // The split that does the work: the others' share of the K loop (0.022 us per f32 k of
+  // a 64-wide tile, 0.007 in 16 bits, three times that 128-wide) has to be worth
+  // publishing the partials and combining them, about 8 us (measured: 1.5 us to
+  // publish, 2 for the arrival, 4.4 to read the partials).
+  const double per_k = (h16 ? 0.007 : 0.022) * (r.T == 128 ? 3 : 1);
+  r.S = S > 1 && r.K * (1.0 - 1.0 / S) * per_k < 8.0 ? 1 : S;
+  const uint32_t bk = h16 ? 32 : 16;
+  r.ksh = ((r.K + r.S - 1) / r.S + bk - 1) / bk * bk;
+  r.subs = 1;
+  r.split = mma_div(S);
+  r.per = mma_div(r.tm * r.tn);
+  r.row = mma_div(r.tn);
+  // 256-wide: the big GEMMs' fast tiles, whole or with ragged edges (16-byte rows,
+  // offsets within 32 bits), and the 16-bit one with a k-contiguous B
+  const uint32_t wide = r.T == 256 ? 3 : r.T == 128 ? 3 : 0, elt = h16 ? f16 : 2;
+  const bool plain = S == 1 && r.T == 256 && !t.p[4] && r.N < (1u << 22) && r.K < (1u << 22) && r.K >= per &&
+                     r.K % per == 0 && r.N % per == 0 && epi_ok;
+  r.route_u = MR_GENERAL + wide + elt;
+  if (epi_ok && r.a.cls != MOP_NONE && r.a.cls != MOP_RUNS && r.b.cls != MOP_NONE) r.route_u = MR_PIPE + wide + elt;
+  if (plain && !t.p[5]) {
+    const bool even = r.M % 256 == 0 && r.N % 256 == 0 && r.K % (h16 ? 64 : 16) == 0;
+    r.route = h16 ? (even ? MR_FAST16 : MR_RAGGED16) + f16 : even ? MR_FAST32 : MR_RAGGED32;
+  } else if (plain && h16 && r.b.kc && r.b.cls == MOP_DMA) {
+    r.route = MR_BT16 + f16;
+  } else {
+    r.route = r.route_u;
+    if (epi_ok && r.a.cls == MOP_RUNS && r.b.cls == MOP_DMA) r.route = MR_PIPE + wide + elt;
+  }
+  // any other 256-wide tile is done as four 128-wide ones
+  if (r.T == 256) r.subs = 4;
+  return r;
 }
 
 // Host half of a load: parse, validate, choose ports, patch buffer ids to handles
@@ -1094,13 +1207,14 @@ static int prepare_program(vmrt_runtime* rt, vmrt_program* lp, const void* bytes
       for (int d = 0; d < rank; ++d) aux[x + 1 + 3 * rank + d] = int32_t(handle(uint32_t(P.aux[x + 1 + 4 * rank + d])));
     }
   }
-  // ---- matmul operand views with one stride per matrix dimension ----
-  for (Task& t : tasks) {
-    if ((t.tile_op & 0xFF) != TOP_MMA) continue;
-    const uint64_t M = t.p[0], N = t.p[1], K = t.p[2], G = std::max<uint32_t>(1, t.p[3] & 0xFFFFFF);
-    if (!M || !N || !K) continue;
-    if (t.p[4]) resolve_mma_view(P, t.p[4], G, M, K, true, &aux, &t.p[4]);
-    if (t.p[5]) resolve_mma_view(P, t.p[5], G, K, N, false, &aux, &t.p[5]);
+  // ---- matmul records, one cache line and more each ----
+  for (size_t i = 0; i < tasks.size(); ++i) {
+    if ((tasks[i].tile_op & 0xFF) != TOP_MMA) continue;
+    const MmaRec rec = mma_record(P, P.tasks[i], lp->mma_t);
+    aux.resize((aux.size() + 15) / 16 * 16);
+    tasks[i].p[0] = uint32_t(aux.size());
+    const int32_t* w = reinterpret_cast<const int32_t*>(&rec);
+    aux.insert(aux.end(), w, w + sizeof rec / 4);
   }
   // ---- patch control entries: cond buffer -> handle, pad -> cond format ----
   std::vector<Entry>& entries = pr->entries;
@@ -1127,7 +1241,7 @@ static int prepare_program(vmrt_runtime* rt, vmrt_program* lp, const void* bytes
   std::vector<uint32_t>& task_scratch = pr->task_scratch;
   task_scratch.assign(tasks.size(), 0);
   for (size_t i = 0; i < tasks.size(); ++i) {
-    const uint64_t nb = task_scratch_bytes(tasks[i], lp->mma_t);
+    const uint64_t nb = task_scratch_bytes(P.tasks[i], lp->mma_t);   // the program's own fields: a matmul's p0 is patched
     if (!nb) continue;
     task_scratch[i] = uint32_t(lp->scratch_bytes);
     lp->scratch_bytes += (nb + 255) & ~uint64_t(255);

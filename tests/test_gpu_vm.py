@@ -688,13 +688,14 @@ def test_dot_split_k_exact(dt, Gb, M, K, N):
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("Gb,M,K,N,tile", [(1, 200, 520, 136, 64), (1, 264, 72, 392, 128), (2, 129, 200, 72, 64),
                                            (1, 61, 131, 77, 64), (1, 259, 333, 131, 128), (3, 70, 9, 67, 64),
-                                           (1, 300, 261, 515, 256), (1, 64, 1100, 64, 0), (1, 8, 8, 9, 64)])
+                                           (1, 300, 261, 515, 256), (1, 64, 1100, 64, 0), (1, 70, 3001, 64, 0),
+                                           (1, 8, 8, 9, 64)])
 def test_dot_operand_layouts_exact(dt, ta, tb, Gb, M, K, N, tile):
     """The 64- and 128-wide tiles with each operand k-contiguous or
     row-contiguous (a transposed view), in whole 16-byte chunks (sizes multiples
     of 8: stages go global -> LDS directly; K one, several and a partial stage)
     and in odd sizes (through registers, chunks cut at the operands' ends), a
-    batch, a K split (tile 0: the scheduler's choice), and a 256-wide tile done
+    batch, a K split (tile 0: the scheduler's choice; 3001 is worth one in every type), and a 256-wide tile done
     as four.  Integer-valued operands give the exact result, whose bias and
     residual epilogue reads ragged rows."""
     rng = np.random.default_rng(79)
