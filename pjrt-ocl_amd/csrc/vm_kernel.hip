@@ -26,6 +26,7 @@ namespace vm {
 
 constexpr int kMaxDepth = 8;
 constexpr uint32_t kRootOwner = 0xFFFFFFFFu;
+__shared__ uint32_t vm_frames[kWaves][kMaxDepth][4];
 
 // LDS shared by the tile ops of one lane (the matmul's double-buffered operand
 // slabs are the largest user).
@@ -116,64 +117,67 @@ __global__ __launch_bounds__(kBlock, 1) void vm_main(VmArgs args) {
                  "s"(t0.p[7]));
   }
 
-  uint32_t f_pc[kMaxDepth], f_end[kMaxDepth], f_own[kMaxDepth], f_phase[kMaxDepth];
-  int sp = 0;
-  f_pc[0] = 0;
-  f_end[0] = span.root_len;
-  f_own[0] = kRootOwner;
-  f_phase[0] = 0;
+  // The current frame's place in registers, the frames below it in LDS, a copy per
+  // wave (waves of a lane may be a control entry apart): as arrays in registers the
+  // eight frames were 32 scalars to save around every tile call.
+  uint32_t (*fr)[4] = vm_frames[uni(threadIdx.x >> 6)];   // {pc, end, own, phase}
+  uint32_t sp = 0, pc = 0, end = span.root_len, own = kRootOwner;
   bool pub = false;     // a tile entry ran since the last barrier
   uint32_t nbar = 0;    // grid barriers this lane has passed in this launch (completion flag values)
+  auto pop = [&] {
+    --sp;
+    pc = uni(fr[sp][0]) + 1;
+    end = uni(fr[sp][1]);
+    own = uni(fr[sp][2]);
+  };
 
   for (;;) {
-    if (f_pc[sp] >= f_end[sp]) {
-      if (f_own[sp] == kRootOwner) break;
-      const Entry w = load_entry(ents + f_own[sp]);
+    if (pc >= end) {
+      if (own == kRootOwner) break;
+      const Entry w = load_entry(ents + own);
       if (w.task == ENT_IF) {                 // branch done
-        --sp;
-        ++f_pc[sp];
+        pop();
         continue;
       }
       // loop bodies end with a grid barrier that publishes the carries
       // (warming a FOR body's first entry when another trip follows)
-      const bool again = w.task == ENT_FOR && f_phase[sp] > 1;
+      const uint32_t phase = uni(fr[sp][3]);
+      const bool again = w.task == ENT_FOR && phase > 1;
       if (!timed_barrier(A, ents, again ? w.tile_lo : 0u, again ? w.tile_lo + w.tile_hi : 0u)) return;
       ++nbar;
       pub = false;
       if (w.task == ENT_FOR) {
-        if (--f_phase[sp] != 0) {
-          f_pc[sp] = w.tile_lo;
-          f_end[sp] = w.tile_lo + w.tile_hi;
+        if (phase > 1) {
+          fr[sp][3] = phase - 1;
+          pc = w.tile_lo;
+          end = w.tile_lo + w.tile_hi;
         } else {
-          --sp;
-          ++f_pc[sp];
+          pop();
         }
         continue;
       }
-      if (f_phase[sp] == 0) {                 // while-cond done: test
+      if (phase == 0) {                       // while-cond done: test
         if (read_cond(resolve(A, w.signal_flag), w.pad)) {
-          f_pc[sp] = w.wait_flag;
-          f_end[sp] = w.wait_flag + w.wait_count;
-          f_phase[sp] = 1;
+          pc = w.wait_flag;
+          end = w.wait_flag + w.wait_count;
+          fr[sp][3] = 1;
         } else {
-          --sp;
-          ++f_pc[sp];
+          pop();
         }
       } else {                                // while-body done: re-test
-        f_pc[sp] = w.tile_lo;
-        f_end[sp] = w.tile_lo + w.tile_hi;
-        f_phase[sp] = 0;
+        pc = w.tile_lo;
+        end = w.tile_lo + w.tile_hi;
+        fr[sp][3] = 0;
       }
       continue;
     }
 
-    const uint32_t epc = f_pc[sp];
-    const Entry en = load_entry(ents + epc);
+    const Entry en = load_entry(ents + pc);
     if (en.task == ENT_BARRIER) {
-      if (!timed_barrier(A, ents, epc + 1, f_end[sp])) return;
+      if (!timed_barrier(A, ents, pc + 1, end)) return;
       ++nbar;
       pub = false;
-      ++f_pc[sp];
+      ++pc;
       continue;
     }
     if (en.task == ENT_WHILE || en.task == ENT_FOR || en.task == ENT_IF) {
@@ -184,7 +188,7 @@ __global__ __launch_bounds__(kBlock, 1) void vm_main(VmArgs args) {
         phase = 0;
       } else if (en.task == ENT_FOR) {
         if (en.wait_flag == 0) {
-          ++f_pc[sp];
+          ++pc;
           continue;
         }
         start = en.tile_lo;
@@ -196,19 +200,22 @@ __global__ __launch_bounds__(kBlock, 1) void vm_main(VmArgs args) {
         len = c ? en.tile_hi : en.wait_count;
         phase = 2;
         if (len == 0) {
-          ++f_pc[sp];
+          ++pc;
           continue;
         }
       }
-      if (sp + 1 >= kMaxDepth) {
+      if (sp + 1 >= uint32_t(kMaxDepth)) {
         raise_error(A, VM_ERR_FRAME_DEPTH, lane);
         return;
       }
+      fr[sp][0] = pc;
+      fr[sp][1] = end;
+      fr[sp][2] = own;
       ++sp;
-      f_pc[sp] = start;
-      f_end[sp] = start + len;
-      f_own[sp] = epc;
-      f_phase[sp] = phase;
+      fr[sp][3] = phase;
+      own = pc;
+      pc = start;
+      end = start + len;
       continue;
     }
     if (en.task != ENT_NOP) {
@@ -239,7 +246,7 @@ __global__ __launch_bounds__(kBlock, 1) void vm_main(VmArgs args) {
       }
       if (en.signal_flag != FLAG_NONE) flag_signal(A, en.signal_flag, phase_tag(A, nbar));
     }
-    ++f_pc[sp];
+    ++pc;
   }
   if (A->stats && threadIdx.x == 0)
     __hip_atomic_fetch_add(A->stats + 2, __builtin_amdgcn_s_memrealtime() - t_launch, __ATOMIC_RELAXED,
