@@ -320,6 +320,47 @@ def fuse_matmul_views(prog: V.VMProgram) -> None:
             break
 
 
+def fold_dot_transposes(prog: V.VMProgram) -> None:
+    """A matmul whose only reader transposes it, (A B)^T, becomes B^T A^T written in
+    the transposed layout: JAX's rule for a weight's gradient is dot_general(g, x)
+    and a transpose.  The operands swap and each reads through its transposed view
+    (none where that is the plain matrix); every output is the same products summed
+    in the same order.  Matmuls with an epilogue, a batch or wider views stay."""
+    if _off("PJRT_AMD_DOT_TRANSPOSE"):
+        return
+
+    def transposed(view1, rows, cols):
+        dims, st, off = _view_desc(prog, view1) if view1 else ([rows, cols], [cols, 1], 0)
+        if len(dims) != 2 or dims != [rows, cols]:
+            return None
+        if off == 0 and st == [1, rows]:
+            return 0
+        prog.aux.extend([2, cols, rows, st[1], st[0], off])
+        return len(prog.aux) - 6 + 1
+
+    sc = scopes(prog)
+    ix = _Index(prog)
+    outs = set(prog.outputs)
+    for gi, g in enumerate(prog.instrs):
+        if g.op != V.OP_GATHER_STRIDED or len(ix.writers.get(g.dst, ())) != 1 or g.a in outs:
+            continue
+        w = ix.unique_writer(g.a)
+        dot = prog.instrs[w] if w is not None else None
+        if dot is None or dot.op != V.OP_DOT or dot.epi or sc[w] != sc[gi] or w > gi or ix.live_readers(g.a) != [gi]:
+            continue
+        M, N, K, G = _dot_fields_pass(dot)[:4]
+        if G != 1 or M > 0xFFFF or _dt(prog, g.dst) != _dt(prog, g.a) or g.n != M * N:
+            continue
+        if _merged(*_view_desc(prog, g.aux + 1)) != _merged([N, M], [1, N], 0):
+            continue
+        a1, b1 = transposed(dot.bview, K, N), transposed(dot.aview, M, K)
+        if a1 is None or b1 is None:
+            continue
+        dot.a, dot.aview, dot.b, dot.bview = dot.b, a1, dot.a, b1
+        dot.n, dot.imm, dot.dst = N, (M << 16) | K, g.dst
+        prog.instrs[gi] = V.Instr(V.OP_NOP)
+
+
 def fuse_views(prog: V.VMProgram) -> None:
     if _off("PJRT_OCL_VIEWFOLD"):
         return
@@ -1711,6 +1752,7 @@ def run_all(prog: V.VMProgram) -> None:
     """The pass pipeline (lowering.py:3027-3106, with the order noted above)."""
     compose_affines(prog)
     fuse_matmul_views(prog)
+    fold_dot_transposes(prog)
     fuse_views(prog)
     dce(prog)
     fuse_norm(prog)

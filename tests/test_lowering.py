@@ -446,3 +446,37 @@ def test_planted_pass_mistake_is_caught(monkeypatch):
     assert V.OP_GELU not in live_ops(prog)
     ln = [i for i in prog.instrs if i.op == V.OP_LAYERNORM_AFFINE]
     assert ln and not prog.aux[ln[0].aux] & V.LN_GELU
+
+
+# --- a product that is transposed (the gradient of a weight) -------------------------------------
+
+@pytest.mark.parametrize("M,K,N,lc,rc", [(5, 24, 36, 0, 0), (8, 3, 16, 1, 0), (7, 9, 4, 1, 1), (6, 10, 1, 0, 0),
+                                         (1, 10, 6, 0, 1)])
+def test_transposed_product_is_the_swapped_product(M, K, N, lc, rc):
+    """transpose(dot_general(a, b)) lowers to one matmul with the operands swapped,
+    in every layout of the two, with the unfused program's values bit for bit; not
+    where the product itself is also returned."""
+    ta, tb = ((M, K) if lc == 1 else (K, M)), ((K, N) if rc == 0 else (N, K))
+    A, B, C, CT = (f"tensor<{a}x{b}xf32>" for a, b in (ta, tb, (M, N), (N, M)))
+
+    def text(also):
+        ret, ty = ("%1, %0", f"{CT}, {C}") if also else ("%1", CT)
+        return f"""
+module @jit_f {{
+  func.func public @main(%arg0: {A}, %arg1: {B}) -> ({ty}) {{
+    %0 = stablehlo.dot_general %arg0, %arg1, contracting_dims = [{lc}] x [{rc}], precision = [DEFAULT, DEFAULT] : ({A}, {B}) -> {C}
+    %1 = stablehlo.transpose %0, dims = [1, 0] : ({C}) -> {CT}
+    return {ret} : {ty}
+  }}
+}}
+"""
+    rng = np.random.default_rng(11)
+    args = [rng.standard_normal(ta).astype(np.float32), rng.standard_normal(tb).astype(np.float32)]
+    fused, got, plain = both(text(False), args)
+    assert live_ops(fused) == [V.OP_DOT]
+    np.testing.assert_array_equal(got[0], plain[0])
+    fused, got, plain = both(text(True), args)
+    if M > 1 and N > 1:
+        assert V.OP_GATHER_STRIDED in live_ops(fused)
+    for x, y in zip(got, plain):
+        np.testing.assert_array_equal(x, y)
