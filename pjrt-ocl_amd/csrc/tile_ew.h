@@ -400,6 +400,62 @@ VM_DEV void copy_elem(gbyte* d, uint64_t di, const gbyte* s, uint64_t si, uint32
   }
 }
 
+// Compare and select on whole 16-byte groups of 4-byte elements (a relu's mask and
+// its gradient): four steps' loads issued before the first store.  One element a
+// step, each waiting on its own loads, a lane took 30-49 us for its share of 1024 x
+// 2048 f32, now 4.5-11.  Predicate as bits of {less, equal, greater, unordered}.
+template <typename T>
+VM_DEV void ew_cmp4(uint32_t p, gbyte* d, const gbyte* a, const gbyte* b, uint64_t q0, uint64_t q1) {
+  typedef T v4t __attribute__((ext_vector_type(4)));
+  // predicates 0-5: eq ne lt le gt ge (ne is also true of unordered operands)
+  const uint32_t bits = p == 0 ? 2u : p == 1 ? 13u : p == 2 ? 1u : p == 3 ? 3u : p == 4 ? 4u : 6u;
+  const bool lt = bits & 1, eq = bits & 2, gt = bits & 4, un = bits & 8;
+  constexpr uint32_t U = 4;
+  for (uint64_t q = q0 + threadIdx.x; q < q1; q += U * kBlock) {
+    v4t x[U], y[U];
+#pragma unroll
+    for (uint32_t k = 0; k < U; ++k) {
+      const uint64_t i = min(q + k * kBlock, q1 - 1);
+      x[k] = ((const VM_G v4t*)a)[i];
+      y[k] = ((const VM_G v4t*)b)[i];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < U; ++k) {
+      if (q + k * kBlock >= q1) break;
+      uint32_t r = 0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const T u = x[k][c], v = y[k][c];
+        const bool t = u < v ? lt : u > v ? gt : u == v ? eq : un;
+        r |= uint32_t(t) << (8 * c);
+      }
+      ((VM_G uint32_t*)d)[q + k * kBlock] = r;
+    }
+  }
+}
+VM_DEV void ew_select4(gbyte* d, const gbyte* pr, const gbyte* a, const gbyte* b, uint64_t q0, uint64_t q1) {
+  constexpr uint32_t U = 4;
+  for (uint64_t q = q0 + threadIdx.x; q < q1; q += U * kBlock) {
+    v4u x[U], y[U];
+    uint32_t m[U];
+#pragma unroll
+    for (uint32_t k = 0; k < U; ++k) {
+      const uint64_t i = min(q + k * kBlock, q1 - 1);
+      m[k] = ((const VM_G uint32_t*)pr)[i];
+      x[k] = ((const VM_G v4u*)a)[i];
+      y[k] = ((const VM_G v4u*)b)[i];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < U; ++k) {
+      if (q + k * kBlock >= q1) break;
+      v4u r;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) r[c] = (m[k] >> (8 * c)) & 0xFF ? x[k][c] : y[k][c];
+      ((VM_G v4u*)d)[q + k * kBlock] = r;
+    }
+  }
+}
+
 // Compare, select, convert, bitcast, is_finite, LTS: mixed-dtype subops.
 VM_DEV void ew_special(Args A, uint32_t ti, uint64_t e0, uint64_t e1) {
   A = uargs(A);
@@ -413,7 +469,14 @@ VM_DEV void ew_special(Args A, uint32_t ti, uint64_t e0, uint64_t e1) {
   switch (sub) {
     case SUB_CMP: {
       const uint32_t p = uni(t.p[2]);
-      for (uint64_t i = e0 + tid; i < e1; i += kBlock) {
+      uint64_t i0 = e0;
+      if ((adt == DT_F32 || adt == DT_I32) && (e0 & 3) == 0 && ((uintptr_t(a) | uintptr_t(b)) & 15) == 0 &&
+          (uintptr_t(d) & 3) == 0) {
+        if (adt == DT_F32) ew_cmp4<float>(p, d, a, b, e0 >> 2, e1 >> 2);
+        else ew_cmp4<int32_t>(p, d, a, b, e0 >> 2, e1 >> 2);
+        i0 = e1 & ~uint64_t(3);
+      }
+      for (uint64_t i = i0 + tid; i < e1; i += kBlock) {
         bool r;
         switch (adt) {
           case DT_I32: r = cmp_pred(p, gcast<int32_t>(a)[i], gcast<int32_t>(b)[i]); break;
@@ -430,7 +493,12 @@ VM_DEV void ew_special(Args A, uint32_t ti, uint64_t e0, uint64_t e1) {
     case SUB_SELECT: {
       const gbyte* pr = resolve(A, t.p[3]);
       const uint32_t es = dt_size(dt);
-      for (uint64_t i = e0 + tid; i < e1; i += kBlock) copy_elem(d, i, pr[i] ? a : b, i, es);
+      uint64_t i0 = e0;
+      if (es == 4 && (e0 & 3) == 0 && ((uintptr_t(a) | uintptr_t(b) | uintptr_t(d)) & 15) == 0 && (uintptr_t(pr) & 3) == 0) {
+        ew_select4(d, pr, a, b, e0 >> 2, e1 >> 2);
+        i0 = e1 & ~uint64_t(3);
+      }
+      for (uint64_t i = i0 + tid; i < e1; i += kBlock) copy_elem(d, i, pr[i] ? a : b, i, es);
       return;
     }
     case SUB_CONVERT:

@@ -155,6 +155,20 @@ VM_DEV bool gather_splat(const VM_K int32_t* aux, uint32_t x, gbyte* d, const gb
   return true;
 }
 
+template <typename T>
+VM_DEV void gather_elems(const ViewMap& m, gbyte* d, const gbyte* a, uint32_t e0, uint32_t e1) {
+  constexpr uint32_t U = 8;
+  for (uint32_t i = e0 + threadIdx.x; i < e1; i += U * kBlock) {
+    T x[U];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) x[u] = gcast<T>(a)[view_at(m, nullptr, 1, min(i + u * kBlock, e1 - 1))];
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u)
+      if (i + u * kBlock < e1) gcast<T>(d)[i + u * kBlock] = x[u];
+  }
+}
+
+
 VM_TILE void gather_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi, bool scatter) {
   A = uargs(A);
   const VM_K Task& t = task_of(A, ti);
@@ -171,6 +185,15 @@ VM_TILE void gather_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi, bool sc
   // which a qualifying view makes a multiple of the elements per 16 bytes
   if (!scatter && gather_splat(aux, t.p[0], d, a, e0, e1, es)) return;
   if (gather_wide(aux, t.p[0], d, a, e0, e1, es, scatter)) return;
+  // Element by element (a transpose's strided side): the index map decoded once per
+  // tile (invariant-divisor quotients) and eight elements' loads issued before the
+  // first store; one at a time, 4096 elements cost 29-37 us.
+  if (!scatter && rank <= kViewRank && n <= 0xFFFFFFF0u && (es == 4 || es == 2)) {
+    const ViewMap m = view_map(aux, t.p[0] + 1);
+    if (es == 4) gather_elems<uint32_t>(m, d, a, uint32_t(e0), uint32_t(e1));
+    else gather_elems<uint16_t>(m, d, a, uint32_t(e0), uint32_t(e1));
+    return;
+  }
   if (rank > 8) {        // wide maps: direct evaluation per element
     for (uint64_t i = e0 + threadIdx.x; i < e1; i += kBlock) {
       const int64_t j = view_index(aux, t.p[0], i);

@@ -226,6 +226,43 @@ def test_convert_f32_to_bf16_bit_patterns():
     assert bad.size == 0, [(hex(int(bits[i])), hex(int(got[0][i])), hex(int(want[i]))) for i in bad[:8]]
 
 
+@pytest.mark.parametrize("n", [4, 1023, 4096, 12289])
+@pytest.mark.parametrize("dt", ["f32", "i32"])
+def test_compare_select_groups_bit_exact(n, dt):
+    """Compare (all six predicates) and select on whole groups of four and their
+    tails, with NaN, infinities, zeros of both signs and equal values."""
+    rng = np.random.default_rng(44)
+    if dt == "f32":
+        pool = np.array([0.0, -0.0, 1.5, -1.5, np.inf, -np.inf, np.nan, 3.0], np.float32)
+    else:
+        pool = np.array([0, -1, 5, -5, 2 ** 31 - 1, -2 ** 31, 7, 8], np.int32)
+    a, b = rng.choice(pool, n), rng.choice(pool, n)
+    g = G.Graph()
+    x, y = g.input((n,), dt), g.input((n,), dt)
+    preds = ["EQ", "NE", "LT", "LE", "GT", "GE"]
+    masks = [g.compare(x, y, p) for p in preds]
+    g.output(*masks, *(g.select(m, x, y) for m in masks))
+    got = run_gpu(blob_for(g.build())[0], [a, b])
+    want = [a == b, a != b, a < b, a <= b, a > b, a >= b]
+    for k, m in enumerate(want):
+        np.testing.assert_array_equal(np.asarray(got[k]) != 0, m, err_msg=preds[k])
+        np.testing.assert_array_equal(np.asarray(got[6 + k]).view(np.uint32), np.where(m, a, b).view(np.uint32))
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "i32"])
+@pytest.mark.parametrize("shape,perm", [((67, 130), (1, 0)), ((5, 33, 70), (2, 0, 1)), ((3, 5, 7, 41), (3, 1, 0, 2)),
+                                        ((4096, 3), (1, 0)), ((2, 1), (1, 0))])
+def test_transposes_bit_exact(dt, shape, perm):
+    """Gathers whose innermost axis is strided, ranks two to four, ragged tiles."""
+    rng = np.random.default_rng(45)
+    a = rng.integers(0, 60000, shape)
+    a = a.astype(np.uint16) if dt == "bf16" else a.astype(np.int32) if dt == "i32" else a.astype(np.float32)
+    g = G.Graph()
+    g.output(g.transpose(g.input(shape, dt), perm))
+    got = run_gpu(blob_for(g.build())[0], [a])[0]
+    np.testing.assert_array_equal(np.asarray(got).view(a.dtype), a.transpose(perm))
+
+
 # --- reductions and row ops ------------------------------------------------------------------
 
 @pytest.mark.parametrize("kind", [0, 1, 2, 3])
