@@ -147,7 +147,7 @@ VM_DEV uint32_t pack_h2(float a, float b) {
 // registers, the LDS slots of K and V chunks past P.hd are zeroed once per sweep
 // by the lanes that own them (which skip those transfers), and O's columns past
 // P.hd are not stored.
-template <int HD, bool BF16, bool PAD>
+template <int HD, bool BF16, bool PAD, int U>
 VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint32_t vrow0, uint32_t vlo,
                             uint32_t vhi) {
   const VM_K Task& t = task_of(A, ti);
@@ -163,7 +163,7 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
   constexpr int KS = HD / 16;            // MFMA steps over hd for S
   constexpr int DB = HD / 32;            // 32-row d blocks of O^T
   const uint32_t lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6), g = lane >> 5;
-  const uint32_t qw0 = row0 + 64 * wave;                    // this wave's first row
+  const uint32_t qw0 = row0 + 32 * U * wave;                    // this wave's first row
   const VM_G uint16_t* Q = gcast<uint16_t>(resolve(A, t.a)) + uint64_t(h) * T * hd;
   const VM_G uint16_t* K = gcast<uint16_t>(resolve(A, t.b)) + uint64_t(h) * C * hd;
   const VM_G uint16_t* V = gcast<uint16_t>(resolve(A, t.p[0])) + uint64_t(h) * C * hd;
@@ -171,26 +171,26 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
 
   // Q^T fragments (B operand) of both sub-tiles: column = query, 8 consecutive hd
   // values; rows past T re-read row T - 1 (results not stored)
-  u16x8 qf[2][KS];
+  u16x8 qf[U][KS];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < U; ++u) {
     const uint32_t qr = min(qw0 + 32 * u + (lane & 31), T - 1);
 #pragma unroll
     for (int s = 0; s < KS; ++s)
       qf[u][s] = (!PAD || 16 * s + 8 * g < hd) ? *(const VM_G u16x8*)(Q + uint64_t(qr) * hd + s * 16 + 8 * g)
                                                 : u16x8{};
   }
-  f32x16 o[2][DB];
+  f32x16 o[U][DB];
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < U; ++u)
 #pragma unroll
     for (int i = 0; i < DB; ++i) o[u][i] = f32x16{};
-  float m_run[2] = {-INFINITY, -INFINITY}, l_part[2] = {0.0f, 0.0f};
+  float m_run[2] = {-INFINITY, -INFINITY}, l_part[2] = {0.0f, 0.0f};      // (U = 1: the second unused)
   const float sl2 = P.scale * 1.4426950408889634f;
 
   // keys this block needs: up to the last query's causal limit
   const int32_t shift = int32_t(C) - int32_t(T);
-  const uint32_t qmax = min(row0 + kAttnRows, T) - 1;
+  const uint32_t qmax = min(row0 + 128 * U, T) - 1;
   uint32_t kend = C;
   if (P.causal) kend = min(C, uint32_t(max(0, int32_t(qmax) + shift + 1)));
   const uint32_t nblk = (kend + kAttnKeys - 1) / kAttnKeys;
@@ -198,7 +198,7 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
   // and last row
   const bool wave_rows = qw0 < T;
   const int32_t wq_lo = int32_t(qw0) + shift;
-  const int32_t wq_hi = int32_t(min(qw0 + 63, T - 1)) + shift;
+  const int32_t wq_hi = int32_t(min(qw0 + 32 * U - 1, T - 1)) + shift;
 
   // Staging: per block, kRounds transfers per operand and thread.  Round j of
   // wave w, lane l fills stage bytes 4096 j + 1024 w + 16 l of the operand: key
@@ -333,15 +333,18 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
 #pragma unroll
       for (int st = 0; st < KS; ++st)
         kf[kh][st] = *(const lds_u16x8*)(S + (kh * 32 + krow) * L::kRow + (((2 * uint32_t(st) + g) ^ ksw) * 16));
-    s0[0] = s0[1] = s1[0] = s1[1] = f32x16{};
+    s0[0] = s0[1] = f32x16{};
+    if constexpr (U == 2) s1[0] = s1[1] = f32x16{};
 #pragma unroll
     for (int st = 0; st < KS; ++st)
 #pragma unroll
       for (int kh = 0; kh < 2; ++kh) s0[kh] = mfma16<BF16>(kf[kh][st], qf[0][st], s0[kh]);
+    if constexpr (U == 2) {
 #pragma unroll
-    for (int st = 0; st < KS; ++st)
+      for (int st = 0; st < KS; ++st)
 #pragma unroll
-      for (int kh = 0; kh < 2; ++kh) s1[kh] = mfma16<BF16>(kf[kh][st], qf[1][st], s1[kh]);
+        for (int kh = 0; kh < 2; ++kh) s1[kh] = mfma16<BF16>(kf[kh][st], qf[1][st], s1[kh]);
+    }
   };
   // One 64-key block: S^T of both sub-tiles (K fragments read once, used twice),
   // sub-tile 0's softmax while sub-tile 1's S^T is on the matrix cores, then
@@ -353,7 +356,7 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
     u16x8 p0[4], p1[4];
     if constexpr (decltype(maskc)::value) mask_s(s0, 0, key0);
     probs(maxc, s0, 0, p0);
-    if constexpr (decltype(maskc)::value) mask_s(s1, 1, key0);
+    if constexpr (U == 2 && decltype(maskc)::value) mask_s(s1, 1, key0);
     u16x8 vf[DB][4];
 #pragma unroll
     for (int db = 0; db < DB; ++db)
@@ -367,11 +370,13 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
       for (int db = 0; db < DB; ++db) o[0][db] = mfma16<BF16>(vf[db][ks], p0[ks], o[0][db]);
-    probs(maxc, s1, 1, p1);
+    if constexpr (U == 2) {
+      probs(maxc, s1, 1, p1);
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+      for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
-      for (int db = 0; db < DB; ++db) o[1][db] = mfma16<BF16>(vf[db][ks], p1[ks], o[1][db]);
+        for (int db = 0; db < DB; ++db) o[1][db] = mfma16<BF16>(vf[db][ks], p1[ks], o[1][db]);
+    }
   };
   // Exact pass 1: the true scaled row maxima over all visible keys.
   auto max_body = [&](auto maskc, auto, const lds_u8* S, uint32_t key0) {
@@ -379,10 +384,10 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
     s_tiles(S, s0, s1);
     if constexpr (decltype(maskc)::value) {
       mask_s(s0, 0, key0);
-      mask_s(s1, 1, key0);
+      if constexpr (U == 2) mask_s(s1, 1, key0);
     }
     m_run[0] = fmaxf(m_run[0], row_max(s0));
-    m_run[1] = fmaxf(m_run[1], row_max(s1));
+    if constexpr (U == 2) m_run[1] = fmaxf(m_run[1], row_max(s1));
   };
 
   // One sweep over the key blocks: per block, start the next block's transfers
@@ -430,7 +435,7 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
     m_run[0] = m_run[1] = -INFINITY;
     sweep(max_body);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < U; ++u) {
       l_part[u] = 0.0f;
 #pragma unroll
       for (int i = 0; i < DB; ++i) o[u][i] = f32x16{};
@@ -438,8 +443,8 @@ VM_DEV void attn_block_mfma(Args A, uint32_t ti, uint32_t h, uint32_t row0, uint
     sweep(body);
   }
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const uint32_t ql = 64 * wave + 32 * u + (lane & 31);   // 0..255 within the block
+  for (int u = 0; u < U; ++u) {
+    const uint32_t ql = 32 * U * wave + 32 * u + (lane & 31);   // within the block
     const uint32_t q = row0 + ql;
     const float l = l_part[u] + xor32(l_part[u]);
     if (q < T && vrow0 + ql >= vlo && vrow0 + ql < vhi) {
@@ -561,9 +566,26 @@ VM_DEV void attn_fast(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
     for (uint32_t vb = a / kAttnRows; vb * kAttnRows < b; ++vb) {
       const uint32_t rb = zig ? ((vb & 1) ? nb - 1 - (vb >> 1) : (vb >> 1)) : vb;
       const uint32_t vrow0 = vb * kAttnRows;
-      attn_block_mfma<HD, BF16, PAD>(A, ti, h, rb * kAttnRows, vrow0, max(a, vrow0), min(b, vrow0 + kAttnRows));
+      attn_block_mfma<HD, BF16, PAD, 2>(A, ti, h, rb * kAttnRows, vrow0, max(a, vrow0), min(b, vrow0 + kAttnRows));
     }
   }
+}
+
+// Half a block, 128 rows (32 per wave): an entry of rows [lo, lo + 128) of one half.
+// The scheduler cuts chunks so where whole blocks would leave half the lanes idle
+// (24 heads x 1000 x 64 f16, 96 blocks on 256 lanes: 31.9 -> 26.5 us a launch, of
+// which 6 are the launch's): a half takes more than half a block's time, since K
+// and V fragments serve one sub-tile instead of two.  The rows' arithmetic is the
+// same, but for the exact pass, which all rows of a block (or half) take together.
+template <int HD, bool BF16, bool PAD>
+VM_DEV void attn_half(Args A, uint32_t ti, uint32_t lo) {
+  const VM_K Task& t = task_of(A, ti);
+  const AttnDesc P = attn_desc(A, t);
+  const uint32_t nb = (P.T + kAttnRows - 1) / kAttnRows, Tp = nb * kAttnRows;
+  const uint32_t h = lo / Tp, v = lo - h * Tp, vb = v / kAttnRows, half = v % kAttnRows;
+  const uint32_t rb = P.causal ? ((vb & 1) ? nb - 1 - (vb >> 1) : (vb >> 1)) : vb;
+  const uint32_t row0 = rb * kAttnRows + half;
+  if (h < P.H && row0 < P.T) attn_block_mfma<HD, BF16, PAD, 1>(A, ti, h, row0, v, v, v + kAttnRows / 2);
 }
 
 // ---- f32 operands -------------------------------------------------------------------
@@ -983,6 +1005,33 @@ VM_DEV void attn_h16w_run(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   });
 }
 
+VM_DEV bool attn_fast_ok(Args A, const AttnDesc& P, uint32_t adt, uint32_t dt) {
+  return (adt == DT_BF16 || adt == DT_F16) && P.hd % 8 == 0 && P.hd >= 8 && P.hd <= 128 && !P.qv && !P.vv &&
+         is_kt_view(aux_of(A), P.kv, P.H, P.C, P.hd) && P.scale > 0.0f && (dt == DT_F32 || dt == DT_BF16 || dt == DT_F16);
+}
+
+// An entry of one half block (a leaf of its own: both forms in one leaf would pass
+// the reach of a short branch).
+VM_LEAF void flash_attn_half(Args A, uint32_t ti, uint32_t lo) {
+  A = uargs(A);
+  ti = uni(ti);
+  lo = uni(lo);
+  const VM_K Task& t = task_of(A, ti);
+  const uint32_t hd = attn_desc(A, t).hd;
+  if (((t.tile_op >> 16) & 0xFF) == DT_BF16) {
+    if (hd == 128) attn_half<128, true, false>(A, ti, lo);
+    else if (hd == 64) attn_half<64, true, false>(A, ti, lo);
+    else if (hd > 64) attn_half<128, true, true>(A, ti, lo);
+    else attn_half<64, true, true>(A, ti, lo);
+  } else {
+    if (hd == 128) attn_half<128, false, false>(A, ti, lo);
+    else if (hd == 64) attn_half<64, false, false>(A, ti, lo);
+    else if (hd > 64) attn_half<128, false, true>(A, ti, lo);
+    else attn_half<64, false, true>(A, ti, lo);
+  }
+}
+
+
 // One leaf holds every attention variant inlined, so the kernel's dispatch switch
 // has a single call site for the op.  Each call site costs the kernel code and
 // register moves around it: with the ten variants as leaves of their own, the
@@ -994,9 +1043,7 @@ VM_LEAF void flash_attn_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   const uint32_t adt = (t.tile_op >> 16) & 0xFF, dt = (t.tile_op >> 8) & 0xFF;
   // head sizes other than 64 and 128 (multiples of 8 up to 128) run the next
   // larger kernel on zero-padded rows
-  const bool fast = (adt == DT_BF16 || adt == DT_F16) && P.hd % 8 == 0 && P.hd >= 8 && P.hd <= 128 && !P.qv &&
-                    !P.vv && is_kt_view(aux_of(A), P.kv, P.H, P.C, P.hd) && P.scale > 0.0f &&
-                    (dt == DT_F32 || dt == DT_BF16 || dt == DT_F16);
+  const bool fast = attn_fast_ok(A, P, adt, dt);
   const bool fast32 = adt == DT_F32 && P.hd % 4 == 0 && P.hd >= 4 && P.hd <= 128 && !P.qv && !P.vv &&
                       is_kt_view(aux_of(A), P.kv, P.H, P.C, P.hd) && P.scale > 0.0f &&
                       (dt == DT_F32 || dt == DT_BF16 || dt == DT_F16);
@@ -1016,6 +1063,24 @@ VM_LEAF void flash_attn_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
     else if (P.hd == 64) attn_fast<64, false, false>(A, ti, lo, hi);
     else if (P.hd > 64) attn_fast<128, false, true>(A, ti, lo, hi);
     else attn_fast<64, false, true>(A, ti, lo, hi);
+  }
+}
+
+// Whole blocks of an entry in one leaf, a half at either end in the other.
+VM_DEV void attn_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  constexpr uint32_t kHalf = kAttnRows / 2;
+  const VM_K Task& t = task_of(A, ti);
+  const bool halves = lo % kHalf == 0 && hi % kHalf == 0 &&
+                      attn_fast_ok(A, attn_desc(A, t), (t.tile_op >> 16) & 0xFF, (t.tile_op >> 8) & 0xFF);
+  while (lo < hi) {
+    if (halves && (lo % kAttnRows || hi - lo < kAttnRows)) {
+      flash_attn_half(A, ti, lo);
+      lo += kHalf;
+    } else {
+      const uint32_t end = halves ? hi - hi % kAttnRows : hi;
+      flash_attn_tiles(A, ti, lo, end);
+      lo = end;
+    }
   }
 }
 

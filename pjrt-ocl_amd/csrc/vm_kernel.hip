@@ -48,7 +48,7 @@ VM_DEV void exec_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
     case TOP_SOFTMAX_SEG: softmax_tiles(A, ti, lo, hi); break;
     case TOP_LAYERNORM_SEG: layernorm_tiles(A, ti, lo, hi); break;
     case TOP_MAP_REGION: map_region_tiles(A, ti, lo, hi); break;
-    case TOP_FLASH_ATTN: flash_attn_tiles(A, ti, lo, hi); break;
+    case TOP_FLASH_ATTN: attn_tiles(A, ti, lo, hi); break;
     case TOP_RED_STRIDED: red_strided_tiles(A, ti, lo, hi); break;
     case TOP_GATHER_INDEX: gather_index_tiles(A, ti, lo, hi); break;
     case TOP_ARGMAX_SEG: argmax_tiles(A, ti, lo, hi); break;

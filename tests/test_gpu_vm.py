@@ -995,6 +995,31 @@ def test_flash_attention(dt, hd, causal, T, C):
                                f"flash {dt} hd {hd}")
 
 
+@pytest.mark.parametrize("dt,hd,causal,T", [("bf16", 64, True, 1), ("f16", 128, False, 127), ("bf16", 128, True, 128),
+                                            ("f16", 64, True, 129), ("bf16", 40, False, 257), ("f16", 96, True, 384),
+                                            ("bf16", 128, True, 700), ("bf16", 200, True, 300)])
+def test_flash_attention_half_blocks_bit_exact(dt, hd, causal, T):
+    """Blocks of 256 query rows (5 lanes), halves of 128 (all lanes) and chunks of
+    a half and whole blocks (two products share 32 lanes) do the same
+    arithmetic on a row: the same bits, and those of float64 to the 16-bit P."""
+    rng = np.random.default_rng(1011)
+    H, C = 5, T + 70
+    cast = (lambda x: vmref.bf16_to_f32(vmref.f32_to_bf16(x))) if dt == "bf16" else (
+        lambda x: x.astype(np.float16).astype(np.float32))
+    q, k, v = (cast(rng.standard_normal((H, n, hd)).astype(np.float32)) for n in (T, C, C))
+    g = G.Graph()
+    Q, K, Vv = g.input(q.shape, dt), g.input(k.shape, dt), g.input(v.shape, dt)
+    g.output(g.flash_attention(Q, K, Vv, 1.0 / np.sqrt(hd), causal, out_dtype="f32"),
+             g.flash_attention(Q, K, Vv, 1.0 / np.sqrt(hd), not causal, out_dtype="f32"))
+    prog = g.build()
+    runs = [run_both(prog, [q, k, v], nlanes=n, oracle=None)[0] for n in (5, 32, None)]
+    for i, c in enumerate((causal, not causal)):
+        want = vmref.attention(q, np.transpose(k, (0, 2, 1)), v, 1.0 / np.sqrt(hd), c)
+        assert np.abs(runs[0][i] - want).max() <= 1e-2 * np.abs(want).max()
+        for r in runs[1:]:
+            np.testing.assert_array_equal(r[i], runs[0][i])
+
+
 @pytest.mark.parametrize("hd,dt", [(64, "bf16"), (128, "bf16"), (96, "bf16"), (24, "bf16"), (128, "f32"), (36, "f32"),
                                    (256, "bf16"), (200, "f16")])
 def test_flash_attention_partial_block_inf_value(hd, dt):
