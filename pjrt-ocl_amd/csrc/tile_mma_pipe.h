@@ -24,8 +24,8 @@
 // one slab in flight, and per-element reads of any operand that was transposed or
 // whose rows were not 16-byte aligned):
 //   bf16 1024^3 23.4 -> 14.9, with W^T 180 -> 15.5, x^T 179 -> 15.8; 2048^3 51 -> 33;
-//   f32 1024^3 53.5 -> 31.0, W^T 261 -> 31.4; 1001x777x1130 262 -> 52;
-//   a decoder block over 512 tokens (d 768) 258 -> 175.
+//   f32 1024^3 53.5 -> 31.0, W^T 261 -> 31.4; 1001x777x1130 262 -> 48;
+//   a decoder block over 512 tokens (d 768) 258 -> 145.
 // What bounds a 64-wide tile of 1024 k in a launch of one round (8.9 us in 16
 // bits): ~1.3 us of prologue, then LDS reads and one barrier per 128 k at one wave
 // per SIMD; in f32 (25 us) the matrix cores, 14.6 us of it.
