@@ -356,97 +356,8 @@ VM_TILE void red_strided_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
 }
 
 // ---- row-resident fused ops -------------------------------------------------------------
-// A row of `seg` elements is held in registers as NV v4f per thread (thread t
-// owns v4f slots t, t+256, ...), so a row costs one HBM read and one write.
-// The next row's loads are issued before the current row's reductions.
-
-template <int NV>
-struct Row { v4f v[NV]; };
-
-template <int NV>
-VM_DEV void row_load(Row<NV>& r, const gbyte* p, uint32_t dt, uint64_t base, uint32_t nv4) {
-#pragma unroll
-  for (int k = 0; k < NV; ++k) {
-    const uint32_t q = threadIdx.x + k * kBlock;
-    if (q < nv4) r.v[k] = ld4(p, dt, base + 4ull * q);
-  }
-}
-
-// LAYERNORM_SEG over rows [r0, r1): p0 n_out, p1 seg, p2 eps bits, p3 flags,
-// b = gamma, p4 = beta (LN_AFFINE).
-template <int NV>
-VM_DEV void ln_rows_vec(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
-  A = uargs(A);
-  const VM_K Task& t = task_of(A, ti);
-  float* red = lds_f32();
-  const uint32_t seg = t.p[1], flags = t.p[3];
-  const float eps = __uint_as_float(t.p[2]);
-  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
-  const gbyte* a = resolve(A, t.a);
-  gbyte* d = resolve(A, t.dst);
-  const bool affine = flags & LN_AFFINE, do_gelu = flags & LN_GELU, two_pass = flags & LN_TWO_PASS;
-  const gbyte* gp = resolve(A, affine ? t.b : t.a);
-  const gbyte* bp = resolve(A, affine ? t.p[4] : t.a);
-  const uint32_t nv4 = seg >> 2;
-  const float inv_n = 1.0f / float(seg);
-  // gamma / beta slots of this thread stay in registers for every row
-  Row<NV> g, be;
-  if (affine) {
-    row_load(g, gp, DT_F32, 0, nv4);
-    row_load(be, bp, DT_F32, 0, nv4);
-  }
-  Row<NV> x, xn;
-  row_load(x, a, adt, uint64_t(r0) * seg, nv4);
-  for (uint32_t r = r0; r < r1; ++r) {
-    if (r + 1 < r1) row_load(xn, a, adt, uint64_t(r + 1) * seg, nv4);
-    float s = 0.0f, s2 = 0.0f;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      if (threadIdx.x + k * kBlock < nv4) {
-        const v4f v = x.v[k];
-        s += (v.x + v.y) + (v.z + v.w);
-        if (!two_pass) s2 = fmaf(v.x, v.x, fmaf(v.y, v.y, fmaf(v.z, v.z, fmaf(v.w, v.w, s2))));
-      }
-    }
-    const float mean = block_reduce(s, OpSum(), red) * inv_n;
-    float var;
-    if (two_pass) {
-      float q = 0.0f;
-#pragma unroll
-      for (int k = 0; k < NV; ++k) {
-        if (threadIdx.x + k * kBlock < nv4) {
-          const v4f v = x.v[k];
-          const float dx = v.x - mean, dy = v.y - mean, dz = v.z - mean, dw = v.w - mean;
-          q = fmaf(dx, dx, fmaf(dy, dy, fmaf(dz, dz, fmaf(dw, dw, q))));
-        }
-      }
-      var = block_reduce(q, OpSum(), red + kWaves) * inv_n;
-    } else {
-      var = block_reduce(s2, OpSum(), red + kWaves) * inv_n - mean * mean;
-    }
-    const float rstd = rsqrtf(var + eps);
-    const float shift = -mean * rstd;
-    const uint64_t base = uint64_t(r) * seg;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      const uint32_t q = threadIdx.x + k * kBlock;
-      if (q < nv4) {
-        float y[4] = {x.v[k].x, x.v[k].y, x.v[k].z, x.v[k].w};
-        const float gg[4] = {g.v[k].x, g.v[k].y, g.v[k].z, g.v[k].w};
-        const float bb[4] = {be.v[k].x, be.v[k].y, be.v[k].z, be.v[k].w};
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          float z = fmaf(y[c], rstd, shift);
-          if (affine) z = fmaf(z, gg[c], bb[c]);
-          if (do_gelu) z = gelu(z);
-          y[c] = z;
-        }
-        st4(d, dt, base + 4ull * q, v4f_make(y[0], y[1], y[2], y[3]));
-      }
-    }
-    if (r + 1 < r1) x = xn;
-  }
-}
+// A row of `seg` elements is held in registers, so it costs one HBM read and one
+// write.  The next row's loads are issued before the current row's reductions.
 
 // Wave-per-row layernorm, specialised on the input / output formats.  Each wave64
 // owns every fourth row of the lane's range and holds a row as NV groups of 4
@@ -641,239 +552,10 @@ VM_DEV void ln_rows_fast(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
   else ln_stream<NV, IN_BF16, OUT_BF16, false, FULL>(L, r0 + wave, mine);
 }
 
-// Wave-per-row layernorm for rows up to 4096 elements: each wave64 owns every
-// fourth row of the lane's range, holds it as NV float4 per thread (thread t:
-// float4 slots t, t+64, ...), prefetches its next row before reducing the current
-// one, and reduces with DPP only -- no block barriers, four rows in flight per CU.
-// gamma / beta are staged once into LDS and read back per row.
-template <int NV>
-VM_DEV void ln_rows_wave(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
-  A = uargs(A);
-  const VM_K Task& t = task_of(A, ti);
-  const uint32_t seg = t.p[1], flags = t.p[3];
-  const float eps = __uint_as_float(t.p[2]);
-  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
-  const gbyte* a = resolve(A, t.a);
-  gbyte* d = resolve(A, t.dst);
-  const bool affine = flags & LN_AFFINE, do_gelu = flags & LN_GELU, two_pass = flags & LN_TWO_PASS;
-  const uint32_t nv4 = seg >> 2;
-  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  v4f* lg = lds_ptr<v4f>();
-  v4f* lb = lg + nv4;
-  if (affine) {
-    const VM_G v4f* g4 = (const VM_G v4f*)gcast<float>(resolve(A, t.b));
-    const VM_G v4f* b4 = (const VM_G v4f*)gcast<float>(resolve(A, t.p[4]));
-    for (uint32_t q = threadIdx.x; q < nv4; q += kBlock) {
-      lg[q] = g4[q];
-      lb[q] = b4[q];
-    }
-  }
-  __syncthreads();
-  const float inv_n = 1.0f / float(seg);
-  v4f x[NV], xn[NV];
-  auto load_row = [&](v4f (&dst)[NV], uint32_t r) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      const uint32_t q = lane + 64 * k;
-      if (q < nv4) dst[k] = ld4(a, adt, uint64_t(r) * seg + 4ull * q);
-    }
-  };
-  uint32_t r = r0 + wave;
-  if (r < r1) load_row(x, r);
-  for (; r < r1; r += kWaves) {
-    if (r + kWaves < r1) load_row(xn, r + kWaves);
-    float s = 0.0f, s2 = 0.0f;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      if (lane + 64 * k < nv4) {
-        s += (x[k].x + x[k].y) + (x[k].z + x[k].w);
-        if (!two_pass) s2 = fmaf(x[k].x, x[k].x, fmaf(x[k].y, x[k].y, fmaf(x[k].z, x[k].z, fmaf(x[k].w, x[k].w, s2))));
-      }
-    }
-    const float mean = wave_sum(s) * inv_n;
-    float var;
-    if (two_pass) {
-      float q2 = 0.0f;
-#pragma unroll
-      for (int k = 0; k < NV; ++k) {
-        if (lane + 64 * k < nv4) {
-          const v4f dv = x[k] - mean;
-          q2 = fmaf(dv.x, dv.x, fmaf(dv.y, dv.y, fmaf(dv.z, dv.z, fmaf(dv.w, dv.w, q2))));
-        }
-      }
-      var = wave_sum(q2) * inv_n;
-    } else {
-      var = wave_sum(s2) * inv_n - mean * mean;
-    }
-    const float rstd = rsqrtf(var + eps);
-    const float shift = -mean * rstd;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      const uint32_t q = lane + 64 * k;
-      if (q < nv4) {
-        v4f z;
-        z.x = fmaf(x[k].x, rstd, shift);
-        z.y = fmaf(x[k].y, rstd, shift);
-        z.z = fmaf(x[k].z, rstd, shift);
-        z.w = fmaf(x[k].w, rstd, shift);
-        if (affine) {
-          const v4f gg = lg[q], bb = lb[q];
-          z.x = fmaf(z.x, gg.x, bb.x);
-          z.y = fmaf(z.y, gg.y, bb.y);
-          z.z = fmaf(z.z, gg.z, bb.z);
-          z.w = fmaf(z.w, gg.w, bb.w);
-        }
-        if (do_gelu) {
-          z.x = gelu(z.x);
-          z.y = gelu(z.y);
-          z.z = gelu(z.z);
-          z.w = gelu(z.w);
-        }
-        st4(d, dt, uint64_t(r) * seg + 4ull * q, z);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < NV; ++k) x[k] = xn[k];
-  }
-}
-
-// Any seg / alignment: three passes over the row in global memory.
-VM_DEV void ln_rows_generic(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
-  A = uargs(A);
-  const VM_K Task& t = task_of(A, ti);
-  float* red = lds_f32();
-  const uint32_t seg = t.p[1], flags = t.p[3];
-  const float eps = __uint_as_float(t.p[2]);
-  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
-  const gbyte* a = resolve(A, t.a);
-  gbyte* d = resolve(A, t.dst);
-  const bool affine = flags & LN_AFFINE, do_gelu = flags & LN_GELU, two_pass = flags & LN_TWO_PASS;
-  const gbyte* gp = resolve(A, affine ? t.b : t.a);
-  const gbyte* bp = resolve(A, affine ? t.p[4] : t.a);
-  const float inv_n = 1.0f / float(seg);
-  for (uint32_t r = r0; r < r1; ++r) {
-    const uint64_t base = uint64_t(r) * seg;
-    float s = 0.0f, s2 = 0.0f;
-    for (uint32_t j = threadIdx.x; j < seg; j += kBlock) {
-      const float v = load_f(a, adt, base + j);
-      s += v;
-      s2 = fmaf(v, v, s2);
-    }
-    const float mean = block_reduce(s, OpSum(), red) * inv_n;
-    float var;
-    if (two_pass) {
-      float q = 0.0f;
-      for (uint32_t j = threadIdx.x; j < seg; j += kBlock) {
-        const float dv = load_f(a, adt, base + j) - mean;
-        q = fmaf(dv, dv, q);
-      }
-      var = block_reduce(q, OpSum(), red + kWaves) * inv_n;
-    } else {
-      var = block_reduce(s2, OpSum(), red + kWaves) * inv_n - mean * mean;
-    }
-    const float rstd = rsqrtf(var + eps);
-    const float shift = -mean * rstd;
-    for (uint32_t j = threadIdx.x; j < seg; j += kBlock) {
-      float z = fmaf(load_f(a, adt, base + j), rstd, shift);
-      if (affine) z = fmaf(z, load_f(gp, DT_F32, j), load_f(bp, DT_F32, j));
-      if (do_gelu) z = gelu(z);
-      store_f(d, dt, base + j, z);
-    }
-  }
-}
-
-VM_DEV bool row_vec_ok(uint32_t seg, const gbyte* a, const gbyte* d, uint32_t adt, uint32_t dt) {
-  const bool fmt = (adt == DT_F32 || adt == DT_BF16 || adt == DT_F16) &&
-                   (dt == DT_F32 || dt == DT_BF16 || dt == DT_F16);
-  return fmt && (seg & 3) == 0 && seg <= 8 * 4 * kBlock && ((uintptr_t(a) | uintptr_t(d)) & 15) == 0;
-}
-
-VM_DEV void layernorm_rows(Args A, uint32_t ti, uint32_t lo, uint32_t hi);
-
-// LAYERNORM_SEG tiles [lo, hi).  Task p5 (scheduler, extension): the lanes'
-// rows interleaved -- logical row i is row (i % p5) * (n_out / p5) + i / p5, so
-// that at any moment the lanes stream neighbouring rows of the input (C2,
-// alternating runs on one MI355X: 38.7 against 39.6 us).  The streaming row
-// kernel applies it per row;
-// the other row kernels take the rows one by one.
-// A leaf with its row kernels inlined, for the reason ew_tile gives: as a
-// function calling them it saved and reloaded 14 registers in scratch around
-// every entry (C2, alternating runs: 41.6-41.8 against 42.2 us).
-VM_LEAF void layernorm_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
-  A = uargs(A);
-  const VM_K Task& t = task_of(A, ti);
-  const uint32_t n_out = t.p[0], seg = t.p[1];
-  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
-  hi = min(hi, n_out);
-  if (lo >= hi) return;
-  bool ok = row_vec_ok(seg, resolve(A, t.a), resolve(A, t.dst), adt, dt);
-  if (ok && (t.p[3] & LN_AFFINE)) ok = ((uintptr_t(resolve(A, t.b)) | uintptr_t(resolve(A, t.p[4]))) & 15) == 0;
-  const uint32_t nv4 = seg >> 2;
-  const bool fast = ok && (adt == DT_F32 || adt == DT_BF16) && (dt == DT_F32 || dt == DT_BF16) && nv4 <= 16 * 64;
-  if (t.p[5] && !fast) {
-    const uint32_t c = t.p[5], stride = n_out / c;
-    for (uint32_t i = lo; i < hi; ++i) {
-      const uint32_t r = (i % c) * stride + i / c;
-      layernorm_rows(A, ti, r, r + 1);
-    }
-    return;
-  }
-  layernorm_rows(A, ti, lo, hi);
-}
-
-// Rows [lo, hi) of a LAYERNORM_SEG task through the fitting row kernel (rows
-// taken as they are, except the streaming kernel, which applies p5 itself).
-VM_DEV void layernorm_rows(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
-  const VM_K Task& t = task_of(A, ti);
-  const uint32_t seg = t.p[1];
-  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
-  bool ok = row_vec_ok(seg, resolve(A, t.a), resolve(A, t.dst), adt, dt);
-  if (ok && (t.p[3] & LN_AFFINE)) ok = ((uintptr_t(resolve(A, t.b)) | uintptr_t(resolve(A, t.p[4]))) & 15) == 0;
-  if (!ok) return ln_rows_generic(A, ti, lo, hi);
-  const uint32_t nv4 = seg >> 2;
-  if ((adt == DT_F32 || adt == DT_BF16) && (dt == DT_F32 || dt == DT_BF16) && nv4 <= 16 * 64) {
-    const bool ib = adt == DT_BF16, ob = dt == DT_BF16;
-#define VM_LN_FAST(NVV, FULLV)                                                               \
-    {                                                                                         \
-      if (ib) return ob ? ln_rows_fast<NVV, true, true, FULLV>(A, ti, lo, hi)                  \
-                        : ln_rows_fast<NVV, true, false, FULLV>(A, ti, lo, hi);                \
-      return ob ? ln_rows_fast<NVV, false, true, FULLV>(A, ti, lo, hi)                         \
-                : ln_rows_fast<NVV, false, false, FULLV>(A, ti, lo, hi);                       \
-    }
-    if (nv4 == 4 * 64) VM_LN_FAST(4, true)
-    if (nv4 < 4 * 64) VM_LN_FAST(4, false)
-    if (nv4 == 16 * 64) VM_LN_FAST(16, true)
-    VM_LN_FAST(16, false)
-#undef VM_LN_FAST
-  }
-  if (nv4 <= 2 * 64) return ln_rows_wave<2>(A, ti, lo, hi);
-  if (nv4 <= 4 * 64) return ln_rows_wave<4>(A, ti, lo, hi);
-  if (nv4 <= 8 * 64) return ln_rows_wave<8>(A, ti, lo, hi);
-  if (nv4 <= 16 * 64) return ln_rows_wave<16>(A, ti, lo, hi);
-  if (nv4 <= 1 * kBlock) return ln_rows_vec<1>(A, ti, lo, hi);
-  if (nv4 <= 2 * kBlock) return ln_rows_vec<2>(A, ti, lo, hi);
-  if (nv4 <= 4 * kBlock) return ln_rows_vec<4>(A, ti, lo, hi);
-  return ln_rows_vec<8>(A, ti, lo, hi);
-}
-
-// SOFTMAX_SEG rows: exp(x - max) / sum, f32 arithmetic.
-//
-// Rows are read in groups of 4 elements with 16- or 8-byte accesses that need only
-// the element's own alignment, so odd row lengths stream like even ones; a row whose
+// Rows in groups of 4 elements, read with 16- or 8-byte accesses that need only the
+// element's own alignment, so odd row lengths stream like even ones; a row whose
 // length is not a multiple of 4 ends in a group that overlaps the one before (its
-// repeated elements count once in the sum and are stored twice, with one value).
-// Loads are not predicated (ln_load's reason): groups past the row re-read its last.
-// Three forms, by how many registers a row takes:
-//   up to 4096 elements: a wave per row, four rows in flight per CU and the next
-//     ones prefetched, DPP reductions and no block barrier;
-//   up to 32768: a row over the block's registers, the next row prefetched;
-//   longer: two passes over the row, the first keeping a running maximum and sum
-//     per thread.
-// Memory bounds them (MI355X, whole launches): 512 x 32000 f32 257 -> 34.9 us (3.75
-// TB/s: two rows per CU, so the first row's load and the last one's store overlap
-// nothing), 8192 x 4096 65 -> 53 (5.06), 4096 x 1000 20 -> 10.6, 1000 x 777 14.4 -> 6.9;
-// before, odd and long rows were read three times in single elements and a row of
-// any length took the whole block and two block barriers.
+// repeated elements count once in sums).
 template <bool IN16>
 struct RowRaw {
   typedef typename std::conditional<IN16, v2u, v4f>::type Raw;
@@ -915,6 +597,293 @@ VM_DEV float sum4(v4f v, uint32_t dup) {
   return (dup > 0 ? 0.0f : v.x) + (dup > 1 ? 0.0f : v.y) + ((dup > 2 ? 0.0f : v.z) + v.w);
 }
 
+// As row_store for a group read after other groups were stored: a destination that
+// is the source may hold the results in its repeated elements already.
+VM_DEV void row_store_own(gbyte* row, uint32_t dt, uint32_t e, v4f v, uint32_t dup) {
+  if (!dup) return row_store(row, dt, e, v);
+  if (dup < 2) store_f(row, dt, e + 1, v.y);
+  if (dup < 3) store_f(row, dt, e + 2, v.z);
+  store_f(row, dt, e + 3, v.w);
+}
+
+// Layernorm rows of any length and alignment, f16 rows, and rows past the streaming
+// kernel's 4096: softmax_rows' forms (below), a row over the TH threads.
+// gamma and beta stay in registers, for rows over 8192 elements they come from L2
+// for every row.  Measured (MI355X, whole launches, us; before: f16 rows through
+// scalar conversions and odd or long rows three times in single elements):
+//   GELU, f32 -> bf16: 1000 x 777 17.5 -> 7.4, 3000 x 4097 187 -> 37, 2048 x 8192 44.7
+//   -> 36, 100 x 30000 96.5 -> 30, 64 x 50257 158 -> 41; f16 4096 x 4096 170 -> 36,
+//   4096 x 1024 50 -> 13.4.  A row or two per lane lose a little to the groups'
+//   masks (300 x 5000 10.4 -> 11.2; f16 2000 x 768 8.7 -> 9.1).
+struct LnTask {
+  const gbyte *a, *gp, *bp;
+  gbyte* d;
+  uint32_t dt, adt, ichunk, istride;
+  float eps, inv_n;
+  bool affine, do_gelu, two_pass;
+  VM_DEV LnTask(Args A, const VM_K Task& t) {
+    const uint32_t flags = t.p[3];
+    a = resolve(A, t.a);
+    d = resolve(A, t.dst);
+    affine = flags & LN_AFFINE, do_gelu = flags & LN_GELU, two_pass = flags & LN_TWO_PASS;
+    gp = resolve(A, affine ? t.b : t.a);
+    bp = resolve(A, affine ? t.p[4] : t.a);
+    dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
+    eps = __uint_as_float(t.p[2]);
+    inv_n = 1.0f / float(t.p[1]);
+    ichunk = max(1u, t.p[5]);
+    istride = t.p[0] / ichunk;
+  }
+  VM_DEV uint32_t row(uint32_t i) const { return (i % ichunk) * istride + i / ichunk; }     // p5, layernorm_tiles
+  VM_DEV v4f out(v4f x, float rstd, float shift, v4f g, v4f b) const {
+    v4f z = v4f_make(fmaf(x.x, rstd, shift), fmaf(x.y, rstd, shift), fmaf(x.z, rstd, shift), fmaf(x.w, rstd, shift));
+    if (affine) z = v4f_make(fmaf(z.x, g.x, b.x), fmaf(z.y, g.y, b.y), fmaf(z.z, g.z, b.z), fmaf(z.w, g.w, b.w));
+    if (do_gelu) z = v4f_make(gelu(z.x), gelu(z.y), gelu(z.z), gelu(z.w));
+    return z;
+  }
+};
+VM_DEV float sumsq4(v4f v, uint32_t dup) { return sum4(v4f_make(v.x * v.x, v.y * v.y, v.z * v.z, v.w * v.w), dup); }
+
+template <int NV, bool IN16, int TH>
+VM_DEV void ln_rows(Args A, uint32_t ti, uint32_t r0, uint32_t r1, uint32_t step) {
+  typedef RowRaw<IN16> R;
+  const VM_K Task& t = task_of(A, ti);
+  const LnTask L(A, t);
+  float* red = lds_f32();
+  const RowGroups G(t.p[1]);
+  const bool bf = L.adt == DT_BF16;
+  const uint32_t me = TH == 64 ? threadIdx.x & 63 : threadIdx.x, dsz = L.dt == DT_F32 ? 4 : 2;
+  if (r0 >= r1) return;
+  typename R::Raw x[NV], xn[NV];
+  auto load = [&](typename R::Raw (&buf)[NV], uint32_t i) {
+    const gbyte* row = L.a + uint64_t(L.row(i)) * G.seg * (IN16 ? 2 : 4);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) buf[k] = R::load(row, G.at(min(me + TH * k, G.n - 1)));
+  };
+  auto sum = [&](float v, float* p) {
+    if constexpr (TH == 64) return wave_sum(v);
+    else return block_reduce(v, OpSum(), p);
+  };
+  constexpr int U = NV <= 16 ? NV : 8;
+  v4f g[U], b[U];
+  auto load_gb = [&](int k0) {
+    if (!L.affine) return;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t e = G.at(min(me + TH * (k0 + u), G.n - 1));
+      g[u] = RowRaw<false>::load(L.gp, e);
+      b[u] = RowRaw<false>::load(L.bp, e);
+    }
+  };
+  load(x, r0);
+  if (U == NV) load_gb(0);
+  for (uint32_t r = r0; r < r1; r += step) {
+    if (r + step < r1) load(xn, r + step);
+    float s = 0.0f, s2 = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const v4f v = R::value(x[k], bf);
+      const uint32_t q = me + TH * k;
+      s += q < G.n ? sum4(v, G.dup(q)) : 0.0f;
+      if (!L.two_pass) s2 += q < G.n ? sumsq4(v, G.dup(q)) : 0.0f;
+    }
+    const float mean = sum(s, red) * L.inv_n;
+    if (L.two_pass) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        const uint32_t q = me + TH * k;
+        s2 += q < G.n ? sumsq4(R::value(x[k], bf) - mean, G.dup(q)) : 0.0f;
+      }
+    }
+    const float m2 = sum(s2, red + kWaves) * L.inv_n;
+    const float rstd = rsqrtf((L.two_pass ? m2 : m2 - mean * mean) + L.eps), shift = -mean * rstd;
+    gbyte* row = L.d + uint64_t(L.row(r)) * G.seg * dsz;
+#pragma unroll
+    for (int k0 = 0; k0 < NV; k0 += U) {
+      if (U < NV) load_gb(k0);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t q = me + TH * (k0 + u);
+        if (q < G.n) row_store(row, L.dt, G.at(q), L.out(R::value(x[k0 + u], bf), rstd, shift, g[u], b[u]));
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NV; ++k) x[k] = xn[k];
+  }
+}
+
+// Rows too long for the registers: the sums, (two-pass) the centred squares and the
+// results each read the row, after the first time from L2 and the memory-side cache.
+template <bool IN16>
+VM_DEV void ln_rows_long(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
+  typedef RowRaw<IN16> R;
+  const VM_K Task& t = task_of(A, ti);
+  const LnTask L(A, t);
+  float* red = lds_f32();
+  const RowGroups G(t.p[1]);
+  const bool bf = L.adt == DT_BF16;
+  constexpr int U = 8;
+  for (uint32_t r = r0; r < r1; ++r) {
+    const gbyte* src = L.a + uint64_t(L.row(r)) * G.seg * (IN16 ? 2 : 4);
+    gbyte* row = L.d + uint64_t(L.row(r)) * G.seg * (L.dt == DT_F32 ? 4 : 2);
+    auto each = [&](auto fn) {
+      for (uint32_t q0 = threadIdx.x; q0 < G.n; q0 += U * kBlock) {
+        typename R::Raw x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = R::load(src, G.at(min(q0 + u * kBlock, G.n - 1)));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (q0 + u * kBlock < G.n) fn(q0 + u * kBlock, R::value(x[u], bf));
+      }
+    };
+    float s = 0.0f, s2 = 0.0f;
+    each([&](uint32_t q, v4f v) {
+      s += sum4(v, G.dup(q));
+      if (!L.two_pass) s2 += sumsq4(v, G.dup(q));
+    });
+    const float mean = block_reduce(s, OpSum(), red) * L.inv_n;
+    if (L.two_pass) each([&](uint32_t q, v4f v) { s2 += sumsq4(v - mean, G.dup(q)); });
+    const float m2 = block_reduce(s2, OpSum(), red + kWaves) * L.inv_n;
+    const float rstd = rsqrtf((L.two_pass ? m2 : m2 - mean * mean) + L.eps), shift = -mean * rstd;
+    each([&](uint32_t q, v4f v) {
+      v4f g = v, b = v;
+      if (L.affine) {
+        g = RowRaw<false>::load(L.gp, G.at(q));
+        b = RowRaw<false>::load(L.bp, G.at(q));
+      }
+      row_store_own(row, L.dt, G.at(q), L.out(v, rstd, shift, g, b), G.dup(q));
+    });
+  }
+}
+
+template <bool IN16>
+VM_DEV void ln_dispatch(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  const uint32_t n = (task_of(A, ti).p[1] + 3) >> 2, wave = uni(threadIdx.x >> 6);
+  if (n <= 4 * 64) ln_rows<4, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (n <= 16 * 64) ln_rows<16, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (n <= 8 * kBlock) ln_rows<8, IN16, kBlock>(A, ti, lo, hi, 1);
+  else if (n <= 32 * kBlock) ln_rows<32, IN16, kBlock>(A, ti, lo, hi, 1);
+  else ln_rows_long<IN16>(A, ti, lo, hi);
+}
+
+// Rows of less than four elements: single elements from global memory.
+VM_DEV void ln_rows_generic(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
+  A = uargs(A);
+  const VM_K Task& t = task_of(A, ti);
+  float* red = lds_f32();
+  const uint32_t seg = t.p[1], flags = t.p[3];
+  const float eps = __uint_as_float(t.p[2]);
+  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
+  const gbyte* a = resolve(A, t.a);
+  gbyte* d = resolve(A, t.dst);
+  const bool affine = flags & LN_AFFINE, do_gelu = flags & LN_GELU, two_pass = flags & LN_TWO_PASS;
+  const gbyte* gp = resolve(A, affine ? t.b : t.a);
+  const gbyte* bp = resolve(A, affine ? t.p[4] : t.a);
+  const float inv_n = 1.0f / float(seg);
+  const uint32_t c = max(1u, t.p[5]), stride = t.p[0] / c;
+  for (uint32_t i = r0; i < r1; ++i) {
+    const uint64_t base = uint64_t((i % c) * stride + i / c) * seg;
+    float s = 0.0f, s2 = 0.0f;
+    for (uint32_t j = threadIdx.x; j < seg; j += kBlock) {
+      const float v = load_f(a, adt, base + j);
+      s += v;
+      s2 = fmaf(v, v, s2);
+    }
+    const float mean = block_reduce(s, OpSum(), red) * inv_n;
+    float var;
+    if (two_pass) {
+      float q = 0.0f;
+      for (uint32_t j = threadIdx.x; j < seg; j += kBlock) {
+        const float dv = load_f(a, adt, base + j) - mean;
+        q = fmaf(dv, dv, q);
+      }
+      var = block_reduce(q, OpSum(), red + kWaves) * inv_n;
+    } else {
+      var = block_reduce(s2, OpSum(), red + kWaves) * inv_n - mean * mean;
+    }
+    const float rstd = rsqrtf(var + eps);
+    const float shift = -mean * rstd;
+    for (uint32_t j = threadIdx.x; j < seg; j += kBlock) {
+      float z = fmaf(load_f(a, adt, base + j), rstd, shift);
+      if (affine) z = fmaf(z, load_f(gp, DT_F32, j), load_f(bp, DT_F32, j));
+      if (do_gelu) z = gelu(z);
+      store_f(d, dt, base + j, z);
+    }
+  }
+}
+
+// Rows of the streaming kernel: whole aligned groups, up to 4096 elements.
+VM_DEV bool row_vec_ok(uint32_t seg, const gbyte* a, const gbyte* d, uint32_t adt, uint32_t dt) {
+  const bool fmt = (adt == DT_F32 || adt == DT_BF16) && (dt == DT_F32 || dt == DT_BF16);
+  return fmt && (seg & 3) == 0 && seg <= 16 * 4 * 64 && ((uintptr_t(a) | uintptr_t(d)) & 15) == 0;
+}
+
+// LAYERNORM_SEG tiles [lo, hi).  Task p5 (scheduler, extension): the lanes'
+// rows interleaved -- logical row i is row (i % p5) * (n_out / p5) + i / p5, so
+// that at any moment the lanes stream neighbouring rows of the input (C2,
+// alternating runs on one MI355X: 38.7 against 39.6 us).  Every row kernel
+// applies it per row.
+// A leaf with its row kernels inlined, for the reason ew_tile gives: as a
+// function calling them it saved and reloaded 14 registers in scratch around
+// every entry (C2, alternating runs: 41.6-41.8 against 42.2 us).
+VM_LEAF void layernorm_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  A = uargs(A);
+  const VM_K Task& t = task_of(A, ti);
+  const uint32_t n_out = t.p[0], nv4 = t.p[1] >> 2;
+  const bool ib = ((t.tile_op >> 16) & 0xFF) == DT_BF16, ob = ((t.tile_op >> 8) & 0xFF) == DT_BF16;
+  hi = min(hi, n_out);
+  if (lo >= hi) return;
+#define VM_LN_FAST(NVV, FULLV)                                                               \
+  {                                                                                           \
+    if (ib) return ob ? ln_rows_fast<NVV, true, true, FULLV>(A, ti, lo, hi)                    \
+                      : ln_rows_fast<NVV, true, false, FULLV>(A, ti, lo, hi);                  \
+    return ob ? ln_rows_fast<NVV, false, true, FULLV>(A, ti, lo, hi)                           \
+              : ln_rows_fast<NVV, false, false, FULLV>(A, ti, lo, hi);                         \
+  }
+  if (nv4 == 4 * 64) VM_LN_FAST(4, true)
+  if (nv4 < 4 * 64) VM_LN_FAST(4, false)
+  if (nv4 == 16 * 64) VM_LN_FAST(16, true)
+  VM_LN_FAST(16, false)
+#undef VM_LN_FAST
+}
+
+// The other rows, in a leaf of their own: inlined into the streaming kernel's they
+// cost it 2 % (8192 x 4096: 41.4 against 40.6 us).
+VM_LEAF void layernorm_any(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  A = uargs(A);
+  const VM_K Task& t = task_of(A, ti);
+  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
+  hi = min(hi, t.p[0]);
+  if (lo >= hi) return;
+  const bool in16 = adt == DT_BF16 || adt == DT_F16;
+  const bool fmt = (in16 || adt == DT_F32) && (dt == DT_F32 || dt == DT_BF16 || dt == DT_F16);
+  if (t.p[1] < 4 || !fmt) return ln_rows_generic(A, ti, lo, hi);
+  if (in16) ln_dispatch<true>(A, ti, lo, hi);
+  else ln_dispatch<false>(A, ti, lo, hi);
+}
+
+VM_DEV void layernorm_run(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  const VM_K Task& t = task_of(A, ti);
+  bool ok = row_vec_ok(t.p[1], resolve(A, t.a), resolve(A, t.dst), (t.tile_op >> 16) & 0xFF, (t.tile_op >> 8) & 0xFF);
+  if (ok && (t.p[3] & LN_AFFINE)) ok = ((uintptr_t(resolve(A, t.b)) | uintptr_t(resolve(A, t.p[4]))) & 15) == 0;
+  if (ok) layernorm_tiles(A, ti, lo, hi);
+  else layernorm_any(A, ti, lo, hi);
+}
+
+// SOFTMAX_SEG rows: exp(x - max) / sum, f32 arithmetic.
+//
+// Loads are not predicated (ln_load's reason): groups past the row re-read its last.
+// Three forms, by how many registers a row takes:
+//   up to 4096 elements: a wave per row, four rows in flight per CU and the next
+//     ones prefetched, DPP reductions and no block barrier;
+//   up to 32768: a row over the block's registers, the next row prefetched;
+//   longer: two passes over the row, the first keeping a running maximum and sum
+//     per thread.
+// Memory bounds them (MI355X, whole launches): 512 x 32000 f32 257 -> 34.9 us (3.75
+// TB/s: two rows per CU, so the first row's load and the last one's store overlap
+// nothing), 8192 x 4096 65 -> 53 (5.06), 4096 x 1000 20 -> 10.6, 1000 x 777 14.4 -> 6.9;
+// before, odd and long rows were read three times in single elements and a row of
+// any length took the whole block and two block barriers.
 // Rows r0, r0 + step, ... < r1, a row over the TH threads (64: the wave; kBlock: the
 // block), this thread's groups t, t + TH, ...
 template <int NV, bool IN16, int TH>
@@ -1017,7 +986,8 @@ VM_DEV void softmax_rows_long(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
         const v4f v = R::value(x[u], bf);
         const uint32_t q = q0 + u * kBlock;
         if (q < G.n)
-          row_store(row, dt, G.at(q), v4f_make(__expf(v.x - M), __expf(v.y - M), __expf(v.z - M), __expf(v.w - M)) * inv);
+          row_store_own(row, dt, G.at(q),
+                        v4f_make(__expf(v.x - M), __expf(v.y - M), __expf(v.z - M), __expf(v.w - M)) * inv, G.dup(q));
       }
     }
   }

@@ -46,7 +46,7 @@ VM_DEV void exec_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
     case TOP_DYN_SCATTER: dyn_tiles(A, ti, lo, hi, true); break;
     case TOP_RED_SEG: red_seg_tiles(A, ti, lo, hi); break;
     case TOP_SOFTMAX_SEG: softmax_tiles(A, ti, lo, hi); break;
-    case TOP_LAYERNORM_SEG: layernorm_tiles(A, ti, lo, hi); break;
+    case TOP_LAYERNORM_SEG: layernorm_run(A, ti, lo, hi); break;
     case TOP_MAP_REGION: map_region_tiles(A, ti, lo, hi); break;
     case TOP_FLASH_ATTN: attn_tiles(A, ti, lo, hi); break;
     case TOP_RED_STRIDED: red_strided_tiles(A, ti, lo, hi); break;

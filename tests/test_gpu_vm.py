@@ -412,6 +412,44 @@ def test_fused_layernorm_affine_gelu(in_dt, out_dt):
     assert_rel(as_f32(got[0], odt), as_f32(want[0], odt), BF16_ULP if out_dt == "bf16" else 1e-5, 1e-5, "ln")
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("seg", [3, 4, 5, 255, 1023, 1025, 4095, 4097, 8192, 8193, 32767, 32769, 50257])
+def test_layernorm_row_forms(dt, seg):
+    """Each row form (elements, wave, block, passes in memory) at the edges of its
+    lengths and odd lengths, in one pass (core) and two (affine, GELU).  f32 sums of
+    at most 50 terms a thread and 8 tree steps: mean and variance within 60 * 2^-24 of
+    a row of unit spread, and results of |z| <= 7 within 4e-5 (one-pass:
+    the square of the mean, 1/16, adds less); a 16-bit result adds its rounding.
+    Tiny rows (seg < 8) may have a small variance, which scales the error."""
+    rng = np.random.default_rng(53)
+    rows = 9
+    a = (rng.standard_normal((rows, seg)) + 0.25).astype(np.float32)
+    if seg < 8:
+        a[:, :3] += np.arange(3, dtype=np.float32)
+    if dt == "bf16":
+        a = vmref.bf16_to_f32(vmref.f32_to_bf16(a))
+    elif dt == "f16":
+        a = a.astype(np.float16).astype(np.float32)
+    gamma = rng.uniform(0.5, 1.5, seg).astype(np.float32)
+    beta = (rng.standard_normal(seg) * 0.1).astype(np.float32)
+    g = G.Graph()
+    x = g.input(a.shape, dt)
+    ga, be = g.input((seg,)), g.input((seg,))
+    g.output(g.layernorm_core(x, 1e-5), g.layernorm(x, ga, be, 1e-5, gelu=True, out_dtype="f32"))
+    blob, _ = blob_for(g.build())
+    print(f"[gpu] case: layernorm {dt} {seg}", file=sys.stderr, flush=True)
+    got = run_gpu(blob, [a, gamma, beta])
+    x64 = a.astype(np.float64)
+    mu, var = x64.mean(1, keepdims=True), x64.var(1, keepdims=True)
+    core = (x64 - mu) / np.sqrt(var + 1e-5)
+    z = core * gamma + beta
+    gelu = 0.5 * z * (1 + np.tanh(0.7978845608 * (z + 0.044715 * z ** 3)))
+    scale = max(1.0, float((1.0 / var).max()))
+    ulp = {"f32": 0.0, "bf16": 2.0 ** -8, "f16": 2.0 ** -10}[dt]
+    assert_rel(as_f32(got[0], V.DT_BY_NAME[dt]), core, ulp, 4e-5 * scale, "core")
+    assert_rel(got[1], gelu, 1e-5, 4e-5 * scale, "affine + gelu")
+
+
 @pytest.mark.parametrize("d,in_dt", [(100, "f32"), (6000, "f32"), (768, "f16"), (768, "f32")])
 def test_layernorm_row_interleave(d, in_dt):
     """Rows a multiple of the lane count: the scheduler interleaves the lanes'
