@@ -25,6 +25,7 @@
 
 #include "../../include/vmrt.h"
 #include "launch_slots.h"
+#include "task_scratch.h"
 #include "vm_abi.h"
 #define VM_HD inline
 #include "vm_divu32.h"
@@ -889,31 +890,6 @@ void vmrt_unload(vmrt_program* p) {
   delete p;
 }
 
-// Scratch bytes a task needs (0: none): a split decode attention keeps one
-// partial (running max, sum, hd channels) per split and head, and one arrival
-// counter per head; a split column reduction 64 partials per split and block of
-// outputs, and one counter per block; a K-split matmul one f32 partial tile per split and output
-// tile, and one arrival counter per output tile.
-static uint64_t task_scratch_bytes(const Task& t, uint32_t mma_t) {
-  if ((t.tile_op & 0xFF) == TOP_MMA && (t.p[3] >> 28)) {
-    const uint32_t code = (t.p[3] >> 24) & 0xF;
-    const uint64_t T = code == 1 ? 64 : code == 2 ? 128 : code == 3 ? 256 : mma_t;
-    const uint64_t tiles = ((t.p[0] + T - 1) / T) * ((t.p[1] + T - 1) / T) * std::max<uint64_t>(1, t.p[3] & 0xFFFFFF);
-    // a 256-wide tile runs as four 128-wide ones, each with a counter of its own
-    return (tiles * (uint64_t(1) << (t.p[3] >> 28)) * T * T + tiles * (T == 256 ? 4 : 1)) * 4;
-  }
-  if ((t.tile_op & 0xFF) == TOP_RED_STRIDED && t.p[4] > 1) {
-    const uint64_t blocks = (uint64_t(t.p[0]) + 63) / 64;
-    return (blocks * t.p[4] * 64 + blocks) * 4;
-  }
-  if ((t.tile_op & 0xFF) == TOP_ARGMAX_SEG && t.p[3] > 1) return (2ull * t.p[0] * t.p[3] + t.p[0]) * 4;
-  if ((t.tile_op & 0xFF) == TOP_DECODE_ATTN && (t.p[4] >> 16) > 1) {
-    const uint64_t H = t.p[4] & 0xFFFF, S = t.p[4] >> 16, hd = t.p[5] & 0xFFFF;
-    return (H * S * (hd + 2) + H) * 4;
-  }
-  return 0;
-}
-
 // The device copy of the lane table carries, in each span's pad word, the
 // task of the lane's first entry (0xFFFFFFFF when it is a control entry or the
 // lane has none): the kernel then requests that entry and its task record
@@ -1054,12 +1030,7 @@ static MmaRec mma_record(const Program& P, const Task& t, uint32_t mma_t) {
   };
   operand(&r.a, t.p[4], true);
   operand(&r.b, t.p[5], false);
-  // The split that does the work: the others' share of the K loop (0.022 us per f32 k of
-  // a 64-wide tile, 0.007 in 16 bits, three times that 128-wide) has to be worth
-  // publishing the partials and combining them, about 8 us (measured: 1.5 us to
-  // publish, 2 for the arrival, 4.4 to read the partials).
-  const double per_k = (h16 ? 0.007 : 0.022) * (r.T == 128 ? 3 : 1);
-  r.S = S > 1 && r.K * (1.0 - 1.0 / S) * per_k < 8.0 ? 1 : S;
+  r.S = mma_effective_split(S, r.K, r.T, r.adt);
   const uint32_t bk = h16 ? 32 : 16;
   r.ksh = ((r.K + r.S - 1) / r.S + bk - 1) / bk * bk;
   r.subs = 1;

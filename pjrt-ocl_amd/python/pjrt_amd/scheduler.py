@@ -569,10 +569,13 @@ def mma_split_log2(M: int, N: int, K: int, G: int, edge: int, adt: int, cfg: Dev
     With more tiles than that, a long K is still split 2 or 4 ways where the last
     round is nearly empty (288 tiles on 256 lanes) and the rounds saved are worth
     the combine: a tile costs about 1.3 us plus its K loop (64-wide: 7.4 us per
-    1024 k in 16 bits, 23 in f32; 128-wide: three times that), a split 3 us more."""
+    1024 k in 16 bits, 23 in f32; 128-wide: three times that), a split 3 us more.
+    Such splits (not those of half-idle lanes, whose partials are at most a tile per
+    lane) share a program's ``SPLIT_SCRATCH``; ``over_split_scratch`` takes those
+    past it back."""
     if not cfg.mma_splitk:
         return 0
-    tiles = math.ceil(M / edge) * math.ceil(N / edge) * max(1, G)
+    tiles = _mma_tiles(M, N, G, edge)
     slab = 16 if adt == V.DT_F32 else 32
     if K < 4 * slab or edge == 256:
         return 0
@@ -582,12 +585,75 @@ def mma_split_log2(M: int, N: int, K: int, G: int, edge: int, adt: int, cfg: Dev
         def cost(lg):
             return math.ceil((tiles << lg) / cfg.nlanes) * (1.3 + (3.0 if lg else 0.0) + per_k * K / (1 << lg))
         best = min((0, 1, 2), key=cost)
+        if mma_effective_split(1 << best, K, edge, adt) == 1:
+            return 0
         return best if cost(best) <= 0.85 * cost(0) else 0
     lg = 0
     while (lg < V.MMA_MAX_SPLIT_LOG2 and tiles << (lg + 1) <= cfg.nlanes
            and math.ceil(K / (1 << (lg + 1))) >= 2 * slab):
         lg += 1
     return lg
+
+
+def _mma_tiles(M: int, N: int, G: int, edge: int) -> int:
+    return math.ceil(M / edge) * math.ceil(N / edge) * max(1, G)
+
+
+def mma_effective_split(S: int, K: int, edge: int, adt: int) -> int:
+    """The splits of a matmul that the loader lets do the work (task_scratch.h, the
+    same rule): all of them, or one where the K loop that they shorten is worth less
+    than publishing and combining the partials, 8 us."""
+    per_k = (0.007 if adt in (V.DT_BF16, V.DT_F16) else 0.022) * (3 if edge == 128 else 1)
+    return 1 if S > 1 and K * (1.0 - 1.0 / S) * per_k < 8.0 else S
+
+
+# Scratch bytes of a program's optional splits: the matmuls split to fill a last
+# round and the column reductions.  Every task keeps its own region for the life of
+# the program (tasks of one phase run at once) and the loader refuses more than 4
+# GiB of them in all, which 64 such products of 1500 x 2048 x 5632 f32 alone would
+# need; past this the products run unsplit.
+SPLIT_SCRATCH = 1 << 30
+
+
+def split_scratch_bytes(task: V.Task, cfg: DeviceConfig) -> int:
+    """Scratch of a split matmul or column reduction (task_scratch.h)."""
+    if task.tile_op == V.TOP_RED_STRIDED and task.p4 > 1:
+        blocks = math.ceil(task.p0 / 64)
+        return (blocks * task.p4 * 64 + blocks) * 4
+    if task.tile_op != V.TOP_MMA:
+        return 0
+    T = mma_tile_edge(task, cfg)
+    S = mma_effective_split(1 << (task.p3 >> V.MMA_SPLIT_SHIFT), task.p2, T, task.adtype)
+    if S == 1:
+        return 0
+    tiles = _mma_tiles(task.p0, task.p1, task.p3 & 0xFFFFFF, T)
+    return (tiles * S * T * T + tiles * (4 if T == 256 else 1)) * 4
+
+
+def over_split_scratch(prog: V.VMProgram, cfg: DeviceConfig) -> set:
+    """Instructions whose optional split is left out: in program order, those whose
+    scratch would take the program's split matmuls and column reductions past
+    ``SPLIT_SCRATCH``.  What the other matmuls' splits need comes first, so a
+    program's scratch passes that bound only by theirs."""
+    need, optional = 0, []
+    for i, ins in enumerate(prog.instrs):
+        if ins.op not in (V.OP_DOT, V.OP_REDUCE_STRIDED):
+            continue
+        t = instr_to_task(ins, prog, cfg)
+        nb = (split_scratch_bytes(t, cfg) + 255) & ~255         # as the loader lays them out
+        if not nb:
+            continue
+        if t.tile_op == V.TOP_MMA and 2 * _mma_tiles(t.p0, t.p1, t.p3 & 0xFFFFFF, mma_tile_edge(t, cfg)) <= cfg.nlanes:
+            need += nb
+        else:
+            optional.append((i, nb))
+    out = set()
+    for i, nb in optional:
+        if need + nb > SPLIT_SCRATCH:
+            out.add(i)
+        else:
+            need += nb
+    return out
 
 
 def _region_inputs_from_aux(ins: V.Instr, prog: V.VMProgram) -> list:
@@ -982,6 +1048,7 @@ class _Scheduler:
         self.weight = 1.0
         self.est = 0.0
         self.n_flags = 0          # completion flags handed out (``emit_flagged``)
+        self.unsplit = over_split_scratch(prog, cfg)
 
     def task_id(self, i: int) -> int:
         tid = self.task_of.get(i)
@@ -989,6 +1056,11 @@ class _Scheduler:
             tid = len(self.tasks)
             self.task_of[i] = tid
             t = instr_to_task(self.prog.instrs[i], self.prog, self.cfg)
+            if i in self.unsplit:
+                if t.tile_op == V.TOP_MMA:
+                    t.p3 &= (1 << V.MMA_SPLIT_SHIFT) - 1
+                else:
+                    t.p4 = 1
             self.tasks.append(t)
             if i in self.ln_pro:
                 # the layernorm's task is a descriptor only: no lane runs it

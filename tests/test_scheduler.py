@@ -257,6 +257,79 @@ def test_mma_split_k_tiles_exact(dt, Gb, M, K, N):
     np.testing.assert_array_equal(got, want.astype(np.float32))
 
 
+SCRATCH_HARNESS = r"""
+#include "task_scratch.h"
+#include <cstdio>
+int main() {
+  vm::Task t;
+  unsigned mma_t;
+  while (std::scanf("%u %u %u %u %u %u %u %u %u %u", &mma_t, &t.tile_op, &t.p[0], &t.p[1], &t.p[2], &t.p[3], &t.p[4],
+                    &t.p[5], &t.p[6], &t.p[7]) == 10)
+    std::printf("%llu\n", (unsigned long long)vm::task_scratch_bytes(t, mma_t));
+}
+"""
+
+
+def loader_scratch(tmp_path, tasks, cfg):
+    """What the loader's own header (task_scratch.h, compiled with g++) gives each task."""
+    import os
+    import shutil
+    import subprocess
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not found")
+    csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "pjrt-ocl_amd", "csrc")
+    src, exe = tmp_path / "scratch.cpp", tmp_path / "scratch"
+    if not exe.exists():
+        src.write_text(SCRATCH_HARNESS)
+        subprocess.run([gxx, "-O1", "-std=c++17", f"-I{csrc}", "-o", str(exe), str(src)], check=True)
+    lines = [" ".join(str(x) for x in (cfg.mma_t, t.tile_op | t.dtype << 8 | t.adtype << 16, *t.params)) for t in tasks]
+    out = subprocess.run([str(exe)], input="\n".join(lines), capture_output=True, text=True, check=True).stdout.split()
+    assert len(out) == len(tasks)
+    return [int(x) for x in out]
+
+
+def test_split_scratch_is_the_loaders(tmp_path):
+    """The scheduler's scratch sizes and effective splits are the loader's, over
+    tile edges, types, splits and both sides of each threshold in K."""
+    cfg = S.DeviceConfig(nlanes=256)
+    tasks = []
+    for edge in (0, 64, 128, 256):
+        for adt in (V.DT_F32, V.DT_BF16, V.DT_F16):
+            for lg in range(V.MMA_MAX_SPLIT_LOG2 + 1):
+                for K in (64, 121, 122, 243, 244, 380, 381, 727, 728, 762, 763, 1142, 1143, 1180, 1524, 2285, 2286, 4096):
+                    tasks.append(V.Task(V.TOP_MMA, p0=300, p1=131, p2=K, adtype=adt, p3=3 | V.MMA_TILE_CODES[edge] << 24
+                                        | lg << V.MMA_SPLIT_SHIFT))
+    tasks += [V.Task(V.TOP_RED_STRIDED, p0=n, p1=4096, p2=n, p4=s) for n in (1, 64, 65, 2048) for s in (0, 1, 2, 64)]
+    want = loader_scratch(tmp_path, tasks, cfg)
+    assert [S.split_scratch_bytes(t, cfg) for t in tasks] == want
+    assert 0 < sum(1 for w in want if w) < len(want)
+
+
+@pytest.mark.parametrize("depth,first,last", [(3, True, True), (64, True, False)])
+def test_deep_stack_of_split_products_fits_the_scratch(tmp_path, depth, first, last):
+    """Products of 1500 x 2048 x 5632 and back in f32 fill their last round by a K
+    split of 34-138 MB of partials each.  A few of them get it; a stack whose splits
+    would pass the loader's 4 GiB keeps what fits ``SPLIT_SCRATCH`` and loads."""
+    g = G.Graph()
+    x = g.input((1500, 2048))
+    w, u = g.input((2048, 5632)), g.input((5632, 2048))
+    for k in range(depth):
+        x = g.dot(x, u if k % 2 else w)
+    g.output(x)
+    prog = g.build()
+    cfg = S.DeviceConfig(nlanes=256)
+    tasks = S.schedule_program(prog, cfg).tasks
+    split = [t.p3 >> V.MMA_SPLIT_SHIFT for t in tasks]
+    assert len(tasks) == depth and (split[0] > 0, split[-1] > 0) == (first, last), split
+    assert sum(-(-b // 256) * 256 for b in loader_scratch(tmp_path, tasks, cfg)) <= S.SPLIT_SCRATCH
+    # splits that half-idle lanes take are not held back, and are counted first
+    g = G.Graph()
+    g.output(*(g.dot(g.input((256, 2048)), g.input((2048, 512))) for _ in range(300)))
+    small = S.schedule_program(g.build(), cfg).tasks
+    assert all(t.p3 >> V.MMA_SPLIT_SHIFT for t in small)
+
+
 # --- skinny matmuls as split-K TOP_GEMV tasks ----------------------------------------
 
 @pytest.mark.parametrize("dt", ["f32", "bf16"])
