@@ -275,7 +275,7 @@ VM_DEV void gemv_tile(Args A, uint32_t ti, uint32_t tile) {
   const gbyte* b = resolve(A, t.b) + uint64_t(g) * K * N * esz;
   const uint32_t cgs = CW / 8, RP = kBlock / cgs;
   // LDS: x [M][K], then the row partials [P][M][CW] (at most 2048 M floats), then
-  // the layernorm's sums; the loader checks that M * K + 4096 M floats fit
+  // the layernorm's sums (3 kWaves); the loader checks that M K + 2048 M + 64 floats fit
   float* xs = lds_ptr<float>();
   float* red = xs + ((M * K + 3) & ~3u);
   float* st = red + 2048 * M;

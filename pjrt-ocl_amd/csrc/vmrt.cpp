@@ -603,7 +603,8 @@ struct Checker {
         if (dt != DT_F32 && dt != DT_BF16 && dt != DT_F16) return fail(ti, "gemv result dtype");
         if (M < 1 || M > kGemvMaxM || N < 8 || N % 8 || K < 1 || CW < 8 || CW > 256 || (CW & (CW - 1)))
           return fail(ti, "gemv shape / strip width");
-        if ((((M * K + 3) & ~uint64_t(3)) + 4096 * M) * 4 > uint64_t(lds_bytes))
+        // x rows, row partials, the layernorm's sums (tile_gemv.h gemv_tile)
+        if ((((M * K + 3) & ~uint64_t(3)) + 2048 * M + 64) * 4 > uint64_t(lds_bytes))
           return fail(ti, "gemv x row does not fit the LDS");
         if (!has(t.a, G * M * K, adt) || !has(t.b, G * K * N, adt)) return fail(ti, "gemv operands");
         if (!has(t.dst, G * M * N, dt)) return fail(ti, "gemv result");

@@ -210,7 +210,7 @@ def attn_rows_padded(T: int) -> int:
 # --- skinny matmuls (TOP_GEMV) ------------------------------------------------------
 
 GEMV_MAX_M = 8
-GEMV_LDS_FLOATS = 147456 // 4   # the kernel's LDS: x rows + row-phase sums
+GEMV_LDS_FLOATS = 133120 // 4   # the kernel's LDS (vm_kernel_smem_bytes)
 _EPI_INLINE = {V.SUB_AFFINE, V.SUB_GELU, V.SUB_COPY, V.SUB_ADD, V.SUB_MUL, V.SUB_SUB, V.SUB_DIV,
                V.SUB_MAX, V.SUB_MIN}
 
@@ -251,7 +251,9 @@ def gemv_strip(N: int, G: int, nlanes: int, min_strip: int = 8) -> int:
 def gemv_eligible(M, N, K, G, aview, bview, epi, adt, dt, prog) -> bool:
     if not (1 <= M <= GEMV_MAX_M and N % 8 == 0 and N >= 8 and K >= 1) or aview or bview:
         return False
-    if (M * K + 3) // 4 * 4 + 4096 * M > GEMV_LDS_FLOATS:
+    # x rows, row partials and a layernorm's sums fit the kernel's LDS, as the loader
+    # checks; of several rows only short ones (8 of 512, 4 of 5120)
+    if (M * K + 3) // 4 * 4 + 2048 * M + 64 > GEMV_LDS_FLOATS or M * K + 4096 * M > 36864:
         return False
     if adt not in (V.DT_BF16, V.DT_F16, V.DT_F32) or dt not in (V.DT_F32, V.DT_BF16, V.DT_F16):
         return False

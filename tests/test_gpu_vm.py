@@ -856,6 +856,24 @@ def test_gemv_split_k_exact(dt, Gb, M, K, N):
         lp.close()
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("M,K", [(1, 31168), (2, 14336), (4, 5120), (7, 1170), (8, 66), (8, 512)])
+def test_gemv_longest_rows_load_and_are_exact(dt, M, K):
+    """Rows that fill the LDS bound, and eight short ones (8 x 66 and up were
+    scheduled as GEMV and then refused by the loader).  Integer-valued operands whose
+    sums stay below 2^24 give the exact result."""
+    rng = np.random.default_rng(82)
+    a = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    b = rng.integers(-3, 4, (K, 136)).astype(np.float32)
+    g = G.Graph()
+    x, y = g.input(a.shape, dt), g.input(b.shape, dt)
+    g.output(g.dot(x, y))
+    blob, _ = blob_for(g.build())
+    assert vmref.parse(blob).tasks[0].top == V.TOP_GEMV
+    print(f"[gpu] case: gemv rows {dt} {M} x {K}", file=sys.stderr, flush=True)
+    np.testing.assert_array_equal(run_gpu(blob, [a, b])[0], a.astype(np.float64) @ b.astype(np.float64))
+
+
 def test_gemv_epilogue_bf16_out():
     rng = np.random.default_rng(75)
     M, K, N = 1, 768, 3072

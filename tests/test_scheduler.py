@@ -355,6 +355,21 @@ def test_gemv_split_k_tiles_exact(dt, Gb, M, K, N):
     np.testing.assert_array_equal(got, np.matmul(a.astype(np.float64), b.astype(np.float64)))
 
 
+def test_gemv_bound_is_the_kernels_lds():
+    """A product is a GEMV only where its x rows, row partials and sums fit the LDS
+    that the kernel declares, which is what the loader checks."""
+    from pjrt_amd import runtime
+    assert S.GEMV_LDS_FLOATS * 4 == runtime.load_library().vm_kernel_smem_bytes()
+    cfg = S.DeviceConfig(nlanes=256)
+    most = {1: 31168, 2: 14336, 3: 8192, 4: 5120, 5: 3276, 6: 2048, 7: 1170, 8: 512}
+    for M, top in most.items():
+        assert (M * top + 3) // 4 * 4 + 2048 * M + 64 <= S.GEMV_LDS_FLOATS
+        for K, op in ((top, V.TOP_GEMV), (top + 1, V.TOP_MMA)):
+            g = G.Graph()
+            g.output(g.dot(g.input((M, K), "bf16"), g.input((K, 64), "bf16")))
+            assert S.schedule_program(g.build(), cfg).tasks[0].tile_op == op, (M, K)
+
+
 def test_gemv_epilogue_matches_tensor_semantics():
     from oracle import vmref
     rng = np.random.default_rng(8)
