@@ -260,6 +260,62 @@ VM_DEV float red_cols_block(Op op, float ident, const gbyte* a, uint32_t adt, ui
   return r;                                              // threads 0..63: output q0 + threadIdx.x
 }
 
+// Outputs [q0, q1) over a short axis: one (VEC: four) per thread, eight loads in
+// flight, no LDS.  A block of 64 outputs costs a round trip, an LDS pass and two
+// barriers however few rows it has; here 1024 (256) outputs share a round trip per
+// eight rows, single elements of two or four rows those of J groups of 256 outputs.
+// Taken where a lane's blocks take no more round trips so (red_cols_tiles).  Whole
+// launches on MI355X, us (blocks of 64 / one output per thread and one load at a time
+// / this): 1M outputs f32 over 2 rows 75.6 / 14.9 / 7.3, 8 rows 77.3 / 48.3 / 11.3, 32
+// rows 78.9 / 176 / 27.5, bf16 8 rows 111 / 43.5 / 12.0; 1000003 outputs over 2 rows 92 /
+// 14.9 / 11.3, 8 rows 91 / 48.9 / 28; 512 x 8 x 4096 f32 over the 8 150 / 97 / 21.
+template <class Op, bool VEC, uint32_t J>
+VM_DEV void red_cols_short(Op op, float ident, const gbyte* a, uint32_t adt, gbyte* d, uint32_t dt, uint32_t q0,
+                           uint32_t q1, uint32_t red, uint32_t inner) {
+  constexpr uint32_t W = VEC ? 4 : 1, R = kRedBatch / J;
+  for (uint32_t qb = q0 + W * threadIdx.x; qb < q1; qb += W * J * kBlock) {
+    uint64_t base[J];
+    float acc[J][W];
+#pragma unroll
+    for (uint32_t j = 0; j < J; ++j) {
+      const uint32_t q = J == 1 ? qb : min(qb + W * j * kBlock, q1 - W), o = q / inner;    // past q1: read again, not stored
+      base[j] = uint64_t(o) * red * inner + (q - o * inner);
+#pragma unroll
+      for (uint32_t w = 0; w < W; ++w) acc[j][w] = ident;
+    }
+    for (uint32_t rb = 0; rb < red; rb += R) {
+      float x[R][J][W];
+#pragma unroll
+      for (uint32_t u = 0; u < R; ++u) {
+        if (rb + u >= red) break;
+#pragma unroll
+        for (uint32_t j = 0; j < J; ++j) {
+          const uint64_t e = base[j] + uint64_t(rb + u) * inner;
+          if constexpr (VEC) {
+            const v4f v = ld4(a, adt, e);
+            x[u][j][0] = v.x; x[u][j][1] = v.y; x[u][j][2] = v.z; x[u][j][3] = v.w;
+          } else {
+            x[u][j][0] = load_f(a, adt, e);
+          }
+        }
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < R; ++u) {
+        if (rb + u >= red) break;
+#pragma unroll
+        for (uint32_t j = 0; j < J; ++j)
+#pragma unroll
+          for (uint32_t w = 0; w < W; ++w) acc[j][w] = op(acc[j][w], x[u][j][w]);
+      }
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < J; ++j)
+#pragma unroll
+      for (uint32_t w = 0; w < W; ++w)
+        if (J == 1 || qb + W * j * kBlock + w < q1) store_f(d, dt, qb + W * j * kBlock + w, acc[j][w]);
+  }
+}
+
 template <class Op>
 VM_DEV void red_cols_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi, Op op, float ident) {
   const VM_K Task& t = task_of(A, ti);
@@ -274,6 +330,17 @@ VM_DEV void red_cols_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi, Op op,
   }
   hi = min(hi, blocks * S);
   const bool vec = (adt == DT_F32 || adt == DT_BF16 || adt == DT_F16) && inner % 4 == 0 && (uintptr_t(a) & 15) == 0;
+  // 16 blocks (4: single elements) of a lane share red_cols_short's round trips, one
+  // per eight rows; the same form for every lane of the task
+  const uint32_t per = min(vec ? 16u : 4u, max(1u, blocks / A->n_lanes));
+  if (S == 1 && red <= kRedBatch * per) {
+    const uint32_t q0 = lo * kRedCols, q1 = min(hi * kRedCols, n_out);
+    if (vec) red_cols_short<Op, true, 1>(op, ident, a, adt, d, dt, q0, q1, red, inner);
+    else if (red <= 2) red_cols_short<Op, false, 4>(op, ident, a, adt, d, dt, q0, q1, red, inner);
+    else if (red <= 4) red_cols_short<Op, false, 2>(op, ident, a, adt, d, dt, q0, q1, red, inner);
+    else red_cols_short<Op, false, 1>(op, ident, a, adt, d, dt, q0, q1, red, inner);
+    return;
+  }
   const uint32_t share = (red + S - 1) / S;
   for (uint32_t tile = lo; tile < hi; ++tile) {
     const uint32_t blk = tile / S, split = tile % S, q0 = blk * kRedCols;

@@ -279,30 +279,62 @@ def test_float_reductions(kind):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("shape,axis", [((1000, 777), 0), ((4099, 68), 0), ((129, 2048), 0), ((5, 300, 36), 1),
+@pytest.mark.parametrize("shape,axis", [((1000, 777), 0), ((4099, 68), 0), ((16500, 100), 0), ((129, 2048), 0), ((5, 300, 36), 1),
                                         ((3, 7, 5), 1), ((2, 3), 0), ((1, 70), 0), ((700, 1), 0), ((33, 64, 4096), 1)])
 def test_column_reductions_exact(dt, shape, axis):
     """Reductions over an outer or middle axis: blocks of 64 outputs whose rows are
-    split over lanes (4099 rows: 64 splits of two blocks; 129: no split), in 16-byte
-    and single-element reads, ragged blocks, blocks over several outer indices and
-    outputs fewer than one read.  Small integers make the sum exact; max and min are
-    exact anyway.  Twice, so the second run finds the split counters reset."""
+    split over lanes (4099 rows: 32 splits of two blocks, 16500: 64, the most; 129: no
+    split), in 16-byte and single-element reads, ragged blocks, blocks over several
+    outer indices and outputs fewer than one read.  Small integers make the sum
+    exact; max and min are exact anyway.  One loaded program runs on three inputs, so
+    that counters which the run before left standing would leave its outputs."""
     rng = np.random.default_rng(24)
-    a = rng.integers(-2, 3, shape).astype(np.float32)
-    if dt != "f32":                       # sums within the 8 bits of a bf16 result
-        a = np.where(rng.random(shape) < 64 / max(64, 4 * shape[axis]), a, 0).astype(np.float32)   # (no -0)
     g = G.Graph()
     x = g.input(shape, dt)
     g.output(*(g.reduce_axis(x, axis, k) for k in (0, 1, 2)))
     blob, _ = blob_for(g.build())
+    splits = vmref.parse(blob).tasks[0].p[4]
+    assert splits == {(1000, 777): 4, (4099, 68): 32, (16500, 100): 64, (129, 2048): 1, (700, 1): 4}.get(shape, splits)
     print(f"[gpu] case: column reduction {dt} {shape} axis {axis}", file=sys.stderr, flush=True)
-    arg = a if dt == "f32" else a.astype(np.float16) if dt == "f16" else vmref.f32_to_bf16(a)
-    want = [a.sum(axis, dtype=np.float64), a.max(axis), a.min(axis)]
-    oracle = vmref.execute_schedule(blob, [arg], check_order=False)
-    for _ in range(2):
-        for gv, wv, ov in zip(run_gpu(blob, [arg]), want, oracle):
-            np.testing.assert_array_equal(as_f32(gv, V.DT_BY_NAME[dt]), wv)
-            np.testing.assert_array_equal(np.asarray(gv), np.asarray(ov).reshape(np.shape(gv)))
+    lp = runtime().load(blob)
+    try:
+        for run in range(3):
+            a = rng.integers(-2, 3, shape).astype(np.float32)
+            if dt != "f32":                       # sums within the 8 bits of a bf16 result
+                a = np.where(rng.random(shape) < 64 / max(64, 4 * shape[axis]), a, 0).astype(np.float32)   # (no -0)
+            arg = a if dt == "f32" else a.astype(np.float16) if dt == "f16" else vmref.f32_to_bf16(a)
+            want = [a.sum(axis, dtype=np.float64), a.max(axis), a.min(axis)]
+            for gv, wv in zip(lp(arg), want):
+                np.testing.assert_array_equal(as_f32(gv, V.DT_BY_NAME[dt]), wv, err_msg=f"run {run}")
+            if run == 0:
+                for wv, ov in zip(want, vmref.execute_schedule(blob, [arg], check_order=False)):
+                    np.testing.assert_array_equal(as_f32(np.asarray(ov), V.DT_BY_NAME[dt]).reshape(np.shape(wv)), wv)
+    finally:
+        lp.close()
+
+
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("shape,axis", [((1, 36), 0), ((2, 100), 0), ((8, 8197), 0), ((9, 32768), 0), ((9, 32767), 0),
+                                        ((17, 49152), 0), ((24, 49151), 0), ((32, 70001), 0), ((41, 70000), 0),
+                                        ((700, 5, 36), 1), ((2100, 2, 9), 1), ((2100, 4, 9), 1), ((900, 3, 68), 1),
+                                        ((3, 2, 4680), 1)])
+def test_short_column_reductions_exact(dt, shape, axis):
+    """Axes too short for blocks of 64 outputs, both sides of the line (8 rows per
+    block and lane: 32768 outputs of 256 lanes give two, 49152 three), whole and
+    ragged last groups, outputs over several outer indices, single elements one, two
+    and four outputs at a time.  Small integers make sum and product exact."""
+    rng = np.random.default_rng(25)
+    a = rng.integers(-2, 3, shape).astype(np.float32)
+    p = rng.choice(np.array([-1, 1, 1], np.float32), shape)
+    g = G.Graph()
+    x, y = g.input(shape, dt), g.input(shape, dt)
+    g.output(*(g.reduce_axis(x, axis, k) for k in (0, 1, 2)), g.reduce_axis(y, axis, 3))
+    blob, _ = blob_for(g.build())
+    print(f"[gpu] case: short column reduction {dt} {shape} axis {axis}", file=sys.stderr, flush=True)
+    enc = {"f32": lambda v: v, "f16": lambda v: v.astype(np.float16), "bf16": vmref.f32_to_bf16}[dt]
+    got = run_gpu(blob, [enc(a), enc(p)])
+    for gv, wv in zip(got, [a.sum(axis, dtype=np.float64), a.max(axis), a.min(axis), p.prod(axis, dtype=np.float64)]):
+        np.testing.assert_array_equal(as_f32(gv, V.DT_BY_NAME[dt]), wv)
 
 
 @pytest.mark.parametrize("dt", ["i32", "u32", "i64", "bool"])
