@@ -263,12 +263,21 @@ VM_DEV float red_cols_block(Op op, float ident, const gbyte* a, uint32_t adt, ui
 // Outputs [q0, q1) over a short axis: one (VEC: four) per thread, eight loads in
 // flight, no LDS.  A block of 64 outputs costs a round trip, an LDS pass and two
 // barriers however few rows it has; here 1024 (256) outputs share a round trip per
-// eight rows, single elements of two or four rows those of J groups of 256 outputs.
+// eight rows, single elements of up to four rows two for J = 4 groups of 256 outputs.
 // Taken where a lane's blocks take no more round trips so (red_cols_tiles).  Whole
 // launches on MI355X, us (blocks of 64 / one output per thread and one load at a time
-// / this): 1M outputs f32 over 2 rows 75.6 / 14.9 / 7.3, 8 rows 77.3 / 48.3 / 11.3, 32
-// rows 78.9 / 176 / 27.5, bf16 8 rows 111 / 43.5 / 12.0; 1000003 outputs over 2 rows 92 /
-// 14.9 / 11.3, 8 rows 91 / 48.9 / 28; 512 x 8 x 4096 f32 over the 8 150 / 97 / 21.
+// / this): 1M outputs f32 over 2 rows 75.6 / 14.9 / 7.2, 8 rows 77.3 / 48.3 / 10.6, 32
+// rows 78.9 / 176 / 25.5, bf16 8 rows 111 / 43.5 / 10.7; 1000003 outputs over 2 rows 92 /
+// 14.9 / 11.6, 8 rows 91 / 48.9 / 28; 512 x 8 x 4096 f32 over the 8 150 / 97 / 19.
+// The stores are one 16-byte one or a rolled loop: unrolled, with a form more, the
+// leaf was 129 KB, a short branch's reach (and 1M over 8 11.3, bf16 12.0).
+template <uint32_t J, uint32_t W>
+VM_DEV float pick(const float (&v)[J][W], uint32_t i) {      // v[i / W][i % W], from registers
+  float r = v[0][0];
+#pragma unroll
+  for (uint32_t k = 1; k < J * W; ++k) r = i == k ? v[k / W][k % W] : r;
+  return r;
+}
 template <class Op, bool VEC, uint32_t J>
 VM_DEV void red_cols_short(Op op, float ident, const gbyte* a, uint32_t adt, gbyte* d, uint32_t dt, uint32_t q0,
                            uint32_t q1, uint32_t red, uint32_t inner) {
@@ -308,11 +317,18 @@ VM_DEV void red_cols_short(Op op, float ident, const gbyte* a, uint32_t adt, gby
           for (uint32_t w = 0; w < W; ++w) acc[j][w] = op(acc[j][w], x[u][j][w]);
       }
     }
-#pragma unroll
-    for (uint32_t j = 0; j < J; ++j)
-#pragma unroll
-      for (uint32_t w = 0; w < W; ++w)
-        if (J == 1 || qb + W * j * kBlock + w < q1) store_f(d, dt, qb + W * j * kBlock + w, acc[j][w]);
+    if constexpr (VEC) {
+      if ((uintptr_t(d) & 15) == 0 && (dt == DT_F32 || dt == DT_BF16 || dt == DT_F16)) {
+        st4(d, dt, qb, v4f_make(acc[0][0], acc[0][1], acc[0][2], acc[0][3]));
+        continue;
+      }
+    }
+#pragma unroll 1
+    for (uint32_t j = 0; j < J * W; ++j) {
+      const float v = pick(acc, j);
+      const uint32_t q = VEC ? qb + j : qb + j * kBlock;
+      if (q < q1) store_f(d, dt, q, v);
+    }
   }
 }
 
@@ -336,8 +352,7 @@ VM_DEV void red_cols_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi, Op op,
   if (S == 1 && red <= kRedBatch * per) {
     const uint32_t q0 = lo * kRedCols, q1 = min(hi * kRedCols, n_out);
     if (vec) red_cols_short<Op, true, 1>(op, ident, a, adt, d, dt, q0, q1, red, inner);
-    else if (red <= 2) red_cols_short<Op, false, 4>(op, ident, a, adt, d, dt, q0, q1, red, inner);
-    else if (red <= 4) red_cols_short<Op, false, 2>(op, ident, a, adt, d, dt, q0, q1, red, inner);
+    else if (red <= 4) red_cols_short<Op, false, 4>(op, ident, a, adt, d, dt, q0, q1, red, inner);
     else red_cols_short<Op, false, 1>(op, ident, a, adt, d, dt, q0, q1, red, inner);
     return;
   }
