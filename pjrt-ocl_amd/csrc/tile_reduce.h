@@ -954,18 +954,17 @@ VM_DEV void layernorm_run(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
 
 // SOFTMAX_SEG rows: exp(x - max) / sum, f32 arithmetic.
 //
-// Loads are not predicated (ln_load's reason): groups past the row re-read its last.
-// Three forms, by how many registers a row takes:
+// Forms, by how many registers a row takes and how many rows a lane has:
 //   up to 4096 elements: a wave per row, four rows in flight per CU and the next
 //     ones prefetched, DPP reductions and no block barrier;
+//   up to 8192 and at most three rows a lane: softmax_rows_few;
 //   up to 32768: a row over the block's registers, the next row prefetched;
 //   longer: two passes over the row, the first keeping a running maximum and sum
 //     per thread.
-// Memory bounds them (MI355X, whole launches): 512 x 32000 f32 257 -> 34.9 us (3.75
-// TB/s: two rows per CU, so the first row's load and the last one's store overlap
-// nothing), 8192 x 4096 65 -> 53 (5.06), 4096 x 1000 20 -> 10.6, 1000 x 777 14.4 -> 6.9;
-// before, odd and long rows were read three times in single elements and a row of
-// any length took the whole block and two block barriers.
+// Loads are not predicated (ln_load's reason), except in softmax_rows_few: groups
+// past the row re-read its last.  Memory bounds them (MI355X, whole launches): 512 x
+// 32000 f32 33.5 us (3.9 TB/s: two rows per CU, so the first row's load and the last
+// one's store overlap nothing), 4096 x 4096 25.0 (5.4 TB/s), 4096 x 1001 8.9.
 // Rows r0, r0 + step, ... < r1, a row over the TH threads (64: the wave; kBlock: the
 // block), this thread's groups t, t + TH, ...
 template <int NV, bool IN16, int TH>
@@ -1018,6 +1017,56 @@ VM_DEV void softmax_rows(Args A, uint32_t ti, uint32_t r0, uint32_t r1, uint32_t
     }
 #pragma unroll
     for (int k = 0; k < NV; ++k) x[k] = xn[k];
+  }
+}
+
+// A lane's one to three rows, over the block's threads: one row's latency is what
+// counts, so groups past the row are skipped (clamped ones cost four exponentials
+// each), and a wave per row would leave waves idle.
+template <int NV, bool IN16>
+VM_DEV void softmax_rows_few(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
+  typedef RowRaw<IN16> R;
+  const VM_K Task& t = task_of(A, ti);
+  float* red = lds_f32();
+  const RowGroups G(t.p[1]);
+  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
+  const bool bf = adt == DT_BF16;
+  const gbyte* a = resolve(A, t.a);
+  gbyte* d = resolve(A, t.dst);
+  const uint32_t me = threadIdx.x, dsz = dt == DT_F32 ? 4 : 2;
+  typename R::Raw x[NV], xn[NV];
+  auto load = [&](typename R::Raw (&buf)[NV], uint32_t r) {
+    const gbyte* row = a + uint64_t(r) * G.seg * (IN16 ? 2 : 4);
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (me + kBlock * k < G.n) buf[k] = R::load(row, G.at(me + kBlock * k));
+  };
+  load(x, r0);
+  for (uint32_t r = r0; r < r1; ++r) {
+    if (r + 1 < r1) load(xn, r + 1);
+    v4f y[NV];
+    float m = -INFINITY, s = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (me + kBlock * k < G.n) {
+        y[k] = R::value(x[k], bf);
+        m = fmaxf(m, fmaxf(fmaxf(y[k].x, y[k].y), fmaxf(y[k].z, y[k].w)));
+      }
+    m = block_reduce(m, OpMax(), red);
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (me + kBlock * k < G.n) {
+        y[k] = v4f_make(__expf(y[k].x - m), __expf(y[k].y - m), __expf(y[k].z - m), __expf(y[k].w - m));
+        s += sum4(y[k], G.dup(me + kBlock * k));
+      }
+    const float inv = 1.0f / block_reduce(s, OpSum(), red + kWaves);
+    gbyte* row = d + uint64_t(r) * G.seg * dsz;
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (me + kBlock * k < G.n) row_store(row, dt, G.at(me + kBlock * k), y[k] * inv);
+    if (r + 1 < r1)
+#pragma unroll
+      for (int k = 0; k < NV; ++k) x[k] = xn[k];
   }
 }
 
@@ -1075,31 +1124,14 @@ VM_DEV void softmax_rows_long(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
   }
 }
 
-template <bool IN16>
-VM_DEV void softmax_dispatch(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
-  const uint32_t n = (task_of(A, ti).p[1] + 3) >> 2, wave = uni(threadIdx.x >> 6);
-  if (n <= 4 * 64) softmax_rows<4, IN16, 64>(A, ti, lo + wave, hi, kWaves);
-  else if (n <= 16 * 64) softmax_rows<16, IN16, 64>(A, ti, lo + wave, hi, kWaves);
-  else if (n <= 8 * kBlock) softmax_rows<8, IN16, kBlock>(A, ti, lo, hi, 1);
-  else if (n <= 32 * kBlock) softmax_rows<32, IN16, kBlock>(A, ti, lo, hi, 1);
-  else softmax_rows_long<IN16>(A, ti, lo, hi);
-}
-
-// A leaf with its row forms inlined, as layernorm_tiles.
-VM_LEAF void softmax_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
-  A = uargs(A);
+// Rows of less than four elements or other types: single elements from memory.
+VM_DEV void softmax_rows_generic(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   const VM_K Task& t = task_of(A, ti);
   float* red = lds_f32();
-  const uint32_t n_out = t.p[0], seg = t.p[1];
+  const uint32_t seg = t.p[1];
   const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
-  lo = uni(lo);
-  hi = uni(min(hi, n_out));
-  if (lo >= hi) return;
   const gbyte* a = resolve(A, t.a);
   gbyte* d = resolve(A, t.dst);
-  const bool out_ok = dt == DT_F32 || dt == DT_BF16 || dt == DT_F16;
-  if (out_ok && seg >= 4 && adt == DT_F32) return softmax_dispatch<false>(A, ti, lo, hi);
-  if (out_ok && seg >= 4 && (adt == DT_BF16 || adt == DT_F16)) return softmax_dispatch<true>(A, ti, lo, hi);
   for (uint32_t r = lo; r < hi; ++r) {
     const uint64_t base = uint64_t(r) * seg;
     float m = -INFINITY;
@@ -1111,6 +1143,81 @@ VM_LEAF void softmax_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
     const float inv = 1.0f / s;
     for (uint32_t j = threadIdx.x; j < seg; j += kBlock) store_f(d, dt, base + j, __expf(load_f(a, adt, base + j) - m) * inv);
   }
+}
+
+// The forms in three leaves, by the registers they need: with all of them in one (135
+// KB) the short ones paid for the long ones' registers and spills.  The whole-row and
+// few-row rules with it, MI355X, whole launches, us (one leaf, a wave per row up to
+// 4096 / a row per block / this): bf16 256 x 2304 9.2 / 5.6 / 5.2, 256 x 4096
+// 9.8 / 5.9 / 5.3, 500 x 1500 9.1 / 6.2 / 5.7, 256 x 6000 8.0 / 6.8 / 6.7; f32 256 x 1500
+// 7.5 / 5.2 / 5.3, 500 x 4096 8.9 / 7.7 / 7.5, 4096 x 48 7.5 / 14.8 / 5.5.  (Each form a
+// leaf, ten calls in the kernel: the same, but 25.4 against 24.8 for an MLP of two
+// products, whose code the calls push apart.  One function that calls them: 20-45 us
+// an entry, saving what they clobber.)
+enum SoftmaxForm : uint32_t {
+  SM_WAVE1, SM_WAVE4, SM_FEW2, SM_FEW4,           // softmax_short
+  SM_FEW8, SM_WAVE16, SM_BLOCK8,                  // softmax_mid
+  SM_BLOCK32, SM_LONG, SM_ELEM                    // softmax_long
+};
+// By the task's rows per lane, not the entry's: one form for all rows of a task.
+VM_DEV uint32_t softmax_form(Args A, const VM_K Task& t) {
+  const uint32_t n = (t.p[1] + 3) >> 2, rows = (t.p[0] - 1) / A->n_lanes + 1;
+  const uint32_t dt = (t.tile_op >> 8) & 0xFF, adt = (t.tile_op >> 16) & 0xFF;
+  const bool fmt = (dt == DT_F32 || dt == DT_BF16 || dt == DT_F16) && (adt == DT_F32 || adt == DT_BF16 || adt == DT_F16);
+  if (!fmt || t.p[1] < 4) return SM_ELEM;
+  if (n <= 64) return SM_WAVE1;
+  if (n <= 8 * kBlock && rows <= (n <= kBlock ? 2u : 3u)) return n <= 2 * kBlock ? SM_FEW2 : n <= 4 * kBlock ? SM_FEW4 : SM_FEW8;
+  return n <= 4 * 64 ? SM_WAVE4 : n <= 16 * 64 ? SM_WAVE16 : n <= 8 * kBlock ? SM_BLOCK8 : n <= 32 * kBlock ? SM_BLOCK32 : SM_LONG;
+}
+
+template <bool IN16>
+VM_DEV void softmax_short_rows(Args A, uint32_t ti, uint32_t lo, uint32_t hi, uint32_t form) {
+  const uint32_t wave = uni(threadIdx.x >> 6);
+  if (form == SM_WAVE1) softmax_rows<1, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (form == SM_WAVE4) softmax_rows<4, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (form == SM_FEW2) softmax_rows_few<2, IN16>(A, ti, lo, hi);
+  else softmax_rows_few<4, IN16>(A, ti, lo, hi);
+}
+template <bool IN16>
+VM_DEV void softmax_mid_rows(Args A, uint32_t ti, uint32_t lo, uint32_t hi, uint32_t form) {
+  const uint32_t wave = uni(threadIdx.x >> 6);
+  if (form == SM_FEW8) softmax_rows_few<8, IN16>(A, ti, lo, hi);
+  else if (form == SM_WAVE16) softmax_rows<16, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else softmax_rows<8, IN16, kBlock>(A, ti, lo, hi, 1);
+}
+template <bool IN16>
+VM_DEV void softmax_long_rows(Args A, uint32_t ti, uint32_t lo, uint32_t hi, uint32_t form) {
+  if (form == SM_BLOCK32) softmax_rows<32, IN16, kBlock>(A, ti, lo, hi, 1);
+  else softmax_rows_long<IN16>(A, ti, lo, hi);
+}
+VM_LEAF void softmax_short(Args A, uint32_t ti, uint32_t lo, uint32_t hi, uint32_t form) {
+  A = uargs(A);
+  const bool f32 = ((task_of(A, uni(ti)).tile_op >> 16) & 0xFF) == DT_F32;
+  if (f32) softmax_short_rows<false>(A, uni(ti), uni(lo), uni(hi), uni(form));
+  else softmax_short_rows<true>(A, uni(ti), uni(lo), uni(hi), uni(form));
+}
+VM_LEAF void softmax_mid(Args A, uint32_t ti, uint32_t lo, uint32_t hi, uint32_t form) {
+  A = uargs(A);
+  const bool f32 = ((task_of(A, uni(ti)).tile_op >> 16) & 0xFF) == DT_F32;
+  if (f32) softmax_mid_rows<false>(A, uni(ti), uni(lo), uni(hi), uni(form));
+  else softmax_mid_rows<true>(A, uni(ti), uni(lo), uni(hi), uni(form));
+}
+VM_LEAF void softmax_long(Args A, uint32_t ti, uint32_t lo, uint32_t hi, uint32_t form) {
+  A = uargs(A);
+  const bool f32 = ((task_of(A, uni(ti)).tile_op >> 16) & 0xFF) == DT_F32;
+  if (uni(form) == SM_ELEM) softmax_rows_generic(A, uni(ti), uni(lo), uni(hi));
+  else if (f32) softmax_long_rows<false>(A, uni(ti), uni(lo), uni(hi), uni(form));
+  else softmax_long_rows<true>(A, uni(ti), uni(lo), uni(hi), uni(form));
+}
+
+VM_DEV void softmax_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
+  const VM_K Task& t = task_of(A, ti);
+  hi = min(hi, t.p[0]);
+  if (lo >= hi) return;
+  const uint32_t form = softmax_form(A, t);
+  if (form <= SM_FEW4) softmax_short(A, ti, lo, hi, form);
+  else if (form <= SM_BLOCK8) softmax_mid(A, ti, lo, hi, form);
+  else softmax_long(A, ti, lo, hi, form);
 }
 
 // ARGMAX_SEG: dst = first index of the row maximum (a NaN wins: its first index),

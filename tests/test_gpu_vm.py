@@ -394,10 +394,11 @@ def test_softmax_and_layernorm_rows(seg):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("seg", [3, 4, 5, 255, 1023, 1025, 4095, 4097, 8191, 8193, 32766, 32769, 50257])
-def test_softmax_row_forms(dt, seg):
-    """Each row form (wave, block, two passes in memory) at the edges of its
-    lengths, odd lengths (the last group of four overlaps the one before), rows
+@pytest.mark.parametrize("nlanes", [None, 2])
+@pytest.mark.parametrize("seg", [3, 4, 5, 255, 257, 1023, 1025, 2047, 2049, 4095, 4097, 8191, 8193, 32766, 32769, 50257])
+def test_softmax_row_forms(dt, seg, nlanes):
+    """Each row form (wave, block, two passes in memory; nine rows on two lanes, and on
+    all of them the forms for a few rows) at the edges of its lengths, odd lengths (the last group of four overlaps the one before), rows
     with -inf entries (one thread's share all -inf among them), a row of -inf
     only (NaN) and a +inf (NaN in that row).  f32 arithmetic: each exponential is
     within 2 ulp plus its argument's rounding (|x - max| <= 40: 40 * 2^-24), the sum's
@@ -416,8 +417,8 @@ def test_softmax_row_forms(dt, seg):
     g = G.Graph()
     x = g.input(a.shape, dt)
     g.output(g.softmax_last(x), g.softmax_last(x, out_dtype="f32"))
-    blob, _ = blob_for(g.build())
-    print(f"[gpu] case: softmax {dt} {seg}", file=sys.stderr, flush=True)
+    blob, _ = blob_for(g.build(), nlanes=nlanes)
+    print(f"[gpu] case: softmax {dt} {seg} lanes {nlanes}", file=sys.stderr, flush=True)
     got = run_gpu(blob, [a])
     with np.errstate(invalid="ignore"):
         e = np.exp(a.astype(np.float64) - a.max(1, keepdims=True))
