@@ -693,10 +693,17 @@ VM_DEV void row_store_own(gbyte* row, uint32_t dt, uint32_t e, v4f v, uint32_t d
 // gamma and beta stay in registers, for rows over 8192 elements they come from L2
 // for every row.  Measured (MI355X, whole launches, us; before: f16 rows through
 // scalar conversions and odd or long rows three times in single elements):
-//   GELU, f32 -> bf16: 1000 x 777 17.5 -> 7.4, 3000 x 4097 187 -> 37, 2048 x 8192 44.7
-//   -> 36, 100 x 30000 96.5 -> 30, 64 x 50257 158 -> 41; f16 4096 x 4096 170 -> 36,
-//   4096 x 1024 50 -> 13.4.  A row or two per lane lose a little to the groups'
-//   masks (300 x 5000 10.4 -> 11.2; f16 2000 x 768 8.7 -> 9.1).
+//   GELU, f32 -> bf16: 1000 x 777 17.5 -> 7.5, 3000 x 4097 186 -> 33, 2048 x 8192 44.8
+//   -> 36.4, 100 x 30000 88 -> 29.6, 64 x 50257 164 -> 40; f16 4096 x 4096 186 -> 39.4,
+//   4096 x 1024 54 -> 14.5.
+// The groups a thread holds follow the row (1, 4, 8, 16 a wave, 6, 8, 32 a block):
+// clamped ones are loaded and summed in vain.  With 4, 16, 8 and 32 only, f16 8656 x
+// 192 took 15.6 (now 11.8, before the groups 12.0), 3439 x 192 10.2 (8.5, 8.3), 800 x
+// 2048 12.0 (10.2, 10.1), bf16 1000 x 4608 19.0 (17.8, 17.5).  A row or two per lane
+// still lose 3-6 % to the masks: f32 300 x 5000 10.4 -> 10.9 (11.3 with 8 groups), 256 x
+// 6000 8.7 -> 9.3, f16 2000 x 768 9.1 -> 9.5.  (In leaves by register need, as softmax's,
+// these take 10.2, 8.6 and 8.7, but the kernel's register saving then changes at every
+// call: 0.7-1.2 us more a launch, 24.8 -> 25.5 for an MLP of two products.)
 struct LnTask {
   const gbyte *a, *gp, *bp;
   gbyte* d;
@@ -841,8 +848,11 @@ VM_DEV void ln_rows_long(Args A, uint32_t ti, uint32_t r0, uint32_t r1) {
 template <bool IN16>
 VM_DEV void ln_dispatch(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
   const uint32_t n = (task_of(A, ti).p[1] + 3) >> 2, wave = uni(threadIdx.x >> 6);
-  if (n <= 4 * 64) ln_rows<4, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  if (n <= 64) ln_rows<1, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (n <= 4 * 64) ln_rows<4, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (n <= 8 * 64) ln_rows<8, IN16, 64>(A, ti, lo + wave, hi, kWaves);
   else if (n <= 16 * 64) ln_rows<16, IN16, 64>(A, ti, lo + wave, hi, kWaves);
+  else if (n <= 6 * kBlock) ln_rows<6, IN16, kBlock>(A, ti, lo, hi, 1);
   else if (n <= 8 * kBlock) ln_rows<8, IN16, kBlock>(A, ti, lo, hi, 1);
   else if (n <= 32 * kBlock) ln_rows<32, IN16, kBlock>(A, ti, lo, hi, 1);
   else ln_rows_long<IN16>(A, ti, lo, hi);

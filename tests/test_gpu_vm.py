@@ -446,7 +446,7 @@ def test_fused_layernorm_affine_gelu(in_dt, out_dt):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("seg", [3, 4, 5, 255, 1023, 1025, 4095, 4097, 8192, 8193, 32767, 32769, 50257])
+@pytest.mark.parametrize("seg", [3, 4, 5, 255, 257, 1023, 1025, 2047, 2049, 4095, 4097, 6143, 6145, 8192, 8193, 32767, 32769, 50257])
 def test_layernorm_row_forms(dt, seg):
     """Each row form (elements, wave, block, passes in memory) at the edges of its
     lengths and odd lengths, in one pass (core) and two (affine, GELU).  f32 sums of
