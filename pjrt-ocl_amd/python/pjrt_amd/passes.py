@@ -324,8 +324,15 @@ def fold_dot_transposes(prog: V.VMProgram) -> None:
     """A matmul whose only reader transposes it, (A B)^T, becomes B^T A^T written in
     the transposed layout: JAX's rule for a weight's gradient is dot_general(g, x)
     and a transpose.  The operands swap and each reads through its transposed view
-    (none where that is the plain matrix); every output is the same products summed
-    in the same order.  Matmuls with an epilogue, a batch or wider views stay."""
+    (none where that is the plain matrix); every output is the same products, summed
+    in the order of the kernel that the swapped shape takes (a K split and TOP_GEMV
+    have orders of their own).  Matmuls with an epilogue, a batch or wider views stay.
+    So do f32 products of one row and K >= 1024 that are TOP_GEMV as they stand: with
+    the row as a column, the f32 tiles walk K for one column of 64 (MI355X, us, swapped
+    / as GEMV and a copy: 1 x 4096 x 4096 37 / 31, 1 x 4096 x 11008 84 / 58; but 1 x 768 x
+    3072 16.0 / 17.1, bf16 1 x 4096 x 4096 20.7 / 25.1, 1 x 768 x 32000 17 / 25, and two to
+    eight rows gain in both: 4 x 768 x 3072 f32 15.7 / 24.6, bf16 2 x 4096 x 11008 24 /
+    78)."""
     if _off("PJRT_AMD_DOT_TRANSPOSE"):
         return
 
@@ -350,6 +357,8 @@ def fold_dot_transposes(prog: V.VMProgram) -> None:
             continue
         M, N, K, G = _dot_fields_pass(dot)[:4]
         if G != 1 or M > 0xFFFF or _dt(prog, g.dst) != _dt(prog, g.a) or g.n != M * N:
+            continue
+        if M == 1 and K >= 1024 and N % 8 == 0 and not (dot.aview or dot.bview) and _dt(prog, dot.a) == V.DT_F32:
             continue
         if _merged(*_view_desc(prog, g.aux + 1)) != _merged([N, M], [1, N], 0):
             continue

@@ -480,3 +480,24 @@ module @jit_f {{
         assert V.OP_GATHER_STRIDED in live_ops(fused)
     for x, y in zip(got, plain):
         np.testing.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("M,K,N,dt,swaps", [(1, 1024, 64, "f32", False), (1, 1023, 64, "f32", True),
+                                            (1, 1024, 60, "f32", True), (1, 1024, 64, "bf16", True),
+                                            (2, 1024, 64, "f32", True), (1024, 1024, 1, "f32", True)])
+def test_transposed_one_row_f32_product_stays_a_gemv(M, K, N, dt, swaps):
+    """x @ W of one f32 row keeps TOP_GEMV when its transpose is asked for; the shapes
+    around it are swapped."""
+    A, B, C, CT = (f"tensor<{a}x{b}x{t}>" for a, b, t in ((M, K, dt), (K, N, dt), (M, N, "f32"), (N, M, "f32")))
+    prog = L.lower_text(f"""
+module @jit_f {{
+  func.func public @main(%arg0: {A}, %arg1: {B}) -> {CT} {{
+    %0 = stablehlo.dot_general %arg0, %arg1, contracting_dims = [1] x [0], precision = [DEFAULT, DEFAULT] : ({A}, {B}) -> {C}
+    %1 = stablehlo.transpose %0, dims = [1, 0] : ({C}) -> {CT}
+    return %1 : {CT}
+  }}
+}}
+""")
+    assert (live_ops(prog) == [V.OP_DOT]) == swaps
+    tops = [t.tile_op for t in S.schedule_program(prog, S.DeviceConfig(nlanes=256)).tasks]
+    assert (V.TOP_GEMV in tops) != swaps, tops
