@@ -955,12 +955,15 @@ def _tile_quantum(task: V.Task, cfg: DeviceConfig, prog: V.VMProgram) -> int:
     """Preferred chunk granularity in tiles (chunk boundaries on multiples of
     it keep the kernel's multi-row blocks whole)."""
     if task.tile_op == V.TOP_FLASH_ATTN:
-        # the matrix-core kernel works on 256-row blocks of one head, and each
+        # the matrix-core kernels work on 256-row blocks of one head, and each
         # head's tiles are padded to whole blocks (attn_rows_padded); where the
-        # blocks would leave half the lanes idle, on halves of them (24 heads x
-        # 1000 f16 on 256 lanes, 96 blocks: 31.9 us in blocks, 26.5 in halves)
+        # blocks would leave half the lanes idle, the 16-bit one for heads of up to
+        # 128 works on halves of them (24 heads x 1000 f16 on 256 lanes, 96 blocks:
+        # 31.9 us in blocks, 26.5 in halves).  The f32 and wide-head kernels compute
+        # every block that a chunk touches whole.
         blocks = task.p1 * attn_rows_padded(task.p2) // ATTN_BLOCK_ROWS
-        if task.adtype in (V.DT_BF16, V.DT_F16) and 2 * blocks <= cfg.nlanes:
+        hd = prog.aux[task.p3 + 3]
+        if task.adtype in (V.DT_BF16, V.DT_F16) and hd <= 128 and hd % 8 == 0 and 2 * blocks <= cfg.nlanes:
             return ATTN_BLOCK_ROWS // 2
         return ATTN_BLOCK_ROWS
     return 1

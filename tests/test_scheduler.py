@@ -210,6 +210,19 @@ def test_mma_autotile_long_k_skinny_takes_split_128():
     assert edge(task(256, 4096, 4096, "f32")) == 64     # f32: the count rule (256 tiles of 64)
 
 
+@pytest.mark.parametrize("dt,hd,rows", [("bf16", 64, 128), ("f16", 128, 128), ("bf16", 40, 128), ("bf16", 136, 256),
+                                        ("f16", 256, 256), ("bf16", 36, 256), ("f32", 64, 256)])
+def test_attention_chunks_are_what_the_kernel_works_on(dt, hd, rows):
+    """Chunks of 128 query rows only for the kernel that computes 128: the wide-head
+    and f32 ones would compute both halves of each block on two lanes."""
+    g = G.Graph()
+    q, k, v = (g.input((8, 2048, hd), dt) for _ in range(3))
+    g.output(g.flash_attention(q, k, v, 0.125, False))
+    sched = S.schedule_program(g.build(), S.DeviceConfig(nlanes=256, fit_lanes=False))
+    ents = [e for lane in sched.lane_streams for e in lane if e.task == 0]
+    assert {e.tile_hi - e.tile_lo for e in ents} == {rows} and len(ents) * rows == 8 * 2048
+
+
 # --- K-split matmuls (extension) -----------------------------------------------------
 
 def test_mma_split_k_choice():
