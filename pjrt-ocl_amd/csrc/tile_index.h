@@ -187,8 +187,9 @@ VM_TILE void gather_tiles(Args A, uint32_t ti, uint32_t lo, uint32_t hi, bool sc
   if (gather_wide(aux, t.p[0], d, a, e0, e1, es, scatter)) return;
   // Element by element (a transpose's strided side): the index map decoded once per
   // tile (invariant-divisor quotients) and eight elements' loads issued before the
-  // first store; one at a time, 4096 elements cost 29-37 us.
-  if (!scatter && rank <= kViewRank && n <= 0xFFFFFFF0u && (es == 4 || es == 2)) {
+  // first store; one at a time, 4096 elements cost 29-37 us.  (A step of 2048 past n
+  // stays in 32 bits.)
+  if (!scatter && rank <= kViewRank && n <= 0xFFFFF7FFu && (es == 4 || es == 2)) {
     const ViewMap m = view_map(aux, t.p[0] + 1);
     if (es == 4) gather_elems<uint32_t>(m, d, a, uint32_t(e0), uint32_t(e1));
     else gather_elems<uint16_t>(m, d, a, uint32_t(e0), uint32_t(e1));

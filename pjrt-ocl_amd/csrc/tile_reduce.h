@@ -973,7 +973,7 @@ VM_DEV void layernorm_run(Args A, uint32_t ti, uint32_t lo, uint32_t hi) {
 //     per thread.
 // Loads are not predicated (ln_load's reason), except in softmax_rows_few: groups
 // past the row re-read its last.  Memory bounds them (MI355X, whole launches): 512 x
-// 32000 f32 33.5 us (3.9 TB/s: two rows per CU, so the first row's load and the last
+// 32000 f32 33.9 us (3.9 TB/s: two rows per CU, so the first row's load and the last
 // one's store overlap nothing), 4096 x 4096 25.0 (5.4 TB/s), 4096 x 1001 8.9.
 // Rows r0, r0 + step, ... < r1, a row over the TH threads (64: the wave; kBlock: the
 // block), this thread's groups t, t + TH, ...
