@@ -17,6 +17,7 @@ import vmprogs as P
 from gpu_util import as_f32, assert_product_elementwise, assert_rel, attention_abs_scale, blob_for, run_both, run_gpu, runtime
 from oracle import vmref
 from pjrt_amd import graph as G
+from pjrt_amd import scheduler as S
 from pjrt_amd import vmprogram as V
 
 pytestmark = pytest.mark.gpu
@@ -483,6 +484,31 @@ def test_layernorm_row_forms(dt, seg):
     assert_rel(got[1], gelu, 1e-5, 4e-5 * scale, "affine + gelu")
 
 
+@pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
+@pytest.mark.parametrize("nlanes", [None, 2])
+@pytest.mark.parametrize("seg", [3, 5, 255, 257, 1023, 2049, 4097, 8193, 32769, 50257])
+def test_row_ops_in_place_bit_exact(seg, nlanes, dt):
+    """Softmax and layernorm with the destination on the source give the bits of the
+    same ops into buffers of their own: odd lengths, whose last group overlaps the one
+    before, in every row form."""
+    rng = np.random.default_rng(54)
+    a = rng.standard_normal((9, seg)).astype(np.float32)
+    if dt != "f32":
+        a = a.astype(np.float16) if dt == "f16" else vmref.f32_to_bf16(a)
+    g = G.Graph()
+    x = g.input(a.shape, dt)
+    own = [g.softmax_last(x), g.layernorm_core(x, 1e-5)]
+    inp = [g.unary("copy", x), g.unary("copy", x)]
+    g.emit(V.Instr(V.OP_SOFTMAX, dst=inp[0].buf, a=inp[0].buf, n=9, imm=seg))
+    g.emit(V.Instr(V.OP_LAYERNORM, dst=inp[1].buf, a=inp[1].buf, n=9, imm=seg, imm2=V.f32_bits(1e-5)))
+    g.output(*own, *inp)
+    blob, _ = blob_for(g.build(), nlanes=nlanes)
+    print(f"[gpu] case: rows in place {dt} {seg} lanes {nlanes}", file=sys.stderr, flush=True)
+    got = run_gpu(blob, [a])
+    for k in (0, 1):
+        np.testing.assert_array_equal(np.asarray(got[2 + k]).view(np.uint8), np.asarray(got[k]).view(np.uint8))
+
+
 @pytest.mark.parametrize("d,in_dt", [(100, "f32"), (6000, "f32"), (768, "f16"), (768, "f32")])
 def test_layernorm_row_interleave(d, in_dt):
     """Rows a multiple of the lane count: the scheduler interleaves the lanes'
@@ -766,27 +792,31 @@ def test_dot_fast_path_epilogue(in_dt, out_dt):
 
 
 @pytest.mark.parametrize("dt", ["f32", "bf16", "f16"])
-@pytest.mark.parametrize("Gb,M,K,N", [(1, 256, 512, 64), (2, 100, 300, 70), (1, 64, 1000, 128), (1, 256, 128, 512)])
+@pytest.mark.parametrize("Gb,M,K,N", [(1, 256, 2048, 64), (2, 100, 1540, 70), (1, 64, 3000, 128), (1, 256, 1400, 512)])
 def test_dot_split_k_exact(dt, Gb, M, K, N):
-    """K-split matmul tiles (few output tiles, deep K; K = 300 leaves the last
-    split short, or empty): each split publishes its partial tile, the last to
-    arrive sums them in split order and applies the bias + relu epilogue.
-    Integer-valued operands give the exact product; the program runs twice, so the
-    second run finds the arrival counters reset."""
+    """K-split matmul tiles (few output tiles, a K long enough in every type that the
+    loader lets the split do the work; 3000 leaves the last split short, 1540 three
+    of sixteen 16-bit splits empty): each split publishes its partial tile, the last
+    to arrive sums them in split order and applies the bias + relu epilogue.
+    Integer-valued operands give the exact product; one loaded program runs on three
+    inputs, so that counters which the run before left standing would show."""
     rng = np.random.default_rng(74)
-    a = rng.integers(-3, 4, (Gb, M, K)).astype(np.float32)
-    b = rng.integers(-3, 4, (Gb, K, N)).astype(np.float32)
-    bias = rng.integers(-9, 10, N).astype(np.float32)
     g = G.Graph()
-    x, y, bb = g.input(a.shape, dt), g.input(b.shape, dt), g.input(bias.shape)
+    x, y, bb = g.input((Gb, M, K), dt), g.input((Gb, K, N), dt), g.input((N,))
     g.output(g.dot(x, y, residual=bb, epilogue=[(V.SUB_ADD, 2, 0.0, 0.0), (V.SUB_MAX, 3, 0.0, 0.0)]))
     blob, cfg = blob_for(g.build())
     task = vmref.parse(blob).tasks[0]
-    assert task.top == V.TOP_MMA and task.p[3] >> V.MMA_SPLIT_SHIFT >= 1, hex(task.p[3])
-    want = np.maximum(np.matmul(a.astype(np.float64), b.astype(np.float64)) + bias, 0.0).astype(np.float32)
+    assert task.top == V.TOP_MMA
+    edge = V.MMA_CODE_TILE.get((task.p[3] >> 24) & 0xF, cfg.mma_t)
+    assert S.mma_effective_split(1 << (task.p[3] >> V.MMA_SPLIT_SHIFT), K, edge, V.DT_BY_NAME[dt]) > 1, hex(task.p[3])
+    print(f"[gpu] case: split K {dt} {Gb} x {M} x {K} x {N}", file=sys.stderr, flush=True)
     lp = runtime().load(blob)
     try:
-        for run in range(2):
+        for run in range(3):
+            a = rng.integers(-3, 4, (Gb, M, K)).astype(np.float32)
+            b = rng.integers(-3, 4, (Gb, K, N)).astype(np.float32)
+            bias = rng.integers(-9, 10, N).astype(np.float32)
+            want = np.maximum(np.matmul(a.astype(np.float64), b.astype(np.float64)) + bias, 0.0).astype(np.float32)
             np.testing.assert_array_equal(lp(a, b, bias)[0], want, err_msg=f"run {run}")
     finally:
         lp.close()
@@ -796,7 +826,8 @@ def test_dot_split_k_exact(dt, Gb, M, K, N):
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("Gb,M,K,N,tile", [(1, 200, 520, 136, 64), (1, 264, 72, 392, 128), (2, 129, 200, 72, 64),
                                            (1, 61, 131, 77, 64), (1, 259, 333, 131, 128), (3, 70, 9, 67, 64),
-                                           (1, 300, 261, 515, 256), (1, 64, 1100, 64, 0), (1, 70, 3001, 64, 0),
+                                           (1, 300, 261, 515, 256), (1, 300, 264, 520, 256), (2, 260, 72, 264, 256),
+                                           (1, 257, 8, 264, 256), (1, 64, 1100, 64, 0), (1, 70, 3001, 64, 0),
                                            (1, 8, 8, 9, 64)])
 def test_dot_operand_layouts_exact(dt, ta, tb, Gb, M, K, N, tile):
     """The 64- and 128-wide tiles with each operand k-contiguous or
@@ -805,7 +836,8 @@ def test_dot_operand_layouts_exact(dt, ta, tb, Gb, M, K, N, tile):
     and in odd sizes (through registers, chunks cut at the operands' ends), a
     batch, a K split (tile 0: the scheduler's choice; 3001 is worth one in every type), and a 256-wide tile done
     as four.  Integer-valued operands give the exact result, whose bias and
-    residual epilogue reads ragged rows."""
+    residual epilogue reads ragged rows.  256-wide with K and N multiples of 8 and B
+    k-contiguous: the fast tile's transposed form in 16 bits (K % 64 zeroed, N ragged)."""
     rng = np.random.default_rng(79)
     a = rng.integers(-3, 4, (Gb, M, K)).astype(np.float32)
     b = rng.integers(-3, 4, (Gb, K, N)).astype(np.float32)
@@ -850,6 +882,23 @@ def test_dot_operand_slices_exact():
         np.testing.assert_array_equal(got[0], np.matmul(q, k.transpose(0, 2, 1)))
         np.testing.assert_array_equal(got[1], rows @ w)
         np.testing.assert_array_equal(got[2], rows @ w8)
+
+
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_dot_wide_tile_k_contiguous_slice_exact(dt):
+    """The 256-wide 16-bit tile with B a slice of wider rows, x @ table[5:525, 16:280].T:
+    the view's row stride and offset, K % 64 and N % 256 left over."""
+    rng = np.random.default_rng(83)
+    M, K, N, ld, r0, c0 = 290, 264, 520, 320, 5, 16
+    a = rng.integers(-3, 4, (M, K)).astype(np.float32)
+    table = rng.integers(-3, 4, (N + 9, ld)).astype(np.float32)
+    g = G.Graph()
+    x, w = g.input(a.shape, dt), g.input(table.shape, dt)
+    g.output(g.dot(x, g.view(w, (K, N), (1, ld), r0 * ld + c0), tile=256))
+    blob, _ = blob_for(g.build())
+    print(f"[gpu] case: wide tile, sliced rows {dt}", file=sys.stderr, flush=True)
+    want = a.astype(np.float64) @ table[r0:r0 + N, c0:c0 + K].T.astype(np.float64)
+    np.testing.assert_array_equal(run_gpu(blob, [a, table])[0], want)
 
 
 def test_dot_fast_path_random_bf16():
@@ -1061,6 +1110,8 @@ def test_dot_views_batch_epilogue():
                                               ("bf16", 256, True, 300, 300), ("f16", 256, False, 129, 200),
                                               ("bf16", 192, True, 640, 700), ("f16", 136, True, 64, 90)])
 def test_flash_attention(dt, hd, causal, T, C):
+    """On all lanes (16-bit heads to 128: halves of a block) and on two, which take
+    whole blocks."""
     rng = np.random.default_rng(1004)
     H = 3
     q = rng.standard_normal((H, T, hd)).astype(np.float32)
@@ -1073,15 +1124,17 @@ def test_flash_attention(dt, hd, causal, T, C):
     g = G.Graph()
     Q, K, Vv = g.input(q.shape, dt), g.input(k.shape, dt), g.input(v.shape, dt)
     g.output(g.flash_attention(Q, K, Vv, 1.0 / np.sqrt(hd), causal, out_dtype="f32"))
-    got, _ = run_both(g.build(), [q, k, v], oracle=None)
+    prog = g.build()
     want = vmref.attention(q, np.transpose(k, (0, 2, 1)), v, 1.0 / np.sqrt(hd), causal)
     # f32: f32 products and sums (matrix cores or the row kernel); 16-bit: P in bf16 / f16
     tol = 2e-5 if dt == "f32" else 1e-2
-    err = np.abs(got[0] - want).max() / max(1e-6, np.abs(want).max())
-    assert err <= tol, err
-    assert_product_elementwise(got[0], want.astype(np.float64),
-                               attention_abs_scale(q, np.transpose(k, (0, 2, 1)), v, 1.0 / np.sqrt(hd), causal), tol,
-                               f"flash {dt} hd {hd}")
+    for nlanes in (None, 2):
+        got, _ = run_both(prog, [q, k, v], nlanes=nlanes, oracle=None)
+        err = np.abs(got[0] - want).max() / max(1e-6, np.abs(want).max())
+        assert err <= tol, err
+        assert_product_elementwise(got[0], want.astype(np.float64),
+                                   attention_abs_scale(q, np.transpose(k, (0, 2, 1)), v, 1.0 / np.sqrt(hd), causal), tol,
+                                   f"flash {dt} hd {hd}")
 
 
 @pytest.mark.parametrize("dt,hd,causal,T", [("bf16", 64, True, 1), ("f16", 128, False, 127), ("bf16", 128, True, 128),
@@ -1126,9 +1179,11 @@ def test_flash_attention_partial_block_inf_value(hd, dt):
     g = G.Graph()
     Q, K, Vv = g.input(q.shape, dt), g.input(k.shape, dt), g.input(v.shape, dt)
     g.output(g.flash_attention(Q, K, Vv, 1.0 / np.sqrt(hd), False, out_dtype="f32"))
-    got, _ = run_both(g.build(), [q, k, v], oracle=None)
+    prog = g.build()
     assert np.isposinf(vmref.attention(q, np.transpose(k, (0, 2, 1)), v, 1.0 / np.sqrt(hd), False)).all()
-    assert np.isposinf(got[0]).all(), int(np.isnan(got[0]).sum())
+    for nlanes in (None, 2):                # halves of a block, and the whole one
+        got, _ = run_both(prog, [q, k, v], nlanes=nlanes, oracle=None)
+        assert np.isposinf(got[0]).all(), (nlanes, int(np.isnan(got[0]).sum()))
 
 
 @pytest.mark.parametrize("dt,hd", [("bf16", 128), ("f16", 64), ("bf16", 96), ("f32", 64), ("bf16", 256),
@@ -1167,8 +1222,9 @@ def test_flash_attention_score_jump(dt, causal, T, C, target, hd):
     """A key late in the sequence whose scaled score with one query is `target`
     above the rest: probabilities against the first block's maximum would
     overflow (f32 for bf16 at 150, f16 at 22), so the kernel must take its exact
-    two-pass route for that block; the result still matches float64 math (also
-    with a padded head size, whose zeroed slots every sweep sets again)."""
+    two-pass route for that block (whole, on two lanes, or half); the result still
+    matches float64 math (also with a padded head size, whose zeroed slots every
+    sweep sets again)."""
     rng = np.random.default_rng(1006)
     H = 2
     q = rng.standard_normal((H, T, hd)).astype(np.float32)
@@ -1184,13 +1240,15 @@ def test_flash_attention_score_jump(dt, causal, T, C, target, hd):
     g = G.Graph()
     Q, K, Vv = g.input(q.shape, dt), g.input(k.shape, dt), g.input(v.shape, dt)
     g.output(g.flash_attention(Q, K, Vv, 1.0 / np.sqrt(hd), causal, out_dtype="f32"))
-    got, _ = run_both(g.build(), [q, k, v], oracle=None)
+    prog = g.build()
     want = vmref.attention(q, np.transpose(k, (0, 2, 1)), v, 1.0 / np.sqrt(hd), causal)
-    assert np.isfinite(got[0]).all()
-    err = np.abs(got[0] - want).max() / max(1e-6, np.abs(want).max())
-    assert err <= 1e-2, err
-    # the jump row follows the far key's value row
-    np.testing.assert_allclose(got[0][:, qi], want[:, qi], rtol=0, atol=2e-2 * np.abs(want).max())
+    for nlanes in (None, 2):
+        got, _ = run_both(prog, [q, k, v], nlanes=nlanes, oracle=None)
+        assert np.isfinite(got[0]).all()
+        err = np.abs(got[0] - want).max() / max(1e-6, np.abs(want).max())
+        assert err <= 1e-2, err
+        # the jump row follows the far key's value row
+        np.testing.assert_allclose(got[0][:, qi], want[:, qi], rtol=0, atol=2e-2 * np.abs(want).max())
 
 
 @pytest.mark.parametrize("dt,H,hd,C,pos,jump,mode", [
